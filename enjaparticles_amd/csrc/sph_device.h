@@ -159,6 +159,9 @@ struct Win {
     // testing those candidates again.
     uint32_t* rows = nullptr;
     uint32_t rows_stride = 0;   // particles per row plane (at least the particle count)
+    // small launches may split their tiles over three waves, one per plane of
+    // the neighbourhood (other roundings than the unsplit kernels' single sequence)
+    bool split = false;
 };
 
 // Candidates per group in the neighbour loops (loads in flight per lane).
@@ -469,6 +472,12 @@ struct ForceAcc {
     float vx, vy, vz;
     float xx, xy, xz;
 };
+
+__device__ __forceinline__ void add_acc(ForceAcc& a, const ForceAcc& b) {
+    a.fx += b.fx; a.fy += b.fy; a.fz += b.fz;
+    a.vx += b.vx; a.vy += b.vy; a.vz += b.vz;
+    a.xx += b.xx; a.xy += b.xy; a.xz += b.xz;
+}
 
 // One accepted pair (rlen <= h, j != i) of force.cl:62-139.  Self pairs add
 // exactly zero in the reference (iej = 0 multiplies a finite value), so they

@@ -134,6 +134,27 @@ __global__ __launch_bounds__(kBlock) void k_cells_permute(int num_host, const in
 }
 
 // ---------------------------------------------------------------------------
+// Split tiles: smaller density and force launches whose caller allows it
+// (Win::split) run blocks of three waves over 64 particles, one wave per plane
+// (dz) of the neighbourhood, instead of one wave over all nine rows.  A wave's
+// nine rows are a chain of dependent loads (window, copy, walk), and the chip
+// has 1024 SIMDs: 65,536 particles are one wave each, which nothing overlaps.
+// Split, they are three waves a SIMD with chains a third as long.  The planes'
+// sums are added at the end, so the roundings differ from the unsplit kernels',
+// and the plain step, whose bits callers compare with other launches', stays
+// unsplit.  Measured with windowed rows (us, unsplit / split): density
+// 16.5 / 8.7 at 2,048 particles, 25.3 / 14.6 at 65,536, 40.2 / 37.8 at 262,144
+// and 161 / 160 at 1,048,576 (settled pools); force 15.4 / 9.4, 43 / 25.3,
+// 71 / 64 and 234 / 247, and 31 / 33 at 262,144 at rest.  With the whole rows of
+// the stage operators a step of 50,021 particles takes 197 us instead of 260.
+// The lines: density to 2^20 particles (equal there); force to 3 * 2^16, past
+// which the repeated loads of a particle's own record, the adding of the
+// planes' sums and the idle end of the block's shorter planes cost more than
+// the waves bring.
+constexpr int kSplitBlock = 192;
+constexpr int kSplitMaxDensity = 1 << 20;
+constexpr int kSplitMaxForce = 3 << 16;
+
 // a7: density.cl:86-126.  PACKED: the density is written to veleval_s[i].w
 // (the system layout, so the force loop loads one float4 per neighbour).
 // candidates per density group, their loads issued together
@@ -152,16 +173,14 @@ int g_density_stage = 1;
 // EMIT: each row's window and the rejection bits of its last 32 candidates
 // go to win.rows (one rej_bit per candidate, the same u as the poly6 term),
 // for every live particle and all nine rows (empty rows as [a, a)).
-template <bool SCALED, bool PACKED, bool STAGE, bool EMIT>
-__device__ __forceinline__ void density_tile(int tile, int num_host, const int* __restrict__ d_num,
-                                             const float4* __restrict__ pos_s, const uint32_t* __restrict__ start,
-                                             const uint32_t* __restrict__ end, const rtps_sph_params& sp,
-                                             const Grid& g, const Win& win, float* __restrict__ dens,
-                                             float4* __restrict__ packed) {
-    const int i = tile * (int)blockDim.x + (int)threadIdx.x;
-    int num = d_num ? *d_num : num_host;
-    if (d_num) effective_num(num, start, g.nb_cells, num);
-    if (i >= num) return;
+//
+// The poly6 sum of particle i over the rows of the planes dz_lo..dz_hi of its
+// neighbourhood.
+template <bool SCALED, bool STAGE, bool EMIT>
+__device__ __forceinline__ float density_planes(int i, int dz_lo, int dz_hi, const float4* __restrict__ pos_s,
+                                                const uint32_t* __restrict__ start,
+                                                const uint32_t* __restrict__ end, const rtps_sph_params& sp,
+                                                const Grid& g, const Win& win) {
     const float scale = sp.simulation_scale;
     const float h = sp.smoothing_distance, h2 = h * h;
     float4 pi = pos_s[i];
@@ -196,7 +215,7 @@ __device__ __forceinline__ void density_tile(int tile, int num_host, const int* 
     // the wave's row unions [A, B) follow the particles' records, two words
     // per row for each wave of 64 particles (written by its first live lane)
     uint32_t* __restrict__ wrec = EMIT ? win.rows + 27 * (size_t)win.rows_stride + 18 * (size_t)(i >> 6) : nullptr;
-    const uint64_t live = __ballot(true);   // lanes past num have returned
+    const uint64_t live = __ballot(true);   // lanes past num are not here
     const uint32_t nlive = (uint32_t)__popcll(live);
     const uint32_t rank = (uint32_t)__popcll(live & ((1ull << (threadIdx.x & 63)) - 1ull));
     auto record = [&](int dz, int dy, uint32_t a, uint32_t b, uint32_t A, uint32_t B) {
@@ -217,7 +236,7 @@ __device__ __forceinline__ void density_tile(int tile, int num_host, const int* 
         extern __shared__ float4 stage_rows[];   // kStageCap per wave
         float4* __restrict__ my = stage_rows + (threadIdx.x >> 6) * kStageCap;
         // the wave's live lanes (rank of nlive) share the copies
-        for (int dz = -1; dz <= 1; ++dz) {
+        for (int dz = dz_lo; dz <= dz_hi; ++dz) {
             for (int dy = -1; dy <= 1; ++dy) {
                 uint32_t a, b;
                 row_window(wc, c, dy, dz, h2, g, start, end, win.keys, a, b, 0u, win.sub);
@@ -237,7 +256,7 @@ __device__ __forceinline__ void density_tile(int tile, int num_host, const int* 
             }
         }
     } else {
-        for (int dz = -1; dz <= 1; ++dz) {
+        for (int dz = dz_lo; dz <= dz_hi; ++dz) {
             for (int dy = -1; dy <= 1; ++dy) {
                 uint32_t a, b;
                 row_window(wc, c, dy, dz, h2, g, start, end, win.keys, a, b, 0u, win.sub);
@@ -248,6 +267,33 @@ __device__ __forceinline__ void density_tile(int tile, int num_host, const int* 
             }
         }
     }
+    return sum;
+}
+
+// SPLIT: the block's three waves take one plane (dz) of the same 64
+// particles each; see kSplitMaxDensity.
+template <bool SCALED, bool PACKED, bool STAGE, bool EMIT, bool SPLIT>
+__device__ __forceinline__ void density_tile(int tile, int num_host, const int* __restrict__ d_num,
+                                             const float4* __restrict__ pos_s, const uint32_t* __restrict__ start,
+                                             const uint32_t* __restrict__ end, const rtps_sph_params& sp,
+                                             const Grid& g, const Win& win, float* __restrict__ dens,
+                                             float4* __restrict__ packed) {
+    const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+    const int i = SPLIT ? tile * 64 + lane : tile * (int)blockDim.x + (int)threadIdx.x;
+    int num = d_num ? *d_num : num_host;
+    if (d_num) effective_num(num, start, g.nb_cells, num);
+    float sum = 0.0f;
+    if constexpr (SPLIT) {
+        __shared__ float part[2][64];
+        if (i < num) sum = density_planes<SCALED, STAGE, EMIT>(i, w - 1, w - 1, pos_s, start, end, sp, g, win);
+        if (w > 0) part[w - 1][lane] = sum;
+        __syncthreads();
+        if (w > 0 || i >= num) return;
+        sum = (sum + part[0][lane]) + part[1][lane];
+    } else {
+        if (i >= num) return;
+        sum = density_planes<SCALED, STAGE, EMIT>(i, -1, 1, pos_s, start, end, sp, g, win);
+    }
     const float rho = sp.wpoly6_coef * sp.mass * sum;
     if (PACKED) packed[i].w = rho; else dens[i] = rho;
 }
@@ -256,8 +302,8 @@ __device__ __forceinline__ void density_tile(int tile, int num_host, const int* 
 // grid working through the per-XCD tile queues of win.tq.  The queued
 // kernels are separate instances: the loop around the body raises its
 // register demand, which must not cost the one-tile kernels.
-template <bool SCALED, bool PACKED, bool STAGE, bool QUEUED, bool EMIT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_vgpr(56))) void k_density(int num_host, const int* __restrict__ d_num,
+template <bool SCALED, bool PACKED, bool STAGE, bool QUEUED, bool EMIT, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? kSplitBlock : kBlock) __attribute__((amdgpu_num_vgpr(56))) void k_density(int num_host, const int* __restrict__ d_num,
                                                     const float4* __restrict__ pos_s,
                                                     const uint32_t* __restrict__ start,
                                                     const uint32_t* __restrict__ end, rtps_sph_params sp, Grid g,
@@ -267,13 +313,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_vgpr(56))) void k
         for (int t = first_tile(win.ntiles);;) {
             if (t < 0) t = claim_tile(win.tq, win.ntiles, q);
             if (t < 0) break;
-            density_tile<SCALED, PACKED, STAGE, EMIT>(t, num_host, d_num, pos_s, start, end, sp, g, win, dens, packed);
+            density_tile<SCALED, PACKED, STAGE, EMIT, false>(t, num_host, d_num, pos_s, start, end, sp, g, win, dens, packed);
             t = -1;
         }
         finish_tiles(win.tq);
     } else {
-        density_tile<SCALED, PACKED, STAGE, EMIT>(remap_tile(win.remap, (int)blockIdx.x, (int)gridDim.x), num_host, d_num,
-                                            pos_s, start, end, sp, g, win, dens, packed);
+        density_tile<SCALED, PACKED, STAGE, EMIT, SPLIT>(remap_tile(win.remap, (int)blockIdx.x, (int)gridDim.x),
+                                                         num_host, d_num, pos_s, start, end, sp, g, win, dens, packed);
     }
 }
 
@@ -319,39 +365,21 @@ constexpr int kStagedWavesPerSimd = 5;
 // The tile-queue instances at four (128 VGPRs): the loop keeps more values live.
 constexpr int kQueuedWavesPerSimd = 4;
 
-template <bool SCALED, bool PACKED, bool FUSED, int LOOP>
-__device__ __forceinline__ void force_tile(int tile, int num_host, int* d_num,
-                                           const float4* __restrict__ pos_s, const float* __restrict__ dens_in,
-                                           const float4* __restrict__ ve_in, const uint32_t* __restrict__ start,
-                                           const uint32_t* __restrict__ end, const rtps_sph_params& sp, const Grid& g,
-                                           const Win& win, float4* __restrict__ force_out,
-                                           float4* __restrict__ xsph_out,
-                                           // FUSED only:
-                                           const float4* __restrict__ vel_s, const uint32_t* __restrict__ idx,
-                                           const GravitySources& gsrc, int collision, const rtps_float4& bmin,
-                                           const rtps_float4& bmax, float dt, float4* __restrict__ pos_u,
-                                           float4* __restrict__ vel_u, float4* __restrict__ veleval_u,
-                                           const float4* __restrict__ color_s, float4* __restrict__ color_u) {
-    const int i = tile * (int)blockDim.x + (int)threadIdx.x;
-    int num = d_num ? *d_num : num_host;
-    bool deleted = false;
-    if (d_num) deleted = effective_num(num, start, g.nb_cells, num);
-    // FUSED: the step's last kernel commits the count of a deletion step for
-    // the next step (SPH.cpp:220-250).  Blocks that read d_num before or
-    // after this store get the same count: effective_num of the committed
-    // count is that count.  (d_num is not __restrict__: it is read and
-    // written here.)
-    if (FUSED && deleted && tile == 0 && threadIdx.x == 0) *d_num = num;
-    if (i >= num) return;
+// The pair sums of particle i over the rows of the planes dz_lo..dz_hi.
+template <bool SCALED, bool PACKED, int LOOP>
+__device__ __forceinline__ ForceAcc force_planes(int i, int dz_lo, int dz_hi, const float4* __restrict__ pos_s,
+                                                 const float* __restrict__ dens_in,
+                                                 const float4* __restrict__ ve_in,
+                                                 const uint32_t* __restrict__ start,
+                                                 const uint32_t* __restrict__ end, const rtps_sph_params& sp,
+                                                 const Grid& g, const Win& win) {
     const float scale = sp.simulation_scale;
     const float h = sp.smoothing_distance, h2 = h * h, eps = sp.EPSILON;
     const float K = sp.K, rho0 = sp.rest_density;
     float4 pi = pos_s[i];
-    const float4 p_unscaled = pi;
     if (SCALED) { pi.x *= scale; pi.y *= scale; pi.z *= scale; }
-    float4 vi;
-    float di;
-    if (PACKED) { vi = ve_in[i]; di = vi.w; } else { vi = ve_in[i]; di = dens_in[i]; }
+    const float4 vi = ve_in[i];
+    const float di = PACKED ? vi.w : dens_in[i];
     const float Pi = K * (di - rho0);
     ForceAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
@@ -370,7 +398,7 @@ __device__ __forceinline__ void force_tile(int tile, int num_host, int* d_num,
     if constexpr (LOOP == kLoopDirect) {
         const int3 c = grid_cell(pi.x, pi.y, pi.z, g);
         const WindowCtx wc = window_ctx(pi.x, pi.y, pi.z, g, c, h, win.keys, win.rx, win.ry, win.rz);
-        for (int dz = -1; dz <= 1; ++dz) {
+        for (int dz = dz_lo; dz <= dz_hi; ++dz) {
             for (int dy = -1; dy <= 1; ++dy) {
                 uint32_t a, b;
                 row_window(wc, c, dy, dz, h2, g, start, end, win.keys, a, b, 0u, win.sub);
@@ -521,7 +549,7 @@ __device__ __forceinline__ void force_tile(int tile, int num_host, int* d_num,
         };
         // the row's window and last-chunk rejection bits: recorded (loop 6) or looked up
         const uint32_t* __restrict__ rec = LOOP == kLoopShared ? win.rows + 3 * (size_t)i : nullptr;
-        for (int dz = -1; dz <= 1; ++dz) {
+        for (int dz = dz_lo; dz <= dz_hi; ++dz) {
             for (int dy = -1; dy <= 1; ++dy) {
                 uint32_t a, b, A, B, rej_last = 0u;
                 if constexpr (LOOP == kLoopShared) {
@@ -558,11 +586,74 @@ __device__ __forceinline__ void force_tile(int tile, int num_host, int* d_num,
             }
         }
     }
+    return acc;
+}
+
+// SPLIT: the block's three waves take one plane each, as for density; the
+// first adds the three sums and goes on to the epilogue.
+template <bool SCALED, bool PACKED, bool FUSED, int LOOP, bool SPLIT>
+__device__ __forceinline__ void force_tile(int tile, int num_host, int* d_num,
+                                           const float4* __restrict__ pos_s, const float* __restrict__ dens_in,
+                                           const float4* __restrict__ ve_in, const uint32_t* __restrict__ start,
+                                           const uint32_t* __restrict__ end, const rtps_sph_params& sp, const Grid& g,
+                                           const Win& win, float4* __restrict__ force_out,
+                                           float4* __restrict__ xsph_out,
+                                           // FUSED only:
+                                           const float4* __restrict__ vel_s, const uint32_t* __restrict__ idx,
+                                           const GravitySources& gsrc, int collision, const rtps_float4& bmin,
+                                           const rtps_float4& bmax, float dt, float4* __restrict__ pos_u,
+                                           float4* __restrict__ vel_u, float4* __restrict__ veleval_u,
+                                           const float4* __restrict__ color_s, float4* __restrict__ color_u) {
+    const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+    const int i = SPLIT ? tile * 64 + lane : tile * (int)blockDim.x + (int)threadIdx.x;
+    int num = d_num ? *d_num : num_host;
+    bool deleted = false;
+    if (d_num) deleted = effective_num(num, start, g.nb_cells, num);
+    // FUSED: the step's last kernel commits the count of a deletion step for
+    // the next step (SPH.cpp:220-250).  Blocks that read d_num before or
+    // after this store get the same count: effective_num of the committed
+    // count is that count.  (d_num is not __restrict__: it is read and
+    // written here.)
+    if (FUSED && deleted && tile == 0 && threadIdx.x == 0) *d_num = num;
+    ForceAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if constexpr (SPLIT) {
+        // the sums of waves 1 and 2 go through their own rows' LDS slices
+        // (free once the wave's last row is done), or their own LDS without one
+        float* part;
+        if constexpr (LOOP == kLoopDirect) {
+            __shared__ float own[3][9 * 64];
+            part = own[0];
+        } else {
+            extern __shared__ float4 force_rows[];
+            part = (float*)force_rows;
+        }
+        constexpr int kSlice = LOOP == kLoopDirect ? 9 * 64 : 8 * kForceStageCap;   // floats per wave
+        if (i < num)
+            acc = force_planes<SCALED, PACKED, LOOP>(i, w - 1, w - 1, pos_s, dens_in, ve_in, start, end, sp, g, win);
+        __builtin_amdgcn_wave_barrier();   // the last row's reads before the slice's reuse
+        if (w > 0) {
+            float (*p)[64] = (float (*)[64])(part + w * kSlice);
+            p[0][lane] = acc.fx; p[1][lane] = acc.fy; p[2][lane] = acc.fz;
+            p[3][lane] = acc.vx; p[4][lane] = acc.vy; p[5][lane] = acc.vz;
+            p[6][lane] = acc.xx; p[7][lane] = acc.xy; p[8][lane] = acc.xz;
+        }
+        __syncthreads();
+        if (w > 0 || i >= num) return;
+        for (int q = 1; q <= 2; ++q) {
+            const float (*p)[64] = (const float (*)[64])(part + q * kSlice);
+            add_acc(acc, ForceAcc{p[0][lane], p[1][lane], p[2][lane], p[3][lane], p[4][lane], p[5][lane], p[6][lane],
+                                  p[7][lane], p[8][lane]});
+        }
+    } else {
+        if (i >= num) return;
+        acc = force_planes<SCALED, PACKED, LOOP>(i, -1, 1, pos_s, dens_in, ve_in, start, end, sp, g, win);
+    }
     float4 F, X;
-    force_epilogue(acc, di, sp, F, X);
+    force_epilogue(acc, PACKED ? ve_in[i].w : dens_in[i], sp, F, X);
     if (force_out) { force_out[i] = F; xsph_out[i] = X; }
     if (FUSED) {
-        gravity_sources(F, p_unscaled, gsrc, scale);
+        const float4 p_unscaled = pos_s[i];
+        gravity_sources(F, p_unscaled, gsrc, sp.simulation_scale);
         const float4 v = vel_s[i];
         if (collision) collision_wall(F, p_unscaled, v, sp, bmin, bmax);
         float4 po, vo, eo;
@@ -580,8 +671,8 @@ __device__ __forceinline__ void force_tile(int tile, int num_host, int* d_num,
 // One tile of blockDim.x sorted particles per block, or (QUEUED) a resident
 // grid working through the per-XCD tile queues of win.tq (separate instances,
 // at four waves per SIMD: the loop around the body needs the registers).
-template <bool SCALED, bool PACKED, bool FUSED, int LOOP, bool QUEUED>
-__global__ __launch_bounds__(kBlock, QUEUED ? kQueuedWavesPerSimd : (LOOP >= kLoopStaged ? kStagedWavesPerSimd : kForceWavesPerSimd)) void k_force(int num_host, int* d_num,
+template <bool SCALED, bool PACKED, bool FUSED, int LOOP, bool QUEUED, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? kSplitBlock : kBlock, QUEUED ? kQueuedWavesPerSimd : (LOOP >= kLoopStaged ? kStagedWavesPerSimd : kForceWavesPerSimd)) void k_force(int num_host, int* d_num,
                                                   const float4* __restrict__ pos_s,
                                                   const float* __restrict__ dens_in,
                                                   const float4* __restrict__ ve_in,
@@ -601,17 +692,17 @@ __global__ __launch_bounds__(kBlock, QUEUED ? kQueuedWavesPerSimd : (LOOP >= kLo
         for (int t = first_tile(win.ntiles);;) {
             if (t < 0) t = claim_tile(win.tq, win.ntiles, q);
             if (t < 0) break;
-            force_tile<SCALED, PACKED, FUSED, LOOP>(t, num_host, d_num, pos_s, dens_in, ve_in, start, end, sp, g, win,
+            force_tile<SCALED, PACKED, FUSED, LOOP, false>(t, num_host, d_num, pos_s, dens_in, ve_in, start, end, sp, g, win,
                                                     force_out, xsph_out, vel_s, idx, gsrc, collision, bmin, bmax, dt,
                                                     pos_u, vel_u, veleval_u, color_s, color_u);
             t = -1;
         }
         finish_tiles(win.tq);
     } else {
-        force_tile<SCALED, PACKED, FUSED, LOOP>(remap_tile(win.remap, (int)blockIdx.x, (int)gridDim.x), num_host,
-                                                d_num, pos_s, dens_in, ve_in, start, end, sp, g, win, force_out,
-                                                xsph_out, vel_s, idx, gsrc, collision, bmin, bmax, dt, pos_u, vel_u,
-                                                veleval_u, color_s, color_u);
+        force_tile<SCALED, PACKED, FUSED, LOOP, SPLIT>(remap_tile(win.remap, (int)blockIdx.x, (int)gridDim.x),
+                                                       num_host, d_num, pos_s, dens_in, ve_in, start, end, sp, g, win,
+                                                       force_out, xsph_out, vel_s, idx, gsrc, collision, bmin, bmax,
+                                                       dt, pos_u, vel_u, veleval_u, color_s, color_u);
     }
 }
 
@@ -763,6 +854,9 @@ int g_force_variant = kLoopStagedBits;
 // Threads per block of a neighbour launch (a multiple of 64, at most kBlock)
 // and its force-loop variant.
 static inline int nbr_block(const Win& w) { return w.block > 0 && w.block <= kBlock && w.block % 64 == 0 ? w.block : kBlock; }
+// Whether a neighbour launch splits its tiles (never with the tile queues or
+// a block size fixed by the caller: Win::split).
+static inline bool nbr_split(int num, const Win& w, int most) { return w.split && !w.tq && num <= most; }
 static inline int nbr_variant(const Win& w) {
     const int v = w.variant >= 0 ? w.variant : g_force_variant;
     return v == kLoopStaged || v == kLoopStagedBits ? v : kLoopDirect;
@@ -852,8 +946,9 @@ hipError_t launch_density(int num, const int* d_num, const float4* pos_s, const 
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     if (num <= 0) return hipSuccess;
     const bool scaled = sp.simulation_scale != 1.0f;
-    const int bs = nbr_block(win_in);
-    const int nb = blocks_for(num, bs);
+    const bool split = nbr_split(num, win_in, kSplitMaxDensity);
+    const int bs = split ? kSplitBlock : nbr_block(win_in);
+    const int nb = blocks_for(num, split ? 64 : bs);
     const bool stage = g_density_stage != 0;
     const size_t lds = stage ? (size_t)(bs / 64) * kStageCap * sizeof(float4) : 0;
     if (win_in.rows && win_in.rows_stride < (uint32_t)num) return hipErrorInvalidValue;
@@ -861,10 +956,15 @@ hipError_t launch_density(int num, const int* d_num, const float4* pos_s, const 
     win.ntiles = nb;
 #define RTPS_DENS(S, P, T, E)                                                                                       \
     if (win.tq && P)                                                                                                \
-        k_density<S, P, T, true, E><<<resident_grid((const void*)&k_density<S, P, T, true, E>, bs, lds, nb), bs,     \
-                                      lds, st>>>(num, d_num, pos_s, start, end, sp, g, win, dens, packed);             \
+        k_density<S, P, T, true, E, false><<<resident_grid((const void*)&k_density<S, P, T, true, E, false>, bs, lds,  \
+                                                           nb),                                                       \
+                                             bs, lds, st>>>(num, d_num, pos_s, start, end, sp, g, win, dens, packed);  \
+    else if (split)                                                                                                 \
+        k_density<S, P, T, false, E, true><<<nb, bs, lds, st>>>(num, d_num, pos_s, start, end, sp, g, win, dens,       \
+                                                                packed);                                              \
     else                                                                                                            \
-        k_density<S, P, T, false, E><<<nb, bs, lds, st>>>(num, d_num, pos_s, start, end, sp, g, win, dens, packed)
+        k_density<S, P, T, false, E, false><<<nb, bs, lds, st>>>(num, d_num, pos_s, start, end, sp, g, win, dens,      \
+                                                                 packed)
 #define RTPS_DENS_T(T, E)                                                                                           \
     if (packed) { if (scaled) { RTPS_DENS(true, true, T, E); } else { RTPS_DENS(false, true, T, E); } }               \
     else { if (scaled) { RTPS_DENS(true, false, T, E); } else { RTPS_DENS(false, false, T, E); } }
@@ -894,8 +994,9 @@ hipError_t launch_force(int num, int* d_num, const float4* pos_s, const float* d
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     if (num <= 0) return hipSuccess;
     const bool scaled = sp.simulation_scale != 1.0f;
-    const int bs = nbr_block(win_in);
-    const int nb = blocks_for(num, bs);
+    const bool split = nbr_split(num, win_in, kSplitMaxForce);
+    const int bs = split ? kSplitBlock : nbr_block(win_in);
+    const int nb = blocks_for(num, split ? 64 : bs);
     const int loop = force_loop(win_in);
     if (win_in.rows && win_in.rows_stride < (uint32_t)num) return hipErrorInvalidValue;
     const size_t lds = force_lds(loop, bs);
@@ -903,15 +1004,18 @@ hipError_t launch_force(int num, int* d_num, const float4* pos_s, const float* d
     rtps_float4 z{0, 0, 0, 0};
     Win win = win_in;
     win.ntiles = nb;
-#define RTPS_FORCE_Q(S, P, L, Q, GRID)                                                                              \
-    k_force<S, P, false, L, Q><<<GRID, bs, lds, st>>>(num, d_num, pos_s, dens, ve, start, end, sp, g, win, force, xsph, \
+#define RTPS_FORCE_Q(S, P, L, Q, SP, GRID)                                                                          \
+    k_force<S, P, false, L, Q, SP><<<GRID, bs, lds, st>>>(num, d_num, pos_s, dens, ve, start, end, sp, g, win, force, xsph, \
                                                      nullptr, nullptr, none, 0, z, z, 0.f, nullptr, nullptr, nullptr, \
                                                      nullptr, nullptr)
 #define RTPS_FORCE_L(S, P, L)                                                                                       \
     if (win.tq && P) {                                                                                              \
-        RTPS_FORCE_Q(S, P, L, true, resident_grid((const void*)&k_force<S, P, false, L, true>, bs, lds, nb));        \
+        RTPS_FORCE_Q(S, P, L, true, false,                                                                          \
+                     resident_grid((const void*)&k_force<S, P, false, L, true, false>, bs, lds, nb));                \
+    } else if (split) {                                                                                             \
+        RTPS_FORCE_Q(S, P, L, false, true, nb);                                                                     \
     } else {                                                                                                        \
-        RTPS_FORCE_Q(S, P, L, false, nb);                                                                           \
+        RTPS_FORCE_Q(S, P, L, false, false, nb);                                                                    \
     }
 #define RTPS_FORCE(S, P)                                                                                            \
     if (loop == kLoopStaged) { RTPS_FORCE_L(S, P, kLoopStaged) }                                                    \
@@ -935,22 +1039,26 @@ hipError_t launch_force_fused(int num, int* d_num, const float4* pos_s, const fl
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     if (num <= 0) return hipSuccess;
     const bool scaled = sp.simulation_scale != 1.0f;
-    const int bs = nbr_block(win_in);
-    const int nb = blocks_for(num, bs);
+    const bool split = nbr_split(num, win_in, kSplitMaxForce);
+    const int bs = split ? kSplitBlock : nbr_block(win_in);
+    const int nb = blocks_for(num, split ? 64 : bs);
     const int loop = force_loop(win_in);
     if (win_in.rows && win_in.rows_stride < (uint32_t)num) return hipErrorInvalidValue;
     const size_t lds = force_lds(loop, bs);
     Win win = win_in;
     win.ntiles = nb;
-#define RTPS_FFUSED_Q(S, L, Q, GRID)                                                                                \
-    k_force<S, true, true, L, Q><<<GRID, bs, lds, st>>>(num, d_num, pos_s, nullptr, ve_packed, start, end, sp, g, win, \
+#define RTPS_FFUSED_Q(S, L, Q, SP, GRID)                                                                            \
+    k_force<S, true, true, L, Q, SP><<<GRID, bs, lds, st>>>(num, d_num, pos_s, nullptr, ve_packed, start, end, sp, g, win, \
                                                        force, xsph, vel_s, idx, gsrc, collision, gps.bnd_min,        \
                                                        gps.bnd_max, dt, pos_u, vel_u, veleval_u, color_s, color_u)
 #define RTPS_FFUSED_L(S, L)                                                                                         \
     if (win.tq) {                                                                                                   \
-        RTPS_FFUSED_Q(S, L, true, resident_grid((const void*)&k_force<S, true, true, L, true>, bs, lds, nb));        \
+        RTPS_FFUSED_Q(S, L, true, false,                                                                            \
+                      resident_grid((const void*)&k_force<S, true, true, L, true, false>, bs, lds, nb));             \
+    } else if (split) {                                                                                             \
+        RTPS_FFUSED_Q(S, L, false, true, nb);                                                                       \
     } else {                                                                                                        \
-        RTPS_FFUSED_Q(S, L, false, nb);                                                                             \
+        RTPS_FFUSED_Q(S, L, false, false, nb);                                                                      \
     }
 #define RTPS_FFUSED(S)                                                                                              \
     if (loop == kLoopStaged) { RTPS_FFUSED_L(S, kLoopStaged) }                                                      \
