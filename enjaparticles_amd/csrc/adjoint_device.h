@@ -22,6 +22,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "sph_device.h"
 
 namespace rtps {
@@ -29,26 +31,28 @@ namespace rtps {
 __device__ __forceinline__ float3 f3(float4 v) { return make_float3(v.x, v.y, v.z); }
 __device__ __forceinline__ float dot3(float3 a, float3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 
-// Neighbour rows of one launch: cell tables (already offset to the scene's
-// cells), sorted keys for the x windows (nullptr = plain rows), grid
-// resolution and the key bits shared by a whole row (the scene id of
-// segmented keys).
+// The neighbour rows of a recorded step (Win::rows: the forward step's density
+// kernel wrote them): for sorted particle i and row r = 3 (dz + 1) + (dy + 1)
+// the three words at rows + 3 (r * stride + i) hold its window [a, b) and the
+// rejection bits of the window's last min(b - a, 32) candidates.
 struct AdjRows {
-    const uint32_t* start;
-    const uint32_t* end;
-    const uint32_t* keys;
-    float rx, ry, rz;
-    uint32_t prefix;
+    const uint32_t* rows;
+    uint32_t stride;
 };
+
+// B2 and B3 run blocks of kAdjThreads = three waves over a tile of 64
+// particles, one plane (dz) of the neighbourhood each (the split tiles of
+// sph_kernels.hip, here at every size: a tile's sums must not depend on how
+// many tiles a launch holds).
+constexpr int kAdjThreads = 192;
 
 // Candidates per LDS copy of a row in B2 (4 records each) and B3 (a position
 // and a float each): 6 KB and 5 KB per wave.
 constexpr int kAdjStageCap = 96;
 constexpr int kAdjB3StageCap = 256;
-// LDS slice of the calling wave (float4 units): B2 needs 4 x kAdjStageCap,
-// B3 kAdjB3StageCap + kAdjB3StageCap / 4.
-constexpr int kAdjStageSlice = 4 * kAdjStageCap > kAdjB3StageCap + kAdjB3StageCap / 4
-                                   ? 4 * kAdjStageCap : kAdjB3StageCap + kAdjB3StageCap / 4;
+// LDS slice of a wave in B2 and B3 (float4 units).
+constexpr int kAdjB2Slice = 4 * kAdjStageCap;
+constexpr int kAdjB3Slice = kAdjB3StageCap + kAdjB3StageCap / 4;
 
 // The wave's live lanes and this lane's rank among them; the union [A, B) of
 // the live lanes' row windows (A >= B: no lane has candidates).
@@ -66,8 +70,8 @@ __device__ __forceinline__ void wave_range(uint32_t a, uint32_t b, uint32_t& A, 
 }
 
 // B1 for sorted particle i.  lam_x/v/e: adjoints of step n+1 (original
-// order).  Writes ga/gX (sorted), lam_v of step n (original order) and the
-// direct part of lam_x (sorted).
+// order; lam_v and lam_e may be null: zero).  Writes ga/gX (sorted), lam_v of
+// step n (original order) and the direct part of lam_x (sorted).
 __device__ __forceinline__ void adj_b1_body(int i, const uint32_t* __restrict__ idx, const float4* __restrict__ pos_s,
                                             const float4* __restrict__ vel_s, const float4* __restrict__ force_s,
                                             const rtps_sph_params& sp, const rtps_float4& bmin,
@@ -77,7 +81,8 @@ __device__ __forceinline__ void adj_b1_body(int i, const uint32_t* __restrict__ 
                                             float4* __restrict__ gX_s, float4* __restrict__ lam_v_out,
                                             float4* __restrict__ lxp_s) {
     const uint32_t o = idx[i];
-    const float3 lx = f3(lam_x[o]), lv = f3(lam_v[o]), le = f3(lam_e[o]);
+    const float3 none = make_float3(0.f, 0.f, 0.f);
+    const float3 lx = f3(lam_x[o]), lv = lam_v ? f3(lam_v[o]) : none, le = lam_e ? f3(lam_e[o]) : none;
     // adjoint of v' (x' = x + dt v', e' = (v + v')/2)
     const float3 lvb = make_float3(lv.x + dt * lx.x + 0.5f * le.x, lv.y + dt * lx.y + 0.5f * le.y,
                                    lv.z + dt * lx.z + 0.5f * le.z);
@@ -132,16 +137,85 @@ __device__ __forceinline__ void adj_b1_body(int i, const uint32_t* __restrict__ 
     lxp_s[i] = make_float4(gx.x, gx.y, gx.z, 0.f);
 }
 
-// B2 for sorted particle i: pair terms.  ve_s = veleval.xyz | density
-// (sorted).  Writes gx2 (d/dx of the pair terms), ge (d/de), grho (sorted);
-// adds particle i's terms of dL/dmu and dL/dK to gmu, gK.  Hardware rsq / rcp
-// (~1 ulp) replace the square root and the divisions.
-__device__ __forceinline__ void adj_b2_body(int i, const float4* __restrict__ pos_s, const float4* __restrict__ ve_s,
-                                            const float4* __restrict__ ga_s, const float4* __restrict__ gX_s,
-                                            const AdjRows& rows, const rtps_sph_params& sp, const Grid& g,
-                                            float4* __restrict__ gx2_s, float4* __restrict__ ge_s,
-                                            float* __restrict__ grho_s, float& gmu, float& gK,
-                                            float4* __restrict__ stage) {
+// The accepted candidates of particle i in plane dz of its recorded rows, in
+// ascending order.  Per row the wave's live lanes copy the union of their
+// windows (when it holds at most CAP candidates) into the wave's LDS slice:
+// `copy(t, j)` stores what candidate j needs besides its position at slot t,
+// the position goes to st[t].  Wider unions are read from global memory.
+// A lane's window is taken in chunks, the first ragged (1-32 candidates), the
+// rest 32 long, so that the last chunk is what the record's bits cover; only
+// earlier chunks are tested again.  pair(staged, o, r, r2): slot or index o of
+// a candidate within h (not i itself), r = p_i - p_j.
+template <int CAP, typename Copy, typename Pair>
+__device__ __forceinline__ void adj_plane(int i, int dz, const AdjRows& rows, const float4& pi, float h2,
+                                          const float4* __restrict__ pos_s, float4* __restrict__ st, Copy&& copy,
+                                          Pair&& pair) {
+    const WaveLanes wl = wave_lanes();
+    uint32_t a[3], b[3], rej_last[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {   // the plane's records are loaded together
+        const uint32_t* __restrict__ o = rows.rows + 3 * ((size_t)(3 * (dz + 1) + k) * rows.stride + (size_t)i);
+        a[k] = o[0];
+        b[k] = o[1];
+        rej_last[k] = o[2];
+    }
+    auto walk = [&](auto staged, uint32_t a, uint32_t b, uint32_t off, uint32_t last) {
+        const float4* __restrict__ P = decltype(staged)::value ? st : pos_s;
+        uint32_t n = ((b - a - 1u) & 31u) + 1u;
+        for (uint32_t j0 = a; j0 < b; j0 += n, n = 32u) {
+            const uint32_t o0 = j0 - off;
+            uint32_t rej = last;
+            if (j0 + n != b) {
+                rej = 0u;
+                for (uint32_t k = 0; k < n; ++k) {
+                    const float4 p = P[o0 + k];
+                    rej = rej_bit(rej, h2_minus_r2(pi.x - p.x, pi.y - p.y, pi.z - p.z, h2));
+                }
+            }
+            uint32_t m = __builtin_bitreverse32(~rej) >> (32u - n);   // bit t = candidate t
+            const uint32_t self = (uint32_t)i - j0;   // the particle itself passes (r = 0): drop it
+            if (self < n) m &= ~(1u << self);
+            while (m != 0u) {
+                const uint32_t o = o0 + (uint32_t)__builtin_ctz(m);
+                m &= m - 1u;
+                const float4 p = P[o];
+                const float3 r = make_float3(pi.x - p.x, pi.y - p.y, pi.z - p.z);
+                pair(staged, o, r, dot3(r, r));
+            }
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        uint32_t A, B;
+        wave_range(a[k], b[k], A, B);
+        if (B <= A) continue;
+        if (B - A <= (uint32_t)CAP) {
+            for (uint32_t t = wl.rank; t < B - A; t += wl.n) {
+                st[t] = pos_s[A + t];
+                copy(t, A + t);
+            }
+            __builtin_amdgcn_wave_barrier();   // the copies before any lane reads them
+            walk(std::true_type{}, a[k], b[k], A, rej_last[k]);
+            __builtin_amdgcn_wave_barrier();   // every read before the next row's copies
+        } else {
+            walk(std::false_type{}, a[k], b[k], 0u, rej_last[k]);
+        }
+    }
+}
+
+// What B2 sums for a particle.
+struct B2Acc {
+    float3 gx, ge;
+    float grho, gmu, gK;
+};
+
+// B2's pair terms of sorted particle i over plane dz.  ve_s = veleval.xyz |
+// density (sorted).  Hardware rsq / rcp (~1 ulp) replace the square root and
+// the divisions.  stage: kAdjB2Slice of the wave.
+__device__ __forceinline__ B2Acc adj_b2_plane(int i, int dz, const float4* __restrict__ pos_s,
+                                              const float4* __restrict__ ve_s, const float4* __restrict__ ga_s,
+                                              const float4* __restrict__ gX_s, const AdjRows& rows,
+                                              const rtps_sph_params& sp, float4* __restrict__ stage) {
     const float h = sp.smoothing_distance, h2 = h * h, eps = sp.EPSILON, eps2 = eps * eps;
     const float m = sp.mass, rho0 = sp.rest_density, K = sp.K, mu = sp.viscosity;
     const float cp = -0.5f * sp.wspiky_d_coef, cv = sp.wvisc_dd_coef;
@@ -151,7 +225,7 @@ __device__ __forceinline__ void adj_b2_body(int i, const float4* __restrict__ po
     const float ri = vei.w;
     const float inv_ri = __builtin_amdgcn_rcpf(ri);
     float3 gx = make_float3(0, 0, 0), ge = make_float3(0, 0, 0);
-    float grho = 0.f;
+    float grho = 0.f, gmu = 0.f, gK = 0.f;
     // one accepted pair (within_h, j != i)
     auto pair = [&](const float3 r, const float q2, const float4 vej, const float4 gaj4, const float4 gXj4) {
         const float3 ej = f3(vej), gaj = f3(gaj4), gXj = f3(gXj4);
@@ -207,237 +281,121 @@ __device__ __forceinline__ void adj_b2_body(int i, const float4* __restrict__ po
         gx.z += yr * r.z;
         grho += -yk * inv_D * dedgX;
     };
-    const int3 c = grid_cell(pi.x, pi.y, pi.z, g);
-    const WindowCtx wc = window_ctx(pi.x, pi.y, pi.z, g, c, h, rows.keys, rows.rx, rows.ry, rows.rz);
-    // candidate j of a row: P[j - off], V / GA / GX[j - off]
-    auto walk = [&](const float4* __restrict__ P, const float4* __restrict__ V, const float4* __restrict__ GA,
-                    const float4* __restrict__ GX, uint32_t a, uint32_t b, uint32_t off) {
-        uint32_t j = a;
-        for (; j + kGroup <= b; j += kGroup) {   // positions, then the accepted records, loaded together
-            float4 p[kGroup];
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k) p[k] = P[j + k - off];
-            float3 r[kGroup];
-            float q2[kGroup];
-            bool ok[kGroup];
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k) {
-                r[k] = make_float3(pi.x - p[k].x, pi.y - p[k].y, pi.z - p[k].z);
-                q2[k] = dot3(r[k], r[k]);
-                ok[k] = within_h(h2_minus_r2(r[k].x, r[k].y, r[k].z, h2)) && j + k != (uint32_t)i;
-            }
-            float4 v[kGroup], ga[kGroup], gX[kGroup];
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k)
-                if (ok[k]) {
-                    v[k] = V[j + k - off];
-                    ga[k] = GA[j + k - off];
-                    gX[k] = GX[j + k - off];
-                }
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k)
-                if (ok[k]) pair(r[k], q2[k], v[k], ga[k], gX[k]);
-        }
-        for (; j < b; ++j) {
-            const float4 pj = P[j - off];
-            const float3 r = make_float3(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z);
-            const float q2 = dot3(r, r);
-            if (within_h(h2_minus_r2(r.x, r.y, r.z, h2)) && j != (uint32_t)i)
-                pair(r, q2, V[j - off], GA[j - off], GX[j - off]);
-        }
-    };
-    // rows of at most kAdjStageCap wave-wide candidates are copied once per
-    // wave into `stage` (full-line loads) and read from there
-    const WaveLanes wl = wave_lanes();
-    float4* __restrict__ sp_ = stage;
     float4* __restrict__ sv = stage + kAdjStageCap;
     float4* __restrict__ sga = stage + 2 * kAdjStageCap;
     float4* __restrict__ sgx = stage + 3 * kAdjStageCap;
-    // the staged copies, a lane's window in chunks of up to 32 candidates:
-    // the tests of a chunk shift one bit per candidate into a mask (the
-    // chunk's first candidate ends in its highest bit), the particle's own
-    // bit is cleared, then the pair terms run once per set bit, highest
-    // first: the same pairs in the same ascending order as walk (the same
-    // sums), with the wave's pair iterations its lanes' largest accepted
-    // count instead of their longest window
-    auto walk_bits = [&](uint32_t a, uint32_t b, uint32_t off) {
-        for (uint32_t j0 = a; j0 < b; j0 += 32u) {
-            const uint32_t n = min(b - j0, 32u);
-            const float4* __restrict__ pc = sp_ + (j0 - off);
-            uint32_t mk = 0u, k = 0u;
-            auto test = [&](const float4 p) {
-                const float3 r = make_float3(pi.x - p.x, pi.y - p.y, pi.z - p.z);
-                mk = mk + mk + (within_h(h2_minus_r2(r.x, r.y, r.z, h2)) ? 1u : 0u);
-            };
-            for (; k + kGroup <= n; k += kGroup) {
-                float4 q[kGroup];
-#pragma unroll
-                for (int t = 0; t < kGroup; ++t) q[t] = pc[k + t];
-#pragma unroll
-                for (int t = 0; t < kGroup; ++t) test(q[t]);
-            }
-            for (; k < n; ++k) test(pc[k]);
-            const uint32_t self = (uint32_t)i - j0;   // the particle itself passes (r = 0): drop it
-            if (self < n) mk &= ~(1u << (n - 1u - self));
-            while (mk != 0u) {
-                const uint32_t hb = 31u - (uint32_t)__builtin_clz(mk);
-                mk ^= 1u << hb;
-                const uint32_t t = n - 1u - hb;
-                const float4 p = pc[t];
-                const float3 r = make_float3(pi.x - p.x, pi.y - p.y, pi.z - p.z);
-                const uint32_t o = j0 + t - off;
-                pair(r, dot3(r, r), sv[o], sga[o], sgx[o]);
-            }
-        }
-    };
-    for (int dz = -1; dz <= 1; ++dz)
-        for (int dy = -1; dy <= 1; ++dy) {
-            uint32_t a, b, A, B;
-            row_window(wc, c, dy, dz, h2, g, rows.start, rows.end, rows.keys, a, b, rows.prefix);
-            wave_range(a, b, A, B);
-            if (B <= A) continue;
-            if (B - A <= (uint32_t)kAdjStageCap) {
-                for (uint32_t t = wl.rank; t < B - A; t += wl.n) {
-                    sp_[t] = pos_s[A + t];
-                    sv[t] = ve_s[A + t];
-                    sga[t] = ga_s[A + t];
-                    sgx[t] = gX_s[A + t];
-                }
-                __builtin_amdgcn_wave_barrier();   // the copies before any lane reads them
-                walk_bits(a, b, A);
-                __builtin_amdgcn_wave_barrier();   // every read before the next row's copies
-            } else {
-                walk(pos_s, ve_s, ga_s, gX_s, a, b, 0u);
-            }
-        }
-    gx2_s[i] = make_float4(gx.x, gx.y, gx.z, 0.f);
-    ge_s[i] = make_float4(ge.x, ge.y, ge.z, 0.f);
-    grho_s[i] = grho;
+    adj_plane<kAdjStageCap>(
+        i, dz, rows, pi, h2, pos_s, stage,
+        [&](uint32_t t, uint32_t j) {
+            sv[t] = ve_s[j];
+            sga[t] = ga_s[j];
+            sgx[t] = gX_s[j];
+        },
+        [&](auto staged, uint32_t o, const float3 r, float r2) {
+            if constexpr (decltype(staged)::value) pair(r, r2, sv[o], sga[o], sgx[o]);
+            else pair(r, r2, ve_s[o], ga_s[o], gX_s[o]);
+        });
+    return B2Acc{gx, ge, grho, gmu, gK};
 }
 
-// B3 for sorted particle i: density backwards and the scatter of lambda_x,
-// lambda_e of step n.
-__device__ __forceinline__ void adj_b3_body(int i, const uint32_t* __restrict__ idx, const float4* __restrict__ pos_s,
-                                            const float* __restrict__ grho_s, const float4* __restrict__ lxp_s,
-                                            const float4* __restrict__ gx2_s, const float4* __restrict__ ge_s,
-                                            const AdjRows& rows, const rtps_sph_params& sp, const Grid& g,
-                                            float4* __restrict__ lam_x_out, float4* __restrict__ lam_e_out,
-                                            float4* __restrict__ stage) {
-    const float h = sp.smoothing_distance, h2 = h * h;
-    const float crho = sp.wpoly6_coef * sp.mass;
-    const float4 pi = pos_s[i];
-    const float gri = grho_s[i];
+// B2 for the block's tile: wave w takes plane w - 1 of particle i (the same 64
+// particles in each wave; valid: i is one of them); wave 0 adds the planes in
+// ascending order and writes gx2 (d/dx of the pair terms), ge (d/de) and grho
+// (sorted), and the tile's share of dL/dmu and dL/dK goes to *partial.
+__device__ __forceinline__ void adj_b2_tile(int i, bool valid, const float4* __restrict__ pos_s,
+                                            const float4* __restrict__ ve_s, const float4* __restrict__ ga_s,
+                                            const float4* __restrict__ gX_s, const AdjRows& rows,
+                                            const rtps_sph_params& sp, float4* __restrict__ gx2_s,
+                                            float4* __restrict__ ge_s, float* __restrict__ grho_s,
+                                            float2* __restrict__ partial) {
+    __shared__ float4 stage[3][kAdjB2Slice];
+    __shared__ float2 share[3];
+    const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+    B2Acc s = {make_float3(0, 0, 0), make_float3(0, 0, 0), 0.f, 0.f, 0.f};
+    if (valid) s = adj_b2_plane(i, w - 1, pos_s, ve_s, ga_s, gX_s, rows, sp, stage[w]);
+    for (int off = 32; off > 0; off >>= 1) {   // idle lanes add zero
+        s.gmu += __shfl_down(s.gmu, off, 64);
+        s.gK += __shfl_down(s.gK, off, 64);
+    }
+    if (lane == 0) share[w] = make_float2(s.gmu, s.gK);
+    __builtin_amdgcn_wave_barrier();   // the last row's reads before the slice's reuse
+    if (w > 0) {
+        float* __restrict__ p = (float*)stage[w] + lane;
+        p[0] = s.gx.x; p[64] = s.gx.y; p[128] = s.gx.z;
+        p[192] = s.ge.x; p[256] = s.ge.y; p[320] = s.ge.z;
+        p[384] = s.grho;
+    }
+    __syncthreads();
+    if (w > 0) return;
+    if (lane == 0)
+        *partial = make_float2((share[0].x + share[1].x) + share[2].x, (share[0].y + share[1].y) + share[2].y);
+    if (!valid) return;
+    for (int q = 1; q <= 2; ++q) {
+        const float* __restrict__ p = (const float*)stage[q] + lane;
+        s.gx.x += p[0]; s.gx.y += p[64]; s.gx.z += p[128];
+        s.ge.x += p[192]; s.ge.y += p[256]; s.ge.z += p[320];
+        s.grho += p[384];
+    }
+    gx2_s[i] = make_float4(s.gx.x, s.gx.y, s.gx.z, 0.f);
+    ge_s[i] = make_float4(s.ge.x, s.ge.y, s.ge.z, 0.f);
+    grho_s[i] = s.grho;
+}
+
+// B3 for the block's tile (as adj_b2_tile): density backwards and the scatter
+// of lambda_x, lambda_e of step n (lam_e_out may be null).
+__device__ __forceinline__ void adj_b3_tile(int i, bool valid, const uint32_t* __restrict__ idx,
+                                            const float4* __restrict__ pos_s, const float* __restrict__ grho_s,
+                                            const float4* __restrict__ lxp_s, const float4* __restrict__ gx2_s,
+                                            const float4* __restrict__ ge_s, const AdjRows& rows,
+                                            const rtps_sph_params& sp, float4* __restrict__ lam_x_out,
+                                            float4* __restrict__ lam_e_out) {
+    __shared__ float4 stage[3][kAdjB3Slice];
+    const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
     float3 gx = make_float3(0, 0, 0);
-    const int3 c = grid_cell(pi.x, pi.y, pi.z, g);
-    const WindowCtx wc = window_ctx(pi.x, pi.y, pi.z, g, c, h, rows.keys, rows.rx, rows.ry, rows.rz);
-    auto term = [&](float4 pj, float grj, bool ok) {
-        const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
-        const float q2 = rx * rx + ry * ry + rz * rz;
-        if (!(ok && q2 <= h2)) return;
-        const float t = h2 - q2;
-        const float k = crho * (-6.f) * t * t * (gri + grj);
-        gx.x += k * rx;
-        gx.y += k * ry;
-        gx.z += k * rz;
-    };
-    // candidate j of a row: P[j - off], GR[j - off]
-    auto walk = [&](const float4* __restrict__ P, const float* __restrict__ GR, uint32_t a, uint32_t b,
-                    uint32_t off) {
-        uint32_t j = a;
-        for (; j + kGroup <= b; j += kGroup) {   // loads of a group issued together
-            float4 p[kGroup];
-            float gr[kGroup];
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k) {
-                p[k] = P[j + k - off];
-                gr[k] = GR[j + k - off];
-            }
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k) term(p[k], gr[k], j + k != (uint32_t)i);
-        }
-        for (; j < b; ++j) term(P[j - off], GR[j - off], j != (uint32_t)i);
-    };
-    // rows of at most kAdjB3StageCap wave-wide candidates are copied once per
-    // wave into `stage` (full-line loads) and read from there
-    const WaveLanes wl = wave_lanes();
-    float4* __restrict__ sp_ = stage;
-    float* __restrict__ sgr = (float*)(stage + kAdjB3StageCap);
-    for (int dz = -1; dz <= 1; ++dz)
-        for (int dy = -1; dy <= 1; ++dy) {
-            uint32_t a, b, A, B;
-            row_window(wc, c, dy, dz, h2, g, rows.start, rows.end, rows.keys, a, b, rows.prefix);
-            wave_range(a, b, A, B);
-            if (B <= A) continue;
-            if (B - A <= (uint32_t)kAdjB3StageCap) {
-                for (uint32_t t = wl.rank; t < B - A; t += wl.n) {
-                    sp_[t] = pos_s[A + t];
-                    sgr[t] = grho_s[A + t];
-                }
-                __builtin_amdgcn_wave_barrier();   // the copies before any lane reads them
-                walk(sp_, sgr, a, b, A);
-                __builtin_amdgcn_wave_barrier();   // every read before the next row's copies
-            } else {
-                walk(pos_s, grho_s, a, b, 0u);
-            }
-        }
+    if (valid) {
+        const float h = sp.smoothing_distance, h2 = h * h;
+        const float c6 = sp.wpoly6_coef * sp.mass * -6.f;
+        const float gri = grho_s[i];
+        float* __restrict__ sgr = (float*)(stage[w] + kAdjB3StageCap);
+        adj_plane<kAdjB3StageCap>(
+            i, w - 1, rows, pos_s[i], h2, pos_s, stage[w], [&](uint32_t t, uint32_t j) { sgr[t] = grho_s[j]; },
+            [&](auto staged, uint32_t o, const float3 r, float r2) {
+                float grj;
+                if constexpr (decltype(staged)::value) grj = sgr[o];
+                else grj = grho_s[o];
+                const float t = h2 - r2;
+                const float k = c6 * t * t * (gri + grj);
+                gx.x += k * r.x;
+                gx.y += k * r.y;
+                gx.z += k * r.z;
+            });
+    }
+    __builtin_amdgcn_wave_barrier();   // the last row's reads before the slice's reuse
+    if (w > 0) {
+        float* __restrict__ p = (float*)stage[w] + lane;
+        p[0] = gx.x; p[64] = gx.y; p[128] = gx.z;
+    }
+    __syncthreads();
+    if (w > 0 || !valid) return;
+    for (int q = 1; q <= 2; ++q) {
+        const float* __restrict__ p = (const float*)stage[q] + lane;
+        gx.x += p[0]; gx.y += p[64]; gx.z += p[128];
+    }
     const float4 lp = lxp_s[i], g2 = gx2_s[i];
     const uint32_t o = idx[i];
     lam_x_out[o] = make_float4(lp.x + g2.x + gx.x, lp.y + g2.y + gx.y, lp.z + g2.z + gx.z, 0.f);
-    lam_e_out[o] = ge_s[i];
+    if (lam_e_out) lam_e_out[o] = ge_s[i];
 }
 
-// Forward integration of a recorded step for sorted particle i: walls (on a
-// copy of the stored SPH force, which B1 needs unchanged) and leapfrog,
-// scattered to the next state.
-__device__ __forceinline__ void adj_integrate_body(int i, const float4* __restrict__ pos_s,
-                                                   const float4* __restrict__ vel_s,
-                                                   const float4* __restrict__ force_s,
-                                                   const float4* __restrict__ xsph_s,
-                                                   const uint32_t* __restrict__ idx, const rtps_sph_params& sp,
-                                                   const rtps_float4& bmin, const rtps_float4& bmax, int collision,
-                                                   float dt, float4* __restrict__ pos_u, float4* __restrict__ vel_u,
-                                                   float4* __restrict__ veleval_u) {
-    const float4 p = pos_s[i], v = vel_s[i];
-    float4 F = force_s[i];
-    if (collision) collision_wall(F, p, v, sp, bmin, bmax);
-    float4 po, vo, eo;
-    leapfrog(p, v, F, xsph_s[i], sp, dt, po, vo, eo);
-    const uint32_t o = idx[i];
-    pos_u[o] = po;
-    vel_u[o] = vo;
-    veleval_u[o] = eo;
-}
-
-// Deterministic wave64 + block sum of (gmu, gK) into partial[slot]; every
-// thread of the block must call it.
-template <int BLOCK>
-__device__ __forceinline__ void adj_block_partial(float gmu, float gK, float2* __restrict__ partial, int slot) {
-    __shared__ float2 red[BLOCK / 64];
-    for (int off = 32; off > 0; off >>= 1) {
-        gmu += __shfl_down(gmu, off, 64);
-        gK += __shfl_down(gK, off, 64);
-    }
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(gmu, gK);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float2 t = make_float2(0.f, 0.f);
-        for (int w = 0; w < BLOCK / 64; ++w) {
-            t.x += red[w].x;
-            t.y += red[w].y;
-        }
-        partial[slot] = t;
-    }
-}
-
-// Sum of partial[first, first + n) in FP64, fixed order, by one block of 256
-// threads; adds the totals to acc[0], acc[1].
-__device__ __forceinline__ void adj_reduce_body(const float2* __restrict__ partial, int first, int n,
-                                                double* __restrict__ acc) {
+// Sum of the n tile shares at partial in FP64, fixed order, by one block of
+// 256 threads, into out[0], out[1].
+__device__ __forceinline__ void adj_reduce_body(const float2* __restrict__ partial, int n,
+                                                double* __restrict__ out) {
     __shared__ double s0[256], s1[256];
     double a = 0.0, b = 0.0;
     for (int k = threadIdx.x; k < n; k += blockDim.x) {
-        a += (double)partial[first + k].x;
-        b += (double)partial[first + k].y;
+        a += (double)partial[k].x;
+        b += (double)partial[k].y;
     }
     s0[threadIdx.x] = a;
     s1[threadIdx.x] = b;
@@ -450,8 +408,8 @@ __device__ __forceinline__ void adj_reduce_body(const float2* __restrict__ parti
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        acc[0] += s0[0];
-        acc[1] += s1[0];
+        out[0] = s0[0];
+        out[1] = s1[0];
     }
 }
 

@@ -113,7 +113,7 @@ uint32_t* rows_of(const rtps_batch* b) { return b->opt_rows ? b->rows : nullptr;
 int launch_density_b(rtps_batch* b, const PairsCfg& c) {
     RTPS_TRY_HIP(launch_pairs_b(kPairsDensity, c, grid_of(b, c), items_of(b, c), nitems_of(b, c), b->queues,
                                 b->scenes, b->d_num, b->pos_s, b->start, b->end, b->keys_sorted, b->ve_s, b->vel_s,
-                                b->idx_sorted, b->pos_u, b->vel_u, b->veleval_u, b->stream, nullptr, nullptr, b->sub,
+                                b->idx_sorted, b->pos_u, b->vel_u, b->veleval_u, b->stream, b->sub,
                                 rows_of(b), (uint32_t)b->T));
     return RTPS_OK;
 }
@@ -122,7 +122,7 @@ int launch_force_b(rtps_batch* b, const PairsCfg& c) {
     RTPS_TRY_HIP(launch_pairs_b(kPairsForceStep, c, grid_of(b, c), items_of(b, c), nitems_of(b, c),
                                 b->queues, b->scenes, b->d_num, b->pos_s, b->start, b->end,
                                 b->keys_sorted, b->ve_s, b->vel_s, b->idx_sorted, b->pos_u, b->vel_u, b->veleval_u,
-                                b->stream, nullptr, nullptr, b->sub, rows_of(b), (uint32_t)b->T));
+                                b->stream, b->sub, rows_of(b), (uint32_t)b->T));
     return RTPS_OK;
 }
 
@@ -396,12 +396,12 @@ int build_batch_layout(int num_scenes, const int* n_settings, const char* const*
     L.item_first.assign(num_scenes + 1, 0);
     for (int s = 0; s < num_scenes; ++s) {
         const SceneDev& d = L.scenes[s];
-        L.item_first[s] = (int)L.items.size();
+        L.item_first[s] = (int)L.items64.size();
         for (int f = 0; f < d.cap; f += 256) L.items.push_back(BatchItem{s, d.off + f, std::min(256, d.cap - f), 0});
         for (int f = 0; f < d.cap; f += 128) L.items128.push_back(BatchItem{s, d.off + f, std::min(128, d.cap - f), 0});
         for (int f = 0; f < d.cap; f += 64) L.items64.push_back(BatchItem{s, d.off + f, std::min(64, d.cap - f), 0});
     }
-    L.item_first[num_scenes] = (int)L.items.size();
+    L.item_first[num_scenes] = (int)L.items64.size();
     return RTPS_OK;
 }
 

@@ -37,12 +37,12 @@ hipError_t launch_hash_b(int T, const uint16_t* sid, const SceneDev* scenes, con
 // sub (optional): sub-cell start table, 16 entries per cell of every scene
 hipError_t launch_cellindices_b(int T, const uint32_t* keys, const SceneDev* scenes, uint32_t* start, uint32_t* end,
                                 hipStream_t st, uint32_t* sub = nullptr);
-constexpr int kPairsDensity = 0, kPairsForceStep = 1, kPairsForceStore = 2;
+constexpr int kPairsDensity = 0, kPairsForceStep = 1;
 // Launch configuration of a persistent pair kernel: `block` threads per block
 // (= slots per work item: 64, 128 or 256) and the register budget of `waves`
 // waves per SIMD (3, 4, 5 or 6: at most 168, 128, 96 or 80 VGPRs); the grid
 // is CUs x waves x 256 / block blocks.  The density kernel is built for 4, 5
-// and 6 waves; the force kernels for 3, 4 and 5 (5 fits their registers only
+// and 6 waves; the force kernel for 3, 4 and 5 (5 fits their registers only
 // on recorded rows: looking the rows up, their live values exceed the 96
 // registers of 5 waves and spill to scratch memory).  The batched system's
 // autotuner picks one per kernel; the defaults are 256 threads at 5 waves
@@ -58,8 +58,16 @@ hipError_t launch_pairs_b(int mode, const PairsCfg& cfg, int grid, const BatchIt
                           const SceneDev* scenes, const int* d_num, const float4* pos_s, const uint32_t* start,
                           const uint32_t* end, const uint32_t* keys, float4* ve, const float4* vel_s,
                           const uint32_t* idx, float4* pos_u, float4* vel_u, float4* veleval_u, hipStream_t st,
-                          float4* force_out = nullptr, float4* xsph_out = nullptr, const uint32_t* sub = nullptr,
-                          uint32_t* rows = nullptr, uint32_t rows_stride = 0);
+                          const uint32_t* sub = nullptr, uint32_t* rows = nullptr, uint32_t rows_stride = 0);
+// The same step with one block per 64-slot item, split over three waves
+// (recorded steps: every slot holds a particle, no deletion; rows required).
+// force_out: the SPH force in sorted order (may be null); *left is set when a
+// particle lies outside its scene's grid.
+hipError_t launch_pairs_split_b(int mode, int n_items64, const BatchItem* items64, const SceneDev* scenes,
+                                const float4* pos_s, const uint32_t* start, const uint32_t* end,
+                                const uint32_t* keys, float4* ve, const float4* vel_s, const uint32_t* idx,
+                                float4* pos_u, float4* vel_u, float4* veleval_u, float4* force_out, int* left,
+                                const uint32_t* sub, uint32_t* rows, uint32_t rows_stride, hipStream_t st);
 hipError_t launch_commit_b(int S, const SceneDev* scenes, int* d_num, const uint32_t* start, hipStream_t st);
 
 }  // namespace rtps

@@ -127,7 +127,7 @@ int rtps_density(int num, const rtps_float4* pos_s, const uint32_t* start, const
     if (num == 0) return RTPS_OK;
     RTPS_CHECK(pos_s && start && end && density, "rtps_density: null buffer");
     Win plain{nullptr, 0.f, 0.f, 0.f, 0, 0, -1};
-    plain.split = true;
+    plain.split = Win::kSmall;
     RTPS_HIP(launch_density(num, nullptr, (const float4*)pos_s, start, end, *sphp, make_grid(*gps), plain, density,
                             nullptr, S(stream)));
     return RTPS_OK;
@@ -140,7 +140,7 @@ int rtps_force(int num, const rtps_float4* pos_s, const float* density, const rt
     if (num == 0) return RTPS_OK;
     RTPS_CHECK(pos_s && density && veleval_s && start && end && force && xsph, "rtps_force: null buffer");
     Win plain{nullptr, 0.f, 0.f, 0.f, 0, 0, -1};
-    plain.split = true;
+    plain.split = Win::kSmall;
     RTPS_HIP(launch_force(num, nullptr, (const float4*)pos_s, density, (const float4*)veleval_s, false, start, end,
                           *sphp, make_grid(*gps), plain, (float4*)force, (float4*)xsph, S(stream)));
     return RTPS_OK;

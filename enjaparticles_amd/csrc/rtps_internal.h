@@ -52,17 +52,20 @@ hipError_t launch_read_nc(const uint32_t* start, int nb_cells, int* nc, hipStrea
 hipError_t launch_permute(int num, const int* d_num, const uint32_t* idx, const float4* pu, const float4* vu,
                           const float4* eu, float4* ps, float4* vs, float4* es, hipStream_t st,
                           const float4* cu = nullptr, float4* cs = nullptr);
-// launch_cellindices and launch_permute in one kernel (the system's step)
+// launch_cellindices and launch_permute in one kernel (the system's step);
+// left (optional) is set to 1 when a particle lies outside the grid
 hipError_t launch_cells_permute(int num, const int* d_num, const uint32_t* keys, int nb_cells, uint32_t* start,
                                 uint32_t* end, int sub_bits, uint32_t* sub, const uint32_t* idx, const float4* pu,
                                 const float4* vu, const float4* eu, float4* ps, float4* vs, float4* es,
-                                hipStream_t st, const float4* cu = nullptr, float4* cs = nullptr);
+                                hipStream_t st, const float4* cu = nullptr, float4* cs = nullptr,
+                                int* left = nullptr);
 hipError_t launch_density(int num, const int* d_num, const float4* pos_s, const uint32_t* start, const uint32_t* end,
                           const rtps_sph_params& sp, const Grid& g, const Win& win, float* dens, float4* packed,
                           hipStream_t st);
 hipError_t launch_force(int num, int* d_num, const float4* pos_s, const float* dens, const float4* ve,
                         bool packed, const uint32_t* start, const uint32_t* end, const rtps_sph_params& sp,
                         const Grid& g, const Win& win, float4* force, float4* xsph, hipStream_t st);
+// force, xsph (optional): stored as well
 hipError_t launch_force_fused(int num, int* d_num, const float4* pos_s, const float4* ve_packed,
                               const uint32_t* start, const uint32_t* end, const rtps_sph_params& sp, const Grid& g,
                               const Win& win, float4* force, float4* xsph, const float4* vel_s, const uint32_t* idx,

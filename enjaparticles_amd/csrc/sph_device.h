@@ -159,9 +159,10 @@ struct Win {
     // testing those candidates again.
     uint32_t* rows = nullptr;
     uint32_t rows_stride = 0;   // particles per row plane (at least the particle count)
-    // small launches may split their tiles over three waves, one per plane of
+    // whether the launches split their tiles over three waves, one per plane of
     // the neighbourhood (other roundings than the unsplit kernels' single sequence)
-    bool split = false;
+    enum Split { kNever, kSmall, kAlways };
+    Split split = kNever;
 };
 
 // Candidates per group in the neighbour loops (loads in flight per lane).

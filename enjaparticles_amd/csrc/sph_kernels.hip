@@ -125,12 +125,14 @@ __global__ __launch_bounds__(kBlock) void k_cells_permute(int num_host, const in
                                                           const float4* __restrict__ pu, const float4* __restrict__ vu,
                                                           const float4* __restrict__ eu, float4* __restrict__ ps,
                                                           float4* __restrict__ vs, float4* __restrict__ es,
-                                                          const float4* __restrict__ cu, float4* __restrict__ cs) {
+                                                          const float4* __restrict__ cu, float4* __restrict__ cs,
+                                                          int* __restrict__ left) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int num = d_num ? *d_num : num_host;
     if (i >= num) return;
     permute_one(i, idx, pu, vu, eu, ps, vs, es, cu, cs);
     cellindices_one(i, num, keys, nb_cells, start, end, sub_bits, sub);
+    if (left && (keys[i] >> sub_bits) >= nb_cells) *left = 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -142,7 +144,8 @@ __global__ __launch_bounds__(kBlock) void k_cells_permute(int num_host, const in
 // Split, they are three waves a SIMD with chains a third as long.  The planes'
 // sums are added at the end, so the roundings differ from the unsplit kernels',
 // and the plain step, whose bits callers compare with other launches', stays
-// unsplit.  Measured with windowed rows (us, unsplit / split): density
+// unsplit.  (The recorded steps of the adjoint split at any size, so that a
+// rollout's bits do not change at a count.)  Measured with windowed rows (us, unsplit / split): density
 // 16.5 / 8.7 at 2,048 particles, 25.3 / 14.6 at 65,536, 40.2 / 37.8 at 262,144
 // and 161 / 160 at 1,048,576 (settled pools); force 15.4 / 9.4, 43 / 25.3,
 // 71 / 64 and 234 / 247, and 31 / 33 at 262,144 at rest.  With the whole rows of
@@ -328,7 +331,7 @@ __global__ __launch_bounds__(SPLIT ? kSplitBlock : kBlock) __attribute__((amdgpu
 // density come from one float4 (xyz = veleval, w = density).  FUSED: the
 // epilogue goes on to the point sources (gravity.cl), the walls
 // (collision_wall.cl) and the leapfrog step (leapfrog.cl), scattering to the
-// unsorted arrays; force/xsph are then stored only if force_out != nullptr.
+// unsorted arrays; force and xsph are then stored only where their arrays are given.
 //
 // LOOP (the force-loop variant):
 // kLoopDirect: each lane walks its own window of every row in global memory,
@@ -650,7 +653,8 @@ __device__ __forceinline__ void force_tile(int tile, int num_host, int* d_num,
     }
     float4 F, X;
     force_epilogue(acc, PACKED ? ve_in[i].w : dens_in[i], sp, F, X);
-    if (force_out) { force_out[i] = F; xsph_out[i] = X; }
+    if (force_out) force_out[i] = F;
+    if (xsph_out) xsph_out[i] = X;
     if (FUSED) {
         const float4 p_unscaled = pos_s[i];
         gravity_sources(F, p_unscaled, gsrc, sp.simulation_scale);
@@ -854,9 +858,10 @@ int g_force_variant = kLoopStagedBits;
 // Threads per block of a neighbour launch (a multiple of 64, at most kBlock)
 // and its force-loop variant.
 static inline int nbr_block(const Win& w) { return w.block > 0 && w.block <= kBlock && w.block % 64 == 0 ? w.block : kBlock; }
-// Whether a neighbour launch splits its tiles (never with the tile queues or
-// a block size fixed by the caller: Win::split).
-static inline bool nbr_split(int num, const Win& w, int most) { return w.split && !w.tq && num <= most; }
+// Whether a neighbour launch splits its tiles (most: the particles up to which that pays).
+static inline bool nbr_split(int num, const Win& w, int most) {
+    return w.split == Win::kAlways || (w.split == Win::kSmall && num <= most);
+}
 static inline int nbr_variant(const Win& w) {
     const int v = w.variant >= 0 ? w.variant : g_force_variant;
     return v == kLoopStaged || v == kLoopStagedBits ? v : kLoopDirect;
@@ -885,12 +890,12 @@ hipError_t launch_cellindices(int num, const int* d_num, const uint32_t* keys, i
 hipError_t launch_cells_permute(int num, const int* d_num, const uint32_t* keys, int nb_cells, uint32_t* start,
                                 uint32_t* end, int sub_bits, uint32_t* sub, const uint32_t* idx, const float4* pu,
                                 const float4* vu, const float4* eu, float4* ps, float4* vs, float4* es,
-                                hipStream_t st, const float4* cu, float4* cs) {
+                                hipStream_t st, const float4* cu, float4* cs, int* left) {
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     if (num <= 0) return hipSuccess;
     k_cells_permute<<<blocks_for(num), kBlock, 0, st>>>(num, d_num, keys, (uint32_t)nb_cells, start, end, sub_bits,
                                                         sub_bits == kSubBits ? sub : nullptr, idx, pu, vu, eu, ps,
-                                                        vs, es, cu, cs);
+                                                        vs, es, cu, cs, left);
     return hipGetLastError();
 }
 

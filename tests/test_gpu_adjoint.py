@@ -118,3 +118,31 @@ def test_adjoint_forward_equals_plain_system(cuda):
     np.testing.assert_allclose(vT.cpu().numpy(), p.read("vel"), rtol=1e-5, atol=1e-6)
     p.close()
     sim.close()
+
+
+def test_backward_with_too_little_memory_for_a_segment(cuda):
+    """Where the device has no room for the records of a whole segment the
+    handle keeps fewer and replays the segment once per part of it: the same
+    kernels on the same states, so the same bits."""
+    import torch
+    from enjaparticles_amd.adjoint import AdjointSPH
+    n, steps = 131072, 64                          # records of 177 bytes per particle and step: 1.48 GB
+    sc = scenes.dam_custom(64, 64, 32, seed=31)
+    assert sc.n == n
+    pos, vel = (torch.from_numpy(x).to(cuda) for x in (sc.pos, sc.vel))
+    g = torch.from_numpy(np.random.default_rng(32).normal(size=(n, 4)).astype(np.float32)).to(cuda)
+    out = []
+    for short in (False, True):
+        torch.cuda.empty_cache()
+        spare = torch.empty(torch.cuda.mem_get_info()[0] - (1250 << 20) if short else 0, dtype=torch.uint8,
+                            device=cuda)
+        sim = AdjointSPH(sc.settings, n, checkpoint_every=steps, max_steps=steps)
+        taken = torch.cuda.mem_get_info()[0]
+        xT, _ = sim.forward(pos, vel, steps, 0.01, 3.0)
+        out.append([t if isinstance(t, float) else t.cpu().numpy() for t in (xT, *sim.backward(g))])
+        if short:
+            assert taken < 1 << 30                 # the device was nearly full, the handle fitted all the same
+        sim.close()
+        del spare
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
