@@ -144,5 +144,6 @@ def test_backward_with_too_little_memory_for_a_segment(cuda):
             assert taken < 1 << 30                 # the device was nearly full, the handle fitted all the same
         sim.close()
         del spare
+        torch.cuda.empty_cache()                       # give the memory back to the device
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
