@@ -160,9 +160,11 @@ int rtps_gravity(int num, int nsrc, const rtps_float4* sources, const float* mas
     }
     rtps_sph_params sp{};
     sp.simulation_scale = scale;
-    rtps_grid_params gz{};
-    RTPS_HIP(launch_post_force(num, nullptr, nullptr, 0, (const float4*)pos_s, nullptr, (float4*)force, sp, g, 0, gz,
-                               S(stream)));
+    AfterForce a;
+    a.gravity = true;
+    RTPS_HIP(launch_after_force(num, nullptr, nullptr, 0, (const float4*)pos_s, nullptr, nullptr, (float4*)force,
+                                nullptr, nullptr, sp, a, g, Grid{}, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                S(stream)));
     return RTPS_OK;
 }
 
@@ -171,9 +173,13 @@ int rtps_collision_wall(int num, const rtps_float4* pos_s, const rtps_float4* ve
     RTPS_CHECK(num >= 0 && sphp && gps, "rtps_collision_wall: bad arguments");
     if (num == 0) return RTPS_OK;
     RTPS_CHECK(pos_s && vel_s && force, "rtps_collision_wall: null buffer");
-    GravitySources none{};
-    RTPS_HIP(launch_post_force(num, nullptr, nullptr, 0, (const float4*)pos_s, (const float4*)vel_s, (float4*)force,
-                               *sphp, none, 1, *gps, S(stream)));
+    AfterForce a;
+    a.walls = true;
+    a.bmin = gps->bnd_min;
+    a.bmax = gps->bnd_max;
+    RTPS_HIP(launch_after_force(num, nullptr, nullptr, 0, (const float4*)pos_s, (const float4*)vel_s, nullptr,
+                                (float4*)force, nullptr, nullptr, *sphp, a, GravitySources{}, Grid{}, nullptr,
+                                nullptr, nullptr, nullptr, nullptr, S(stream)));
     return RTPS_OK;
 }
 
@@ -184,19 +190,12 @@ int rtps_collision_triangles(int num, const rtps_float4* pos_s, const rtps_float
     RTPS_CHECK(pos_s && vel_s && force, "rtps_collision_triangles: null buffer");
     std::vector<TriPrep> prep = prepare_triangles(tris, n, sphp->simulation_scale);
     set_triangle_reach(prep, sphp->boundary_distance);
-    const std::vector<float4> reach = triangle_reach(prep);
-    TriPrep* dev = nullptr;
-    RTPS_HIP(hipMalloc(&dev, prep.size() * (sizeof(TriPrep) + sizeof(float4))));
-    float4* dev_reach = reinterpret_cast<float4*>(dev + prep.size());
-    hipError_t e = hipMemcpyAsync(dev, prep.data(), prep.size() * sizeof(TriPrep), hipMemcpyHostToDevice, S(stream));
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(dev_reach, reach.data(), reach.size() * sizeof(float4), hipMemcpyHostToDevice, S(stream));
-    if (e == hipSuccess)
-        e = launch_collision_tri(num, nullptr, nullptr, 0, (const float4*)pos_s, (const float4*)vel_s, (float4*)force,
-                                 dev, dev_reach, n, *sphp, S(stream));
-    if (e == hipSuccess) e = hipStreamSynchronize(S(stream));   // the triangle buffer is freed below
-    (void)hipFree(dev);
-    RTPS_HIP(e);
+    TriDevice dev;
+    RTPS_HIP(dev.load(prep, sphp->boundary_distance, S(stream)));
+    RTPS_HIP(launch_after_force(num, nullptr, nullptr, 0, (const float4*)pos_s, (const float4*)vel_s, nullptr,
+                                (float4*)force, nullptr, nullptr, *sphp, AfterForce{}, GravitySources{}, Grid{},
+                                &dev.set, nullptr, nullptr, nullptr, nullptr, S(stream)));
+    RTPS_HIP(hipStreamSynchronize(S(stream)));   // the triangle memory goes with dev
     return RTPS_OK;
 }
 
@@ -206,9 +205,13 @@ int rtps_leapfrog(int num, const rtps_float4* pos_s, const rtps_float4* vel_s, c
     RTPS_CHECK(num >= 0 && sphp, "rtps_leapfrog: bad arguments");
     if (num == 0) return RTPS_OK;
     RTPS_CHECK(pos_s && vel_s && force && xsph && idx && pos_u && vel_u && veleval_u, "rtps_leapfrog: null buffer");
-    RTPS_HIP(launch_leapfrog(num, nullptr, nullptr, 0, (const float4*)pos_s, (const float4*)vel_s,
-                             (const float4*)force, (const float4*)xsph, idx, *sphp, dt, (float4*)pos_u,
-                             (float4*)vel_u, (float4*)veleval_u, S(stream)));
+    AfterForce a;
+    a.store = false;
+    a.integrate = AfterForce::kLeapfrog;
+    a.dt = dt;
+    RTPS_HIP(launch_after_force(num, nullptr, nullptr, 0, (const float4*)pos_s, (const float4*)vel_s, nullptr,
+                                (float4*)force, (const float4*)xsph, idx, *sphp, a, GravitySources{}, Grid{}, nullptr,
+                                nullptr, (float4*)pos_u, (float4*)vel_u, (float4*)veleval_u, S(stream)));
     return RTPS_OK;
 }
 

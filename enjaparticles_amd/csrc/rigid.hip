@@ -5,8 +5,8 @@
 // A set of rigid-body particles (positions, and for a moving body velocities
 // and masses) is hashed into the fluid's cell grid, sorted and given cell
 // start/end tables with the same kernels as the fluid (System::hash_and_sort,
-// System.cpp:145-170, on the rigid system).  k_rigid_force then adds, for each
-// sorted fluid particle i and every set particle j in the 27 cells around i's
+// System.cpp:145-170, on the rigid system).  rigid_force (obstacles_device.h)
+// then adds, for each sorted fluid particle i and every set particle j in the 27 cells around i's
 // cell with |r| <= 2h (cl_sph_neighbors.h:99-140 iteration, 2h cut-off):
 //   norm = (x_j - x_i) / max(|r|, eps), stiff = s0 m
 //   F += -stiff (2h - |r|) norm + s1 sqrt(stiff mn) ((vrel . norm) norm)
@@ -43,80 +43,20 @@ __global__ __launch_bounds__(kRBlock) void k_rigid_gather(int n, const uint32_t*
     if (ms) ms[i] = mu[s];
 }
 
-template <bool MOVING>
-__global__ __launch_bounds__(kRBlock) void k_rigid_force(int num_host, const int* __restrict__ d_num,
-                                                         const uint32_t* __restrict__ fstart, int nb_cells,
-                                                         const float4* __restrict__ pos_s,
-                                                         const float4* __restrict__ ve_s, float4* __restrict__ force,
-                                                         const float4* __restrict__ bpos,
-                                                         const float4* __restrict__ bvel,
-                                                         const float* __restrict__ bmass,
-                                                         const uint32_t* __restrict__ bstart,
-                                                         const uint32_t* __restrict__ bend, rtps_sph_params sp,
-                                                         Grid gs, float s0, float s1) {
+// Marks every cell one of whose 27 cells (linear hashes, as the force's own
+// loop forms them) holds one of the n sorted particles.
+__global__ __launch_bounds__(kRBlock) void k_rigid_near(int n, const uint32_t* __restrict__ keys, int nb_cells, int rx,
+                                                        int ry, uint8_t* __restrict__ near) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int num = d_num ? *d_num : num_host;
-    if (d_num) effective_num(num, fstart, nb_cells, num);
-    if (i >= num) return;
-    const float scale = sp.simulation_scale, h = sp.smoothing_distance, eps = sp.EPSILON, m = sp.mass;
-    const float h2x = 2.0f * h;
-    const float4 p = pos_s[i];
-    const float px = p.x * scale, py = p.y * scale, pz = p.z * scale;
-    const float4 e = ve_s[i];   // veleval.xyz | density
-    const float stiff = s0 * m;
-    float fx = 0.f, fy = 0.f, fz = 0.f, vx = 0.f, vy = 0.f, vz = 0.f;
-    const int3 c = grid_cell(px, py, pz, gs);
-    for (int z = c.z - 1; z <= c.z + 1; ++z)
-        for (int y = c.y - 1; y <= c.y + 1; ++y)
-            for (int x = c.x - 1; x <= c.x + 1; ++x) {
-                const uint32_t ch = (uint32_t)grid_hash(x, y, z, gs);
-                if (ch >= (uint32_t)nb_cells) continue;
-                const uint32_t a = bstart[ch];
-                if (a == kEmpty) continue;
-                const uint32_t b = bend[ch];
-                for (uint32_t j = a; j < b; ++j) {
-                    const float4 q = bpos[j];
-                    const float rx = q.x * scale - px, ry = q.y * scale - py, rz = q.z * scale - pz;
-                    float rl = __builtin_sqrtf(rx * rx + ry * ry + rz * rz);
-                    if (!(rl <= h2x)) continue;
-                    rl = fmaxf(rl, eps);
-                    const float inv = 1.0f / rl;
-                    const float nx = rx * inv, ny = ry * inv, nz = rz * inv;
-                    float ux = -e.x, uy = -e.y, uz = -e.z, mn;
-                    if (MOVING) {
-                        const float4 v = bvel[j];
-                        ux += v.x;
-                        uy += v.y;
-                        uz += v.z;
-                        const float mj = bmass[j];
-                        mn = (m * mj) / (m + mj);
-                    } else {
-                        mn = (m * m) / (m + m);
-                    }
-                    const float un = ux * nx + uy * ny + uz * nz;
-                    const float spr = -stiff * (h2x - rl);
-                    const float dmp = s1 * __builtin_sqrtf(stiff * mn);
-                    fx += spr * nx + dmp * (un * nx);
-                    fy += spr * ny + dmp * (un * ny);
-                    fz += spr * nz + dmp * (un * nz);
-                    const float lap = h - rl;
-                    if (MOVING) {
-                        ux -= un * nx;
-                        uy -= un * ny;
-                        uz -= un * nz;
-                    }
-                    vx += ux * lap;
-                    vy += uy * lap;
-                    vz += uz * lap;
-                }
+    if (i >= n || (i > 0 && keys[i - 1] == keys[i])) return;
+    const int h = (int)keys[i];
+    if (h >= nb_cells) return;
+    for (int dz = -1; dz <= 1; ++dz)
+        for (int dy = -1; dy <= 1; ++dy)
+            for (int dx = -1; dx <= 1; ++dx) {
+                const long t = (long)h - (((long)dz * ry + dy) * rx + dx);
+                if (t >= 0 && t < nb_cells) near[t] = 1;
             }
-    const float cv = m * (1.0f / (e.w * e.w)) * (sp.viscosity * sp.wvisc_dd_coef);
-    const float sg = MOVING ? cv : -cv;
-    float4 f = force[i];
-    f.x += fx / m + sg * vx;
-    f.y += fy / m + sg * vy;
-    f.z += fz / m + sg * vz;
-    force[i] = f;
 }
 
 hipError_t rigid_prepare(int n, const float4* pos_u, const float4* vel_u, const float* mass_u, RigidDev& r,
@@ -134,21 +74,11 @@ hipError_t rigid_prepare(int n, const float4* pos_u, const float4* vel_u, const 
     if (n > 0)
         k_rigid_gather<<<rblocks(n), kRBlock, 0, st>>>(n, is, pos_u, vel_u, mass_u, r.pos, vel_u ? r.vel : nullptr,
                                                        mass_u ? r.mass : nullptr);
-    return hipGetLastError();
-}
-
-hipError_t launch_rigid_force(int num, const int* d_num, const uint32_t* fstart, int nb_cells, const float4* pos_s,
-                              const float4* ve_s, float4* force, const RigidDev& r, const rtps_sph_params& sp,
-                              const Grid& gs, hipStream_t st) {
-    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    if (num <= 0 || r.n <= 0) return hipSuccess;
-    if (r.moving)
-        k_rigid_force<true><<<rblocks(num), kRBlock, 0, st>>>(num, d_num, fstart, nb_cells, pos_s, ve_s, force, r.pos,
-                                                              r.vel, r.mass, r.start, r.end, sp, gs, r.s0, r.s1);
-    else
-        k_rigid_force<false><<<rblocks(num), kRBlock, 0, st>>>(num, d_num, fstart, nb_cells, pos_s, ve_s, force,
-                                                               r.pos, nullptr, nullptr, r.start, r.end, sp, gs, r.s0,
-                                                               r.s1);
+    if (r.near) {
+        e = launch_fill_u32((uint32_t*)r.near, 0u, ((long)g.nb_cells + 3) / 4, st);
+        if (e != hipSuccess) return e;
+        if (n > 0) k_rigid_near<<<rblocks(n), kRBlock, 0, st>>>(n, ks, g.nb_cells, g.irx, g.iry, r.near);
+    }
     return hipGetLastError();
 }
 

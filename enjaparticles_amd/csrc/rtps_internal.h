@@ -72,23 +72,9 @@ hipError_t launch_force_fused(int num, int* d_num, const float4* pos_s, const fl
                               const GravitySources& gsrc, int collision, const rtps_grid_params& gps, float dt,
                               float4* pos_u, float4* vel_u, float4* veleval_u, hipStream_t st,
                               const float4* color_s = nullptr, float4* color_u = nullptr);
-hipError_t launch_post_force(int num, const int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
-                             const float4* vel_s, float4* force, const rtps_sph_params& sp,
-                             const GravitySources& gsrc, int collision, const rtps_grid_params& gps, hipStream_t st);
-hipError_t launch_leapfrog(int num, const int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
-                           const float4* vel_s, const float4* force, const float4* xsph, const uint32_t* idx,
-                           const rtps_sph_params& sp, float dt, float4* pos_u, float4* vel_u, float4* veleval_u,
-                           hipStream_t st, const float4* color_s = nullptr, float4* color_u = nullptr);
-// euler.cl (integrator "euler"); ve_s: the sorted veleval|density records,
-// copied to veleval_u on a deletion step
-hipError_t launch_euler(int num, const int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
-                        const float4* vel_s, const float4* force, const float4* ve_s, const uint32_t* idx,
-                        const rtps_sph_params& sp, float dt, float4* pos_u, float4* vel_u, float4* veleval_u,
-                        hipStream_t st, const float4* color_s = nullptr, float4* color_u = nullptr);
 hipError_t launch_count_pairs(int num, const int* d_num, const float4* pos_s, const uint32_t* start,
                               const uint32_t* end, const rtps_sph_params& sp, const Grid& g, const Win& win,
                               unsigned long long* out, hipStream_t st);
-hipError_t launch_commit_num(int* d_num, const uint32_t* start, int nb_cells, hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, long n, hipStream_t st);
 
 // Default particle colour of System::pushParticles (System.h:160).
@@ -105,11 +91,32 @@ struct TriPrep {
 };
 std::vector<TriPrep> prepare_triangles(const rtps_triangle* tris, int n, float scale);
 void set_triangle_reach(std::vector<TriPrep>& t, float dist);
-// (centre, reach squared) per triangle, for the block cull
-std::vector<float4> triangle_reach(const std::vector<TriPrep>& t);
-hipError_t launch_collision_tri(int num, const int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
-                                const float4* vel_s, float4* force, const TriPrep* tris, const float4* reach, int ntri,
-                                const rtps_sph_params& sp, hipStream_t st);
+// The triangles on the device, and a grid over them: a particle in cell c can
+// touch the triangles list[q], q in start[c]..start[c + 1] - 1, whose bounding
+// spheres (centre, reach squared) are sphere[q].
+struct TriSet {
+    int n = 0;   // 0 = none
+    const TriPrep* tris = nullptr;
+    const float4* sphere = nullptr;
+    const uint32_t *start = nullptr, *list = nullptr;
+    float3 min{};
+    float inv = 0.f;   // cells per unit of length
+    int nx = 0, ny = 0, nz = 0;
+};
+// Owner of a TriSet's device memory.
+struct TriDevice {
+    TriSet set;
+    char* mem = nullptr;
+    size_t cap = 0;
+    TriDevice() = default;
+    TriDevice(const TriDevice&) = delete;
+    TriDevice& operator=(const TriDevice&) = delete;
+    ~TriDevice() {
+        if (mem) (void)hipFree(mem);
+    }
+    // Replaces the set (waits for the work on st).
+    hipError_t load(const std::vector<TriPrep>& prep, float dist, hipStream_t st);
+};
 
 // ---- colour field and iso-surface (surface.hip) ----
 size_t surface_scan_tiles(long ncubes);
@@ -139,15 +146,31 @@ struct RigidDev {
     float *mass = nullptr, *in_mass = nullptr;
     uint32_t *keys = nullptr, *idx = nullptr, *start = nullptr, *end = nullptr;
     void* sort_tmp = nullptr;
+    uint8_t* near = nullptr;   // per cell: 1 where one of its 27 cells holds a particle (nullptr: not kept)
 };
 // Hashes, sorts and tables n particles of pos_u (vel_u / mass_u may be null)
 // into r on the unscaled grid g.
 hipError_t rigid_prepare(int n, const float4* pos_u, const float4* vel_u, const float* mass_u, RigidDev& r,
                          const Grid& g, hipStream_t st);
-// Adds the forces of set r to the sorted fluid forces (gs: the scaled grid).
-hipError_t launch_rigid_force(int num, const int* d_num, const uint32_t* fstart, int nb_cells, const float4* pos_s,
-                              const float4* ve_s, float4* force, const RigidDev& r, const rtps_sph_params& sp,
-                              const Grid& gs, hipStream_t st);
+
+// ---- after the pair sums (after_force.hip) ----
+struct AfterForce {
+    enum { kNone = 0, kLeapfrog = 1, kEuler = 2 };
+    bool gravity = false;          // point sources
+    bool walls = false;            // of the domain bmin..bmax (scaled)
+    bool store = true;             // the force with what was added
+    int integrate = kNone;         // with the count commit of a deletion step
+    float dt = 0.f;
+    rtps_float4 bmin{}, bmax{};
+};
+// tri, rigid[2] (moving body, static boundary): optional.  idx, xsph and the
+// unsorted arrays are used by the integration, ve_s by rigid bodies and euler.
+hipError_t launch_after_force(int num, int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
+                              const float4* vel_s, const float4* ve_s, float4* force, const float4* xsph,
+                              const uint32_t* idx, const rtps_sph_params& sp, const AfterForce& a,
+                              const GravitySources& gsrc, const Grid& gs, const TriSet* tri, const RigidDev* rigid,
+                              float4* pos_u, float4* vel_u, float4* veleval_u, hipStream_t st,
+                              const float4* color_s = nullptr, float4* color_u = nullptr);
 
 // ---- hoses (hose.cpp) ----
 std::vector<rtps_float4> hose_spray(rtps_hose* h);

@@ -1,7 +1,8 @@
 // Per-stage HIP kernels of the SPH step for gfx950 and their C-ABI launchers
-// (hash, cellindices, permute, density, force, gravity, collision, leapfrog),
-// plus the fused force+gravity+collision+leapfrog kernel used by the system
-// step.  The radix sort lives in radix_sort.hip.
+// (hash, cellindices, permute, density, force), plus the fused
+// force+gravity+collision+leapfrog kernel used by the system step.  The sorts
+// live in bucket_sort.hip and radix_sort.hip, what follows a force that is not
+// fused in after_force.hip.
 //
 // Layout in HBM: one float4 (16 B) per particle for position, velocity and
 // veleval; sorted copies are separate arrays; keys/idx are u32; start/end
@@ -710,81 +711,6 @@ __global__ __launch_bounds__(SPLIT ? kSplitBlock : kBlock, QUEUED ? kQueuedWaves
     }
 }
 
-// a9 + a10 on stored forces (the unfused update() path): point sources then
-// walls, in the reference's order (SPH.cpp:289-297).
-__global__ __launch_bounds__(kBlock) void k_post_force(int num_host, const int* __restrict__ d_num,
-                                                       const uint32_t* __restrict__ start, int nb_cells,
-                                                       const float4* __restrict__ pos_s,
-                                                       const float4* __restrict__ vel_s, float4* __restrict__ force,
-                                                       rtps_sph_params sp, GravitySources gsrc, int collision,
-                                                       rtps_float4 bmin, rtps_float4 bmax) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int num = d_num ? *d_num : num_host;
-    if (d_num) effective_num(num, start, nb_cells, num);
-    if (i >= num) return;
-    float4 f = force[i];
-    const float4 p = pos_s[i];
-    gravity_sources(f, p, gsrc, sp.simulation_scale);
-    if (collision) collision_wall(f, p, vel_s[i], sp, bmin, bmax);
-    force[i] = f;
-}
-
-// a11: leapfrog.cl:30-121.
-__global__ __launch_bounds__(kBlock) void k_leapfrog(int num_host, const int* __restrict__ d_num,
-                                                     const uint32_t* __restrict__ start, int nb_cells,
-                                                     const float4* __restrict__ pos_s,
-                                                     const float4* __restrict__ vel_s,
-                                                     const float4* __restrict__ force,
-                                                     const float4* __restrict__ xsph,
-                                                     const uint32_t* __restrict__ idx, rtps_sph_params sp, float dt,
-                                                     float4* __restrict__ pos_u, float4* __restrict__ vel_u,
-                                                     float4* __restrict__ veleval_u, const float4* __restrict__ color_s,
-                                                     float4* __restrict__ color_u) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int num = d_num ? *d_num : num_host;
-    bool deleted = false;
-    if (d_num) deleted = effective_num(num, start, nb_cells, num);
-    if (i >= num) return;
-    float4 po, vo, eo;
-    leapfrog(pos_s[i], vel_s[i], force[i], xsph[i], sp, dt, po, vo, eo);
-    const uint32_t o = deleted ? (uint32_t)i : idx[i];
-    pos_u[o] = po;
-    vel_u[o] = vo;
-    veleval_u[o] = eo;
-    if (deleted && color_u) color_u[i] = color_s[i];   // leapfrog.cl:107
-}
-
-// a11 alternative: euler.cl:33-78 (integrator "euler").  veleval is not
-// written (euler.cl leaves it alone); on a deletion step the survivors'
-// sorted records become the unsorted ones (call_prep, SPH.cpp:445-457), so
-// veleval and the colours are copied from the sorted arrays there.  The
-// sorted veleval array holds veleval.xyz | density; its copy gets w = 0 (no
-// kernel reads veleval.w).
-__global__ __launch_bounds__(kBlock) void k_euler(int num_host, const int* __restrict__ d_num,
-                                                  const uint32_t* __restrict__ start, int nb_cells,
-                                                  const float4* __restrict__ pos_s, const float4* __restrict__ vel_s,
-                                                  const float4* __restrict__ force, const float4* __restrict__ ve_s,
-                                                  const uint32_t* __restrict__ idx, rtps_sph_params sp, float dt,
-                                                  float4* __restrict__ pos_u, float4* __restrict__ vel_u,
-                                                  float4* __restrict__ veleval_u,
-                                                  const float4* __restrict__ color_s, float4* __restrict__ color_u) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int num = d_num ? *d_num : num_host;
-    bool deleted = false;
-    if (d_num) deleted = effective_num(num, start, nb_cells, num);
-    if (i >= num) return;
-    float4 po, vo;
-    euler(pos_s[i], vel_s[i], force[i], sp, dt, po, vo);
-    const uint32_t o = deleted ? (uint32_t)i : idx[i];
-    pos_u[o] = po;
-    vel_u[o] = vo;
-    if (deleted) {
-        const float4 e = ve_s[i];
-        veleval_u[i] = make_float4(e.x, e.y, e.z, 0.0f);
-        if (color_u) color_u[i] = color_s[i];
-    }
-}
-
 // Pair totals of the neighbour loop on the current sorted state: out[0] =
 // candidates of the reference's 27-cell loop (K), out[1] = accepted pairs
 // (M, self included), out[2] = candidates the windowed rows actually test.
@@ -836,15 +762,6 @@ hipError_t launch_count_pairs(int num, const int* d_num, const float4* pos_s, co
     if (num <= 0) return hipSuccess;
     k_count_pairs<<<blocks_for(num), kBlock, 0, st>>>(num, d_num, pos_s, start, end, sp, g, win, out);
     return hipGetLastError();
-}
-
-// Commits the deletion path's particle count for the next step.
-__global__ void k_commit_num(int* __restrict__ d_num, const uint32_t* __restrict__ start, int nb_cells) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        int num = *d_num;
-        int nc = (int)start[nb_cells];
-        if (nc >= 0 && nc <= num) *d_num = nc;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1074,45 +991,6 @@ hipError_t launch_force_fused(int num, int* d_num, const float4* pos_s, const fl
 #undef RTPS_FFUSED
 #undef RTPS_FFUSED_L
 #undef RTPS_FFUSED_Q
-    return hipGetLastError();
-}
-
-hipError_t launch_post_force(int num, const int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
-                             const float4* vel_s, float4* force, const rtps_sph_params& sp,
-                             const GravitySources& gsrc, int collision, const rtps_grid_params& gps, hipStream_t st) {
-    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    if (num <= 0) return hipSuccess;
-    if (gsrc.n == 0 && !collision) return hipSuccess;
-    k_post_force<<<blocks_for(num), kBlock, 0, st>>>(num, d_num, start, nb_cells, pos_s, vel_s, force, sp, gsrc,
-                                                      collision, gps.bnd_min, gps.bnd_max);
-    return hipGetLastError();
-}
-
-hipError_t launch_leapfrog(int num, const int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
-                           const float4* vel_s, const float4* force, const float4* xsph, const uint32_t* idx,
-                           const rtps_sph_params& sp, float dt, float4* pos_u, float4* vel_u, float4* veleval_u,
-                           hipStream_t st, const float4* color_s, float4* color_u) {
-    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    if (num <= 0) return hipSuccess;
-    k_leapfrog<<<blocks_for(num), kBlock, 0, st>>>(num, d_num, start, nb_cells, pos_s, vel_s, force, xsph, idx, sp, dt,
-                                                    pos_u, vel_u, veleval_u, color_s, color_u);
-    return hipGetLastError();
-}
-
-hipError_t launch_euler(int num, const int* d_num, const uint32_t* start, int nb_cells, const float4* pos_s,
-                        const float4* vel_s, const float4* force, const float4* ve_s, const uint32_t* idx,
-                        const rtps_sph_params& sp, float dt, float4* pos_u, float4* vel_u, float4* veleval_u,
-                        hipStream_t st, const float4* color_s, float4* color_u) {
-    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    if (num <= 0) return hipSuccess;
-    k_euler<<<blocks_for(num), kBlock, 0, st>>>(num, d_num, start, nb_cells, pos_s, vel_s, force, ve_s, idx, sp, dt,
-                                                 pos_u, vel_u, veleval_u, color_s, color_u);
-    return hipGetLastError();
-}
-
-hipError_t launch_commit_num(int* d_num, const uint32_t* start, int nb_cells, hipStream_t st) {
-    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    k_commit_num<<<1, 64, 0, st>>>(d_num, start, nb_cells);
     return hipGetLastError();
 }
 

@@ -94,10 +94,7 @@ struct rtps_sph {
     int mesh_ntri = 0;
     std::vector<rtps_hose*> hoses;   // SPH::hoses (SPH.h), sprayed at the start of every update
     std::vector<rtps_triangle> triangles;   // SPH::loadTriangles, world units
-    TriPrep* tri_dev = nullptr;   // tri_cap records, then tri_cap reach spheres (tri_reach)
-    float4* tri_reach = nullptr;
-    size_t tri_cap = 0;
-    int ntri = 0;
+    TriDevice tri;
     std::vector<rtps_float4> hose_color;
     // rigid-body particle sets of SPH::interact: [0] a moving body, [1] the static boundary
     RigidDev rigid[2];
@@ -112,13 +109,12 @@ struct rtps_sph {
                         color_s, keys, idx, start, end, d_num, sort_tmp, sub_start, tile_q, rows};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
-        void* sbufs[] = {cf_field, mc_cases, mc_counts, mc_offs, mc_tiles, mc_total, mc_words, mc_ntri, mesh_v, mesh_n,
-                         tri_dev};
+        void* sbufs[] = {cf_field, mc_cases, mc_counts, mc_offs, mc_tiles, mc_total, mc_words, mc_ntri, mesh_v, mesh_n};
         for (void* b : sbufs)
             if (b) (void)hipFree(b);
         for (RigidDev& r : rigid) {
             void* rb[] = {r.pos, r.vel, r.in_pos, r.in_vel, r.mass, r.in_mass, r.keys, r.idx, r.start, r.end,
-                          r.sort_tmp};
+                          r.sort_tmp, r.near};
             for (void* b : rb)
                 if (b) (void)hipFree(b);
         }
@@ -173,31 +169,10 @@ void load_gravity_sources(rtps_sph* s) { gravity_sources_of(s->settings, s->gsrc
 
 // Triangles in the current simulation scale and boundary distance, on the device.
 hipError_t upload_triangles(rtps_sph* s) {
-    s->ntri = 0;
-    if (s->triangles.empty()) return hipSuccess;
     std::vector<TriPrep> prep = prepare_triangles(s->triangles.data(), (int)s->triangles.size(),
                                                   s->sp.simulation_scale);
     set_triangle_reach(prep, s->sp.boundary_distance);
-    const std::vector<float4> reach = triangle_reach(prep);
-    if (prep.size() > s->tri_cap) {
-        hipError_t e = hipStreamSynchronize(s->stream);
-        if (e == hipSuccess && s->tri_dev) e = hipFree(s->tri_dev);
-        s->tri_dev = nullptr;
-        s->tri_reach = nullptr;
-        s->tri_cap = 0;
-        if (e == hipSuccess) e = hipMalloc(&s->tri_dev, prep.size() * (sizeof(TriPrep) + sizeof(float4)));
-        if (e != hipSuccess) return e;
-        s->tri_cap = prep.size();
-        s->tri_reach = reinterpret_cast<float4*>(s->tri_dev + s->tri_cap);
-    }
-    hipError_t e = hipMemcpyAsync(s->tri_dev, prep.data(), prep.size() * sizeof(TriPrep), hipMemcpyHostToDevice,
-                                  s->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(s->tri_reach, reach.data(), reach.size() * sizeof(float4), hipMemcpyHostToDevice,
-                           s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    if (e == hipSuccess) s->ntri = (int)prep.size();
-    return e;
+    return s->tri.load(prep, s->sp.boundary_distance, s->stream);
 }
 
 void apply_settings(rtps_sph* s) {
@@ -206,7 +181,7 @@ void apply_settings(rtps_sph* s) {
     s->sp.num = s->num_host;
     s->dt = s->settings.GetSettingAs<float>("time_step");
     load_gravity_sources(s);
-    if (!s->triangles.empty()) (void)upload_triangles(s);   // a failure leaves ntri = 0: reported by the next load
+    if (!s->triangles.empty()) (void)upload_triangles(s);   // a failure leaves none: reported by the next load
     s->settings.updated();
     s->graph_valid = false;
     s->timed_graph_valid = false;
@@ -267,58 +242,43 @@ int launch_front(rtps_sph* s, StageTimer& t) {
 
 bool rigid_on(const rtps_sph* s) { return s->rigid[0].n > 0 || s->rigid[1].n > 0; }
 
-// SPH::interact (SPH.cpp:610-663): the moving body's particles, then the
-// static boundary's, add their forces to the sorted forces of update().
-int launch_interact(rtps_sph* s) {
-    for (const RigidDev& r : s->rigid)
-        RTPS_TRY_HIP(launch_rigid_force(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->ve_s, s->force_s, r,
-                                        s->sp, s->gs, s->stream));
-    return RTPS_OK;
-}
-
-// SPH::integrate (SPH.cpp:389-441) on the stored forces: euler.cl or leapfrog.cl.
-int launch_integrate(rtps_sph* s) {
-    if (s->integrator == 1)
-        RTPS_TRY_HIP(launch_euler(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->vel_s, s->force_s,
-                                  s->ve_s, s->idx_sorted, s->sp, s->dt, s->pos_u, s->vel_u, s->veleval_u, s->stream,
-                                  col_s(s), col_u(s)));
-    else
-        RTPS_TRY_HIP(launch_leapfrog(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->vel_s, s->force_s,
-                                     s->xsph_s, s->idx_sorted, s->sp, s->dt, s->pos_u, s->vel_u, s->veleval_u,
-                                     s->stream, col_s(s), col_u(s)));
+// The parts of a step after the stored pair sums: gravity sources and walls,
+// triangles (SPH::collision, SPH.cpp:303-336), rigid-body particles
+// (SPH::interact, SPH.cpp:610-663: the moving body's, then the static
+// boundary's) and the integration (SPH::integrate, SPH.cpp:389-441).
+int launch_after(rtps_sph* s, bool forces, bool interact, bool integrate) {
+    AfterForce a;
+    a.gravity = forces && s->gsrc.n > 0;
+    a.walls = forces && s->opt_collision;
+    a.integrate = !integrate ? AfterForce::kNone : s->integrator == 1 ? AfterForce::kEuler : AfterForce::kLeapfrog;
+    a.store = forces || interact;
+    a.dt = s->dt;
+    a.bmin = s->gps.bnd_min;
+    a.bmax = s->gps.bnd_max;
+    RTPS_TRY_HIP(launch_after_force(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->vel_s, s->ve_s,
+                                    s->force_s, s->xsph_s, s->idx_sorted, s->sp, a, s->gsrc, s->gs,
+                                    forces && s->opt_collision ? &s->tri.set : nullptr,
+                                    interact ? s->rigid : nullptr, s->pos_u, s->vel_u, s->veleval_u, s->stream,
+                                    col_s(s), col_u(s)));
     return RTPS_OK;
 }
 
 // Force through integration + count commit, as the application loop runs a
 // step (update, interact, integrate; TestApplication.cpp:815-835).  One
 // fused kernel, or, with the euler integrator, triangles in the collisions or
-// rigid-body sets loaded: force; gravity sources and walls; triangles
-// (SPH::collision, SPH.cpp:303-336); rigid-body forces; the integration, as
-// separate kernels.
+// rigid-body sets loaded, the force kernel and launch_after's.
 int launch_back(rtps_sph* s) {
     const bool fo = s->opt_force_out != 0;
-    const bool tri = s->ntri > 0 && s->opt_collision;
-    if (s->integrator == 1 || tri || rigid_on(s)) {
+    if (s->integrator == 1 || (s->tri.set.n > 0 && s->opt_collision) || rigid_on(s)) {
         RTPS_TRY_HIP(launch_force(s->num_host, s->d_num, s->pos_s, nullptr, s->ve_s, true, s->start, s->end, s->sp,
                                   s->gs, win(s, true), s->force_s, s->xsph_s, s->stream));
-        RTPS_TRY_HIP(launch_post_force(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->vel_s, s->force_s,
-                                       s->sp, s->gsrc, s->opt_collision, s->gps, s->stream));
-        if (tri)
-            RTPS_TRY_HIP(launch_collision_tri(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->vel_s,
-                                              s->force_s, s->tri_dev, s->tri_reach, s->ntri, s->sp, s->stream));
-        int rc = launch_interact(s);
-        if (rc) return rc;
-        rc = launch_integrate(s);
-        if (rc) return rc;
-    } else {
-        RTPS_TRY_HIP(launch_force_fused(s->num_host, s->d_num, s->pos_s, s->ve_s, s->start, s->end, s->sp, s->gs,
-                                        win(s, true), fo ? s->force_s : nullptr, fo ? s->xsph_s : nullptr, s->vel_s,
-                                        s->idx_sorted, s->gsrc, s->opt_collision, s->gps, s->dt, s->pos_u, s->vel_u,
-                                        s->veleval_u, s->stream, col_s(s), col_u(s)));
-        return RTPS_OK;   // the fused kernel commits the count of a deletion step itself
+        return launch_after(s, true, true, true);
     }
-    RTPS_TRY_HIP(launch_commit_num(s->d_num, s->start, s->nb_cells, s->stream));
-    return RTPS_OK;
+    RTPS_TRY_HIP(launch_force_fused(s->num_host, s->d_num, s->pos_s, s->ve_s, s->start, s->end, s->sp, s->gs,
+                                    win(s, true), fo ? s->force_s : nullptr, fo ? s->xsph_s : nullptr, s->vel_s,
+                                    s->idx_sorted, s->gsrc, s->opt_collision, s->gps, s->dt, s->pos_u, s->vel_u,
+                                    s->veleval_u, s->stream, col_s(s), col_u(s)));
+    return RTPS_OK;   // either way the last kernel commits the count of a deletion step
 }
 
 // One step: front + launch_back.
@@ -877,11 +837,8 @@ int rtps_sph_update(rtps_sph* s) {
     if (rc) return rc;
     RTPS_TRY_HIP(launch_force(s->num_host, s->d_num, s->pos_s, nullptr, s->ve_s, true, s->start, s->end, s->sp, s->gs,
                               win(s, true), s->force_s, s->xsph_s, s->stream));
-    RTPS_TRY_HIP(launch_post_force(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->vel_s, s->force_s,
-                                   s->sp, s->gsrc, s->opt_collision, s->gps, s->stream));
-    if (s->ntri > 0 && s->opt_collision)
-        RTPS_TRY_HIP(launch_collision_tri(s->num_host, s->d_num, s->start, s->nb_cells, s->pos_s, s->vel_s,
-                                          s->force_s, s->tri_dev, s->tri_reach, s->ntri, s->sp, s->stream));
+    rc = launch_after(s, true, false, false);
+    if (rc) return rc;
     s->update_pending = true;
     return RTPS_OK;
 }
@@ -889,9 +846,8 @@ int rtps_sph_update(rtps_sph* s) {
 int rtps_sph_integrate(rtps_sph* s) {
     if (!s) return set_error(RTPS_ERR_ARG, "rtps_sph_integrate: null handle");
     if (!s->update_pending) return set_error(RTPS_ERR_STATE, "integrate() needs a preceding update()");
-    int rc = launch_integrate(s);   // SPH::integrate (SPH.cpp:392-409)
+    int rc = launch_after(s, false, false, true);   // SPH::integrate (SPH.cpp:392-409)
     if (rc) return rc;
-    RTPS_TRY_HIP(launch_commit_num(s->d_num, s->start, s->nb_cells, s->stream));
     s->update_pending = false;
     return RTPS_OK;
 }
@@ -899,7 +855,7 @@ int rtps_sph_integrate(rtps_sph* s) {
 int rtps_sph_interact(rtps_sph* s) {
     if (!s) return set_error(RTPS_ERR_ARG, "rtps_sph_interact: null handle");
     if (!s->update_pending) return set_error(RTPS_ERR_STATE, "interact() needs a preceding update()");
-    return launch_interact(s);
+    return launch_after(s, false, true, false);
 }
 
 namespace {
@@ -919,13 +875,18 @@ int load_rigid(rtps_sph* s, int k, const rtps_float4* pos, const rtps_float4* ve
         RTPS_TRY_HIP(dalloc(&r.start, (size_t)s->nb_cells + 1));
         RTPS_TRY_HIP(dalloc(&r.end, (size_t)s->nb_cells + 1));
         RTPS_TRY_HIP(launch_fill_u32(r.end, 666u, (long)s->nb_cells + 1, s->stream));   // as SPH.cpp:512-517
+        // linear cell hashes are exact floats up to here: a cell's 27 neighbours are fixed offsets
+        if (s->nb_cells < (1 << 23)) RTPS_TRY_HIP(dalloc(&r.near, (size_t)s->nb_cells));
     }
     if (n > r.cap) {
         void* old[] = {r.pos, r.vel, r.in_pos, r.in_vel, r.mass, r.in_mass, r.keys, r.idx, r.sort_tmp};
         for (void* b : old)
             if (b) RTPS_TRY_HIP(hipFree(b));
-        r = RigidDev{0, 0, false, 0.f, 0.f, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                     nullptr, nullptr, r.start, r.end, nullptr};
+RigidDev kept;   // the cell tables stay
+        kept.start = r.start;
+        kept.end = r.end;
+        kept.near = r.near;
+        r = kept;
         const size_t N = (size_t)n;
         RTPS_TRY_HIP(dalloc(&r.pos, N));
         RTPS_TRY_HIP(dalloc(&r.vel, N));
