@@ -2,7 +2,7 @@
 // adjoint (no reference counterpart).
 //
 // forward(pos0, vel0, T steps, mu, K) runs the plain system's step kernels
-// (bucket sort, cells + permute, density, force + walls + leapfrog) from the
+// (sort, cells + permute, density, force + walls + leapfrog) from the
 // given state (veleval starts at zero, SPH.cpp:491-492) and keeps the state
 // every `checkpoint_every` steps.  backward(dL/dx_T, dL/dv_T) walks the
 // segments from the last: it replays a segment from its checkpoint, keeping
@@ -117,18 +117,28 @@ hipError_t alloc_records(rtps_adj* a, int want) {
 // force: also the SPH force, which only the adjoint reads.
 int forward_step(rtps_adj* a, const State& in, const State& out, Record& r, bool force, hipStream_t st) {
     const int n = a->N;
-    uint32_t *ks = a->keys, *is = r.idx;
-    if (bucket_sort_fits(n, a->key_bits))
-        RTPS_TRY_HIP(hash_bucket_sort(n, a->key_bits, in.pos, n, nullptr, a->pad_key, a->g, kSubBits, a->start,
-                                      a->nb_cells + 1, a->keys, r.idx, a->sort_tmp, st));
-    else
-        RTPS_TRY_HIP(hash_sort_pairs(n, a->key_bits, in.pos, n, nullptr, a->pad_key, a->g, kSubBits, a->start,
-                                     a->nb_cells + 1, a->keys, r.idx, a->sort_tmp, st, &ks, &is));
-    if (is != r.idx) RTPS_TRY_HIP(hipMemcpyAsync(r.idx, is, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
-    RTPS_TRY_HIP(launch_cells_permute(n, nullptr, ks, a->nb_cells, a->start, a->end, kSubBits, a->sub, r.idx, in.pos,
-                                      in.vel, in.ve, r.pos_s, r.vel_s, r.ve_s, st, nullptr, nullptr, a->left_grid));
+    const uint32_t* keys = a->keys;
+    if (cell_sort_fits(n, a->nb_cells)) {
+        RTPS_TRY_HIP(cell_sort_place(n, n, nullptr, in.pos, a->g, a->keys, r.idx, a->start, a->end, a->sort_tmp, st));
+        RTPS_TRY_HIP(cell_sort_finish(n, n, nullptr, a->pad_key, a->nb_cells, a->start, a->end, a->sub, a->keys, r.idx,
+                                      in.pos, in.vel, in.ve, r.pos_s, r.vel_s, r.ve_s, a->sort_tmp, st, nullptr,
+                                      nullptr, a->left_grid));
+    } else {
+        uint32_t *ks = a->keys, *is = r.idx;
+        if (bucket_sort_fits(n, a->key_bits))
+            RTPS_TRY_HIP(hash_bucket_sort(n, a->key_bits, in.pos, n, nullptr, a->pad_key, a->g, kSubBits, a->start,
+                                          a->nb_cells + 1, a->keys, r.idx, a->sort_tmp, st));
+        else
+            RTPS_TRY_HIP(hash_sort_pairs(n, a->key_bits, in.pos, n, nullptr, a->pad_key, a->g, kSubBits, a->start,
+                                         a->nb_cells + 1, a->keys, r.idx, a->sort_tmp, st, &ks, &is));
+        if (is != r.idx) RTPS_TRY_HIP(hipMemcpyAsync(r.idx, is, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
+        RTPS_TRY_HIP(launch_cells_permute(n, nullptr, ks, a->nb_cells, a->start, a->end, kSubBits, a->sub, r.idx,
+                                          in.pos, in.vel, in.ve, r.pos_s, r.vel_s, r.ve_s, st, nullptr, nullptr,
+                                          a->left_grid));
+        keys = ks;
+    }
     // force loop 5 on recorded rows, which the adjoint reads as well
-    Win w{ks, a->gps.grid_res.x, a->gps.grid_res.y, a->gps.grid_res.z, 0, 0, 5};
+    Win w{keys, a->gps.grid_res.x, a->gps.grid_res.y, a->gps.grid_res.z, 0, 0, 5};
     w.sub = a->sub;
     w.rows = r.rows;
     w.rows_stride = (uint32_t)n;
@@ -200,7 +210,9 @@ int rtps_adj_create(const char* const* keys, const char* const* vals, int n, int
         RTPS_TRY_HIP(a->alloc(&a->end, C));
         if ((size_t)a->nb_cells * kSubCells * sizeof(uint32_t) <= ((size_t)2 << 30))   // as the system's
             RTPS_TRY_HIP(a->alloc(&a->sub, (size_t)a->nb_cells * kSubCells));
-        RTPS_TRY_HIP(a->alloc((char**)&a->sort_tmp, bucket_temp_bytes((int)N, a->key_bits)));
+        const bool by_cell = cell_sort_fits((int)N, a->nb_cells);
+        RTPS_TRY_HIP(a->alloc((char**)&a->sort_tmp, by_cell ? cell_sort_temp_bytes((int)N, a->nb_cells)
+                                                            : bucket_temp_bytes((int)N, a->key_bits)));
         RTPS_TRY_HIP(a->alloc(&a->ga, N));
         RTPS_TRY_HIP(a->alloc(&a->gX, N));
         RTPS_TRY_HIP(a->alloc(&a->lxp, N));
@@ -212,7 +224,8 @@ int rtps_adj_create(const char* const* keys, const char* const* vals, int n, int
         RTPS_TRY_HIP(a->alloc(&a->left_grid, 1));
         RTPS_TRY_HIP(alloc_records(a.get(), std::min(checkpoint_every, max_steps)));
         RTPS_TRY_HIP(a->alloc(&a->partial, a->rec.size() * (size_t)adjoint_tiles((int)N)));
-        RTPS_TRY_HIP(sort_clear_temp(a->sort_tmp, (int)N, nullptr));
+        RTPS_TRY_HIP(by_cell ? cell_sort_clear_temp(a->sort_tmp, a->nb_cells, nullptr)
+                             : sort_clear_temp(a->sort_tmp, (int)N, nullptr));
         RTPS_TRY_HIP(launch_fill_u32(a->end, 0u, (long)C, nullptr));
         RTPS_TRY_HIP(hipDeviceSynchronize());
         *out = a.release();

@@ -1,0 +1,277 @@
+// Sort of the step's particles by cell key, with the cell tables and the
+// permute (System::hash_and_sort of the reference: hash.cl, the bitonic sort of
+// System.cpp:407-480, cellindices.cl, permute.cl), as one counting sort over
+// the grid's cells.  The order is the stable sort's: keys (cell << 4 | x
+// sixteenth) ascending, equal keys by particle index.
+//
+//   k_cell_count    the key of every particle (hash_key) and its arrival rank
+//                   in its cell: one atomic on the cell's counter.
+//   k_cell_scan     counters to cell starts and ends (the start/end tables of
+//                   cellindices.cl); the counters are zero again.
+//   k_cell_place    (key, index) pairs to cell start + rank: cells together,
+//                   any order inside a cell.
+//   k_cell_finish   each pair's place in its cell is the number of the cell's
+//                   pairs that precede it (x sixteenth, then index); the pair,
+//                   the particle's records and its entries of the sub-cell
+//                   table go there.
+//
+// Against digit passes this reads and writes the keys once, needs no look-back
+// between tiles, and writes the cell tables on the way.  A cell holds 8
+// particles at rest and 20 to 40 in a settled pool, so the counting inside a
+// cell is short; a cell of m particles costs m^2 comparisons, 9,000 stacked in
+// one cell 0.3 ms.
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "rtps_internal.h"
+#include "sort_layout.h"
+#include "sph_device.h"
+
+namespace rtps {
+
+constexpr int kCsThreads = 256;
+constexpr int kScanThreads = 1024, kScanWaves = kScanThreads / 64;
+constexpr int kScanTile = 4 * kScanThreads;   // counters per round of a scanning block
+constexpr int kScanBlocks = 256;              // at most: a block adds up every earlier block's total
+
+static inline int cs_blocks(long n) { return (int)((n + kCsThreads - 1) / kCsThreads); }
+
+// Layout of the temp: the counters (zero between sorts), the scan's status
+// words, the pairs.
+struct CellTemp {
+    uint32_t* count;
+    unsigned long long* status;
+    uint2* pairs;
+};
+static size_t cell_layout(int n, int nb_cells, CellTemp* t, char* p) {
+    size_t off = 0;
+    if (t) t->count = (uint32_t*)(p + off);
+    off += (((size_t)nb_cells + 1) * 4 + 255) & ~(size_t)255;
+    if (t) t->status = (unsigned long long*)(p + off);
+    off += kScanBlocks * sizeof(unsigned long long);
+    if (t) t->pairs = (uint2*)(p + off);
+    return off + (size_t)std::max(n, 1) * sizeof(uint2);
+}
+
+size_t cell_sort_temp_bytes(int n, int nb_cells) { return cell_layout(n, nb_cells, nullptr, nullptr); }
+
+hipError_t cell_sort_clear_temp(void* temp, int nb_cells, hipStream_t st) {
+    return hipMemsetAsync(temp, 0, ((size_t)nb_cells + 1) * 4, st);
+}
+
+// The line: one atomic per particle costs more than the bucket sort's one per
+// bucket that a tile touches where consecutive particles are neighbours, and
+// less where they are not.  Measured for sort + cells (us, bucket / counting; at
+// rest, then in a settled pool whose order is mixed): 22 / 16 and 21 / 16 at
+// 2,048 particles, 31 / 24 and 37 / 29 at 99,991, 34 / 33 and 58 / 49 at
+// 262,144, 42 / 45 and 94 / 81 at 524,288, 58 / 77 and 175 / 147 at 1,048,576
+// (digit passes: 91 and 137).  At rest the two meet near 330,000.
+// Grids with many more cells than particles take a sort of the keys instead:
+// the scan reads every cell's counter.
+bool cell_sort_fits(int n, int nb_cells) { return n <= kCellSortMax && (long)nb_cells <= 16L * n + (1 << 20); }
+
+__global__ __launch_bounds__(kCsThreads) void k_cell_count(int num_host, const int* __restrict__ d_num,
+                                                           const float4* __restrict__ pos_u, Grid g,
+                                                           uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                                                           uint32_t* __restrict__ count,
+                                                           unsigned long long* __restrict__ status) {
+    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    if (i < kScanBlocks) status[i] = 0ull;
+    const int num = d_num ? *d_num : num_host;
+    if (i >= num) return;
+    const uint32_t key = hash_key(pos_u[i], g, kSubBits);
+    keys[i] = key;
+    rank[i] = atomicAdd(&count[key >> kSubBits], 1u);
+}
+
+// Block b scans the cells [b * chunk, (b + 1) * chunk) of the n_cells = nb_cells
+// + 1 counters (the last one: particles outside the grid).  It publishes its
+// total first and then adds up those of every earlier block, which have come
+// in by the time its own counters are read (blocks start in order and publish
+// before they wait).
+__global__ __launch_bounds__(kScanThreads) void k_cell_scan(int n_cells, int chunk, uint32_t* __restrict__ count,
+                                                            uint32_t* __restrict__ start, uint32_t* __restrict__ end,
+                                                            unsigned long long* status) {
+    __shared__ uint32_t wsum[kScanWaves];
+    __shared__ uint32_t prior[kScanBlocks / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int c0 = blockIdx.x * chunk, c1 = min(c0 + chunk, n_cells);
+    auto load = [&](int base, uint32_t (&v)[4]) {   // four counters of the thread (c0 and chunk are multiples of 4)
+        if (base + 4 <= c1) {
+            const uint4 q = *(const uint4*)(count + base);
+            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = base + k < c1 ? count[base + k] : 0u;
+        }
+    };
+    // the block's sum of s over its threads (every thread)
+    auto block_sum = [&](uint32_t s) {
+        s = wave_incl_scan(s);
+        __syncthreads();
+        if (lane == 63) wsum[w] = s;
+        __syncthreads();
+        uint32_t t = 0;
+#pragma unroll
+        for (int q = 0; q < kScanWaves; ++q) t += wsum[q];
+        return t;
+    };
+    uint32_t v[4], sum = 0;
+    for (int t0 = c0; t0 < c1; t0 += kScanTile) {
+        load(t0 + 4 * tid, v);
+        sum += v[0] + v[1] + v[2] + v[3];
+    }
+    const uint32_t total = block_sum(sum);
+    if (tid == 0)
+        __hip_atomic_store(&status[blockIdx.x], (1ull << 63) | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t before = 0;
+    if (tid < (int)blockIdx.x) {
+        unsigned long long s;
+        do {
+            s = __hip_atomic_load(&status[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } while (!(s >> 63));
+        before = (uint32_t)s;
+    }
+    if (tid < kScanBlocks) {
+        before = wave_incl_scan(before);
+        if (lane == 63) prior[w] = before;
+    }
+    __syncthreads();
+    uint32_t run = 0;
+#pragma unroll
+    for (int q = 0; q < kScanBlocks / 64; ++q) run += prior[q];
+    for (int t0 = c0; t0 < c1; t0 += kScanTile) {
+        const int base = t0 + 4 * tid;
+        if (c1 - c0 > kScanTile) load(base, v);   // one round: still in registers
+        const uint32_t s = v[0] + v[1] + v[2] + v[3], inc = wave_incl_scan(s);
+        __syncthreads();   // the former round's sums are read
+        if (lane == 63) wsum[w] = inc;
+        __syncthreads();
+        uint32_t at = run + inc - s, all = 0;
+#pragma unroll
+        for (int q = 0; q < kScanWaves; ++q) {
+            if (q < w) at += wsum[q];
+            all += wsum[q];
+        }
+        run += all;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (base + k < c1) {
+                start[base + k] = v[k] ? at : kEmpty;
+                at += v[k];
+                if (v[k]) {   // end[] of empty cells is left as it is (cellindices.cl)
+                    end[base + k] = at;
+                    count[base + k] = 0u;
+                }
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(kCsThreads) void k_cell_place(int num_host, const int* __restrict__ d_num,
+                                                           const uint32_t* __restrict__ keys,
+                                                           const uint32_t* __restrict__ rank,
+                                                           const uint32_t* __restrict__ start,
+                                                           uint2* __restrict__ pairs) {
+    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    const int num = d_num ? *d_num : num_host;
+    if (i >= num) return;
+    const uint32_t key = keys[i];
+    const uint32_t at = start[key >> kSubBits] + rank[i];
+    if (at < (uint32_t)num) pairs[at] = make_uint2(key, (uint32_t)i);
+}
+
+__global__ __launch_bounds__(kCsThreads) void k_cell_finish(int n, int num_host, const int* __restrict__ d_num,
+                                                            uint32_t pad_key, const uint2* __restrict__ pairs,
+                                                            int nb_cells, const uint32_t* __restrict__ start,
+                                                            const uint32_t* __restrict__ end,
+                                                            uint32_t* __restrict__ sub, uint32_t* __restrict__ keys,
+                                                            uint32_t* __restrict__ idx, const float4* __restrict__ pu,
+                                                            const float4* __restrict__ vu,
+                                                            const float4* __restrict__ eu, float4* __restrict__ ps,
+                                                            float4* __restrict__ vs, float4* __restrict__ es,
+                                                            const float4* __restrict__ cu, float4* __restrict__ cs,
+                                                            int* __restrict__ left) {
+    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    const int num = d_num ? *d_num : num_host;
+    if (i >= num) {
+        if (i < n) {   // slots past the device's count: the pad key, as the stable sort leaves them
+            keys[i] = pad_key;
+            idx[i] = (uint32_t)i;
+        }
+        return;
+    }
+    const uint2 kv = pairs[i];
+    const float4 p = pu[kv.y], v = vu[kv.y], e = eu[kv.y];
+    const uint32_t cell = kv.x >> kSubBits, a = start[cell], b = end[cell];
+    // x sixteenth and index as one number: the order inside a cell
+    auto order = [](const uint2& q) { return (q.x << 28) | q.y; };
+    const uint32_t mine = order(kv);
+    uint32_t before = 0u, prev = 0u;   // pairs that precede this one; the last of them
+    auto member = [&](uint32_t o) {
+        const bool less = o < mine;
+        before += less ? 1u : 0u;
+        prev = max(prev, less ? o : 0u);
+    };
+    uint32_t j = a;
+    for (; j + 4 <= b; j += 4) {
+        uint2 q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[k] = pairs[j + k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) member(order(q[k]));
+    }
+    for (; j < b; ++j) member(order(pairs[j]));
+    const uint32_t to = a + before;
+    keys[to] = kv.x;
+    idx[to] = kv.y;
+    ps[to] = p;
+    vs[to] = v;
+    es[to] = e;
+    if (cu) cs[to] = cu[kv.y];   // permute.cl:41 (colours, when the system keeps them)
+    if (left && cell >= (uint32_t)nb_cells) *left = 1;
+    if (sub && cell < (uint32_t)nb_cells) {
+        // sub-cell starts: entry q = first index of the cell with x sixteenth
+        // >= q (the cell's end when none); each is written by the pair that
+        // starts it
+        const uint32_t xq = kv.x & (kSubCells - 1);
+        uint32_t* row = sub + (size_t)cell * kSubCells;
+        for (uint32_t q = before ? (prev >> 28) + 1u : 0u; q <= xq; ++q) row[q] = to;
+        if (to + 1 == b)
+            for (uint32_t q = xq + 1; q < (uint32_t)kSubCells; ++q) row[q] = b;
+    }
+}
+
+hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* pos_u, const Grid& g,
+                           uint32_t* keys, uint32_t* idx, uint32_t* start, uint32_t* end, void* temp,
+                           hipStream_t st) {
+    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
+    if (n <= 0) return hipSuccess;
+    CellTemp t;
+    cell_layout(n, g.nb_cells, &t, (char*)temp);
+    k_cell_count<<<cs_blocks(std::max(n, kScanBlocks)), kCsThreads, 0, st>>>(num_host, d_num, pos_u, g, keys, idx,
+                                                                             t.count, t.status);
+    const int n_cells = g.nb_cells + 1;
+    const int want = std::min(kScanBlocks, (n_cells + kScanTile - 1) / kScanTile);
+    const int chunk = ((n_cells + want - 1) / want + 3) & ~3;
+    k_cell_scan<<<(n_cells + chunk - 1) / chunk, kScanThreads, 0, st>>>(n_cells, chunk, t.count, start, end, t.status);
+    k_cell_place<<<cs_blocks(n), kCsThreads, 0, st>>>(num_host, d_num, keys, idx, start, t.pairs);
+    return hipGetLastError();
+}
+
+hipError_t cell_sort_finish(int n, int num_host, const int* d_num, uint32_t pad_key, int nb_cells,
+                            const uint32_t* start, const uint32_t* end, uint32_t* sub, uint32_t* keys, uint32_t* idx,
+                            const float4* pu, const float4* vu, const float4* eu, float4* ps, float4* vs, float4* es,
+                            void* temp, hipStream_t st, const float4* cu, float4* cs, int* left) {
+    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
+    if (n <= 0) return hipSuccess;
+    CellTemp t;
+    cell_layout(n, nb_cells, &t, (char*)temp);
+    k_cell_finish<<<cs_blocks(n), kCsThreads, 0, st>>>(n, num_host, d_num, pad_key, t.pairs, nb_cells, start, end, sub,
+                                                       keys, idx, pu, vu, eu, ps, vs, es, cu, cs, left);
+    return hipGetLastError();
+}
+
+}  // namespace rtps

@@ -196,6 +196,24 @@ hipError_t hash_sort_pairs(int n, int key_bits, const float4* pos_u, int num_hos
 hipError_t sort_segments(int batch, int length, int dir, uint32_t* dkeys, uint32_t* dvals, const uint32_t* skeys,
                          const uint32_t* svals, void* temp, hipStream_t st);
 
+// ---- counting sort of the step's particles by cell (cell_sort.hip) ----
+constexpr int kCellSortMax = 5 << 16;   // particles
+// True when cell_sort_place takes n particles on a grid of nb_cells cells.
+bool cell_sort_fits(int n, int nb_cells);
+size_t cell_sort_temp_bytes(int n, int nb_cells);   // for every count up to n
+hipError_t cell_sort_clear_temp(void* temp, int nb_cells, hipStream_t st);   // before the first sort
+// hash, sort and cellindices up to the order inside the cells (start and end
+// are written); then that order (keys, idx: hash_sort_pairs's result), the
+// sub-cell table (may be null) and the permute, as launch_cells_permute.
+hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* pos_u, const Grid& g,
+                           uint32_t* keys, uint32_t* idx, uint32_t* start, uint32_t* end, void* temp,
+                           hipStream_t st);
+hipError_t cell_sort_finish(int n, int num_host, const int* d_num, uint32_t pad_key, int nb_cells,
+                            const uint32_t* start, const uint32_t* end, uint32_t* sub, uint32_t* keys, uint32_t* idx,
+                            const float4* pu, const float4* vu, const float4* eu, float4* ps, float4* vs, float4* es,
+                            void* temp, hipStream_t st, const float4* cu = nullptr, float4* cs = nullptr,
+                            int* left = nullptr);
+
 // ---- bucket sort of the step's cell keys (bucket_sort.hip) ----
 // True when hash_bucket_sort takes n keys of key_bits bits.
 bool bucket_sort_fits(int n, int key_bits);

@@ -55,13 +55,14 @@ struct rtps_sph {
     int* d_num = nullptr;
     int* tile_q = nullptr;   // per-XCD tile queue counters of the neighbour kernels (kTileQueueWords)
     void* sort_tmp = nullptr;
+    void* cell_tmp = nullptr;   // the counting sort's (cell_sort.hip)
     // the neighbour rows the density kernel records for force loop 5 (Win::rows):
     // 9 rows x 3 words per particle slot, then 9 x 2 words per wave of 64 slots
     uint32_t* rows = nullptr;
     GravitySources gsrc{};
     int opt_collision = 1, opt_graph = 1, opt_force_out = 0, opt_timers = 0, opt_window = 1, opt_remap = 0,
         opt_queues = 0;
-    int opt_bucket = 1;   // the step's keys: bucket sort where the key space allows it (1) or LSD radix sort (0)
+    int opt_bucket = 1;   // the step's sort: by cell or by bucket where they apply (1) or LSD radix sort (0)
     int opt_rows = 1;     // density records the neighbour rows for force loop 5 (1) or force looks them up (0)
     int opt_autotune = 1;
     int opt_color = 0;   // permute colours every step (set by the first non-default colour pushed)
@@ -106,7 +107,7 @@ struct rtps_sph {
         for (auto& g : gexec_t)
             if (g) (void)hipGraphExecDestroy(g);
         void* bufs[] = {pos_u, vel_u, veleval_u, pos_s, vel_s, ve_s,  force_s,  xsph_s,   color_u,
-                        color_s, keys, idx, start, end, d_num, sort_tmp, sub_start, tile_q, rows};
+                        color_s, keys, idx, start, end, d_num, sort_tmp, cell_tmp, sub_start, tile_q, rows};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
         void* sbufs[] = {cf_field, mc_cases, mc_counts, mc_offs, mc_tiles, mc_total, mc_words, mc_ntri, mesh_v, mesh_n};
@@ -216,7 +217,13 @@ int launch_front(rtps_sph* s, StageTimer& t) {
     // stage holds both, the "hash" stage is empty
     t.mark(ST_HASH);
     t.mark(ST_SORT);
-    if (s->opt_bucket && bucket_sort_fits(n, s->key_bits)) {
+    const bool by_cell = s->opt_bucket && cell_sort_fits(n, s->nb_cells);
+    if (by_cell) {
+        RTPS_TRY_HIP(cell_sort_place(n, n, s->d_num, s->pos_u, s->g, s->keys, s->idx, s->start, s->end, s->cell_tmp,
+                                     s->stream));
+        s->keys_sorted = s->keys;
+        s->idx_sorted = s->idx;
+    } else if (s->opt_bucket && bucket_sort_fits(n, s->key_bits)) {
         RTPS_TRY_HIP(hash_bucket_sort(n, s->key_bits, s->pos_u, n, s->d_num, s->pad_key, s->g, kSubBits, s->start,
                                       s->nb_cells + 1, s->keys, s->idx, s->sort_tmp, s->stream));
         s->keys_sorted = s->keys;
@@ -226,12 +233,18 @@ int launch_front(rtps_sph* s, StageTimer& t) {
                                      s->nb_cells + 1, s->keys, s->idx, s->sort_tmp, s->stream, &s->keys_sorted,
                                      &s->idx_sorted));
     }
-    // cellindices and permute in one kernel: the "cellindices" stage holds
-    // both, the "permute" stage is empty
+    // cellindices and permute in one kernel (with the order inside the cells,
+    // where the sort is by cell): the "cellindices" stage holds both, the
+    // "permute" stage is empty
     t.mark(ST_CELL);
-    RTPS_TRY_HIP(launch_cells_permute(n, s->d_num, s->keys_sorted, s->nb_cells, s->start, s->end, kSubBits,
-                                      sub_table_to_write(s), s->idx_sorted, s->pos_u, s->vel_u, s->veleval_u,
-                                      s->pos_s, s->vel_s, s->ve_s, s->stream, col_u(s), col_s(s)));
+    if (by_cell)
+        RTPS_TRY_HIP(cell_sort_finish(n, n, s->d_num, s->pad_key, s->nb_cells, s->start, s->end, sub_table_to_write(s),
+                                      s->keys, s->idx, s->pos_u, s->vel_u, s->veleval_u, s->pos_s, s->vel_s, s->ve_s,
+                                      s->cell_tmp, s->stream, col_u(s), col_s(s)));
+    else
+        RTPS_TRY_HIP(launch_cells_permute(n, s->d_num, s->keys_sorted, s->nb_cells, s->start, s->end, kSubBits,
+                                          sub_table_to_write(s), s->idx_sorted, s->pos_u, s->vel_u, s->veleval_u,
+                                          s->pos_s, s->vel_s, s->ve_s, s->stream, col_u(s), col_s(s)));
     s->sub_valid = sub_table_to_write(s) != nullptr;
     t.mark(ST_PERMUTE);
     t.mark(ST_DENSITY);
@@ -661,6 +674,8 @@ int rtps_sph_create(const char* const* keys, const char* const* vals, int n, rtp
             RTPS_TRY_HIP(dalloc(&s->sub_start, (size_t)s->nb_cells * kSubCells));
         // the bucket sort's temp, a superset of the radix sort's, for every count up to N
         RTPS_TRY_HIP(hipMalloc(&s->sort_tmp, bucket_temp_bytes((int)N, s->key_bits)));
+        RTPS_TRY_HIP(hipMalloc(&s->cell_tmp, cell_sort_temp_bytes(std::min((int)N, kCellSortMax), s->nb_cells)));
+        RTPS_TRY_HIP(cell_sort_clear_temp(s->cell_tmp, s->nb_cells, s->stream));
         RTPS_TRY_HIP(dalloc(&s->rows, 27 * N + 18 * ((N + 63) / 64)));
         float4* zf[] = {s->pos_u, s->vel_u, s->veleval_u, s->pos_s, s->vel_s, s->ve_s, s->force_s, s->xsph_s};
         for (float4* p : zf) RTPS_TRY_HIP(hipMemsetAsync(p, 0, N * sizeof(float4), s->stream));

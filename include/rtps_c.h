@@ -320,9 +320,11 @@ int rtps_sph_get_params(rtps_sph* s, rtps_sph_params* sphp, rtps_grid_params* gp
  *                        XCD's L2 then serves one stretch of the neighbour
  *                        rows); 0 = one tile per block in RTPS_OPT_TILE_REMAP
  *                        order.  The same results either way.
- *   RTPS_OPT_BUCKET_SORT 1 = the step sorts its cell keys by bucket (a
+ *   RTPS_OPT_BUCKET_SORT 1 = the step sorts its particles by grid cell (a
+ *                        counting sort, up to 327,680 particles on grids of
+ *                        few enough cells) or its cell keys by bucket (a
  *                        histogram of key buckets, the keys placed by bucket,
- *                        each bucket sorted by one wave) where the key space
+ *                        each bucket sorted by one wave), where the key space
  *                        has at most 2^16 buckets averaging at most 1024 keys
  *                        (default), 0 = the LSD radix sort of rtps_sort_pairs.
  *                        The same order either way (keys ascending, equal keys

@@ -115,3 +115,21 @@ def test_bucket_sort_option_is_checked(cuda):
     with pytest.raises(RTPSError):
         s.setOption(OPT_BUCKET_SORT, 2)
     s.close()
+
+
+@pytest.mark.parametrize("n", [5 << 16, (5 << 16) + 1])
+def test_sorts_at_the_line_between_them_equal_the_radix_sort(cuda, n):
+    """The counting sort by cell takes up to 5 * 2^16 particles, the bucket sort
+    more: at both counts a scene with mixed order, 9000 particles in one cell,
+    a run of 400 equal keys and particles outside the grid gives the radix
+    sort's step."""
+    dam = scenes.dam_custom(128, 128, 21, seed=33)
+    box = dict(dam.settings, max_num_particles=str(n))
+    pos = dam.pos[:n][np.random.default_rng(34).permutation(n)].copy()
+    pos[:9000, :3] = _clump(9000, 0.5, 35, (0.7, 0.7, 0.7))[:, :3]
+    pos[9000:9400, :3] = np.float32(0.9)
+    pos[9400:12000:13, 1] = np.float32(-7.0)
+    vel = np.zeros_like(pos)
+    a, b = (_run(box, pos, vel, bucket, 1) for bucket in (1, 0))
+    for x, y in zip(a, b):
+        np.testing.assert_array_equal(x, y)
