@@ -495,12 +495,15 @@ __global__ __launch_bounds__(192, 5) void k_pairs_split_b(const BatchItem* __res
     }
 }
 
+// The scenes' counts after the step, on the device and in host memory (a read
+// of a count then costs the wait for the step, not a transfer of 20 us).
 __global__ void k_commit_b(int S, const SceneDev* __restrict__ scenes, int* __restrict__ d_num,
-                           const uint32_t* __restrict__ start) {
+                           int* __restrict__ num_seen, const uint32_t* __restrict__ start) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= S) return;
     int num;
     if (scene_num(scenes[s], d_num[s], start, num)) d_num[s] = num;
+    num_seen[s] = num;
 }
 
 hipError_t launch_hash_b(int T, const uint16_t* sid, const SceneDev* scenes, const int* d_num, const float4* pos_u,
@@ -592,9 +595,10 @@ hipError_t launch_pairs_split_b(int mode, int n_items64, const BatchItem* items6
     return hipGetLastError();
 }
 
-hipError_t launch_commit_b(int S, const SceneDev* scenes, int* d_num, const uint32_t* start, hipStream_t st) {
+hipError_t launch_commit_b(int S, const SceneDev* scenes, int* d_num, int* num_seen, const uint32_t* start,
+                           hipStream_t st) {
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    k_commit_b<<<(S + 63) / 64, 64, 0, st>>>(S, scenes, d_num, start);
+    k_commit_b<<<(S + 63) / 64, 64, 0, st>>>(S, scenes, d_num, num_seen, start);
     return hipGetLastError();
 }
 

@@ -35,6 +35,7 @@ struct rtps_batch {
     hipStream_t stream = nullptr;
     SceneDev* scenes = nullptr;
     int* d_num = nullptr;
+    int* num_seen = nullptr;   // d_num in pinned host memory, as of the last finished step (commit writes both)
     uint16_t* sid = nullptr;
     float4 *pos_u = nullptr, *vel_u = nullptr, *veleval_u = nullptr, *pos_s = nullptr, *vel_s = nullptr,
            *ve_s = nullptr;
@@ -71,6 +72,7 @@ struct rtps_batch {
                         start, end, items, items128, items64, queues, sort_tmp, sub, rows};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
+        if (num_seen) (void)hipHostFree(num_seen);
         for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);
@@ -150,7 +152,7 @@ int launch_step(rtps_batch* b) {
     mark(b, B_FORCE);
     rc = launch_force_b(b, b->cfg_force);
     if (rc) return rc;
-    RTPS_TRY_HIP(launch_commit_b(b->S, b->scenes, b->d_num, b->start, b->stream));
+    RTPS_TRY_HIP(launch_commit_b(b->S, b->scenes, b->d_num, b->num_seen, b->start, b->stream));
     mark(b, B_N);
     return RTPS_OK;
 }
@@ -297,7 +299,7 @@ int autotune_step_b(rtps_batch* b, bool measure) {
     // finish the step: the force step with the chosen configuration, then the count commit
     rc = launch_force_b(b, b->cfg_force);
     if (rc) return rc;
-    RTPS_TRY_HIP(launch_commit_b(b->S, b->scenes, b->d_num, b->start, b->stream));
+    RTPS_TRY_HIP(launch_commit_b(b->S, b->scenes, b->d_num, b->num_seen, b->start, b->stream));
     return RTPS_OK;
 }
 
@@ -450,6 +452,8 @@ int rtps_batch_create(int num_scenes, const int* n_settings, const char* const* 
         const size_t NT = (size_t)T;
         RTPS_TRY_HIP(hipMalloc((void**)&b->scenes, sizeof(SceneDev) * num_scenes));
         RTPS_TRY_HIP(hipMalloc((void**)&b->d_num, sizeof(int) * num_scenes));
+        RTPS_TRY_HIP(hipHostMalloc((void**)&b->num_seen, sizeof(int) * num_scenes, hipHostMallocDefault));
+        std::fill(b->num_seen, b->num_seen + num_scenes, 0);
         RTPS_TRY_HIP(hipMalloc((void**)&b->sid, sizeof(uint16_t) * NT));
         float4** f4[] = {&b->pos_u, &b->vel_u, &b->veleval_u, &b->pos_s, &b->vel_s, &b->ve_s};
         for (float4** p : f4) {
@@ -507,8 +511,8 @@ int rtps_batch_num_scenes(rtps_batch* b, int* num_scenes, int* total_slots) {
 
 int rtps_batch_get_num(rtps_batch* b, int scene, int* num) {
     if (!b || !num || scene < 0 || scene >= b->S) return set_error(RTPS_ERR_ARG, "rtps_batch_get_num: bad arguments");
-    RTPS_TRY_HIP(hipMemcpyAsync(num, b->d_num + scene, sizeof(int), hipMemcpyDeviceToHost, b->stream));
     RTPS_TRY_HIP(hipStreamSynchronize(b->stream));
+    *num = b->num_seen[scene];
     return RTPS_OK;
 }
 
@@ -532,6 +536,7 @@ int rtps_batch_push_particles(rtps_batch* b, int scene, const rtps_float4* pos, 
     RTPS_TRY_HIP(hipMemcpyAsync(b->d_num + scene, &num, sizeof(int), hipMemcpyHostToDevice, b->stream));
     RTPS_TRY_HIP(hipStreamSynchronize(b->stream));
     b->num_h[scene] = num;
+    b->num_seen[scene] = num;
     return RTPS_OK;
 }
 

@@ -68,6 +68,7 @@ hipError_t launch_pairs_split_b(int mode, int n_items64, const BatchItem* items6
                                 const uint32_t* keys, float4* ve, const float4* vel_s, const uint32_t* idx,
                                 float4* pos_u, float4* vel_u, float4* veleval_u, float4* force_out, int* left,
                                 const uint32_t* sub, uint32_t* rows, uint32_t rows_stride, hipStream_t st);
-hipError_t launch_commit_b(int S, const SceneDev* scenes, int* d_num, const uint32_t* start, hipStream_t st);
+hipError_t launch_commit_b(int S, const SceneDev* scenes, int* d_num, int* num_seen, const uint32_t* start,
+                           hipStream_t st);
 
 }  // namespace rtps
