@@ -124,14 +124,16 @@ hipError_t launch_color_field(int res, const float4* pos_s, const float4* ve_s, 
                               const uint32_t* end, const rtps_sph_params& sp, const Grid& g, const Win& win,
                               const rtps_float4& bmin_scaled, const rtps_float4& bmax_scaled, float* field,
                               hipStream_t st);
+// tile_sums: surface_scan_tiles() + 1 words, afterwards each tile's first triangle and the total
 hipError_t launch_mc_count(int res, float iso, const float* field, const uint8_t* ntri, uint8_t* cases,
-                           uint32_t* counts, uint32_t* offs, uint32_t* tile_sums, uint32_t* total, hipStream_t st);
+                           uint32_t* tile_sums, hipStream_t st);
 // the corner and edge tables into the emit kernel's constant memory (once per process)
 hipError_t mc_upload_geometry();
-hipError_t launch_mc_emit(int res, float iso, const float* field, const uint8_t* cases, const uint32_t* counts,
-                          const uint32_t* offs, const uint32_t* tile_offs, const uint64_t* words,
-                          const rtps_float4& wmin, const rtps_float4& wmax, int frame, long capacity, float* verts,
-                          float* normals, hipStream_t st);
+// The surface's triangles at their scanned offsets.
+hipError_t launch_mc_emit(int res, float iso, const float* field, const uint8_t* cases, const uint8_t* ntri,
+                          const uint32_t* tile_offs, const uint64_t* words, const rtps_float4& wmin,
+                          const rtps_float4& wmax, int frame, long capacity, float* verts, float* normals,
+                          hipStream_t st);
 
 // ---- rigid-body coupling (rigid.hip) ----
 // One set of rigid-body particles in the fluid's grid: sorted positions (and,

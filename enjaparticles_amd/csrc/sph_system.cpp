@@ -87,7 +87,7 @@ struct rtps_sph {
     int cf_res = 0;
     float* cf_field = nullptr;
     uint8_t* mc_cases = nullptr;
-    uint32_t *mc_counts = nullptr, *mc_offs = nullptr, *mc_tiles = nullptr, *mc_total = nullptr;
+    uint32_t* mc_tiles = nullptr;   // the cube tiles' first triangles, then the total
     uint64_t* mc_words = nullptr;   // the case table, one packed word per case
     uint8_t* mc_ntri = nullptr;
     float *mesh_v = nullptr, *mesh_n = nullptr;
@@ -110,7 +110,7 @@ struct rtps_sph {
                         color_s, keys, idx, start, end, d_num, sort_tmp, cell_tmp, sub_start, tile_q, rows};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
-        void* sbufs[] = {cf_field, mc_cases, mc_counts, mc_offs, mc_tiles, mc_total, mc_words, mc_ntri, mesh_v, mesh_n};
+        void* sbufs[] = {cf_field, mc_cases, mc_tiles, mc_words, mc_ntri, mesh_v, mesh_n};
         for (void* b : sbufs)
             if (b) (void)hipFree(b);
         for (RigidDev& r : rigid) {
@@ -1046,23 +1046,20 @@ int surface_buffers(rtps_sph* s, int res) {
         RTPS_TRY_HIP(hipMalloc(&s->mc_ntri, sizeof(t.ntri)));
         RTPS_TRY_HIP(hipMemcpy(s->mc_words, kMcCaseWords, sizeof(kMcCaseWords), hipMemcpyHostToDevice));
         RTPS_TRY_HIP(hipMemcpy(s->mc_ntri, t.ntri, sizeof(t.ntri), hipMemcpyHostToDevice));
-        RTPS_TRY_HIP(hipMalloc(&s->mc_total, sizeof(uint32_t)));
     }
     if (s->cf_res == res) return RTPS_OK;
     RTPS_TRY_HIP(hipStreamSynchronize(s->stream));
-    void* old[] = {s->cf_field, s->mc_cases, s->mc_counts, s->mc_offs, s->mc_tiles};
+    void* old[] = {s->cf_field, s->mc_cases, s->mc_tiles};
     for (void* b : old)
         if (b) RTPS_TRY_HIP(hipFree(b));
     s->cf_field = nullptr;
     s->mc_cases = nullptr;
-    s->mc_counts = s->mc_offs = s->mc_tiles = nullptr;
+    s->mc_tiles = nullptr;
     s->cf_res = 0;
     const size_t nodes = (size_t)res * res * res, m = (size_t)(res - 1), cubes = m * m * m;
     RTPS_TRY_HIP(hipMalloc(&s->cf_field, nodes * sizeof(float)));
     RTPS_TRY_HIP(hipMalloc(&s->mc_cases, cubes));
-    RTPS_TRY_HIP(hipMalloc(&s->mc_counts, cubes * sizeof(uint32_t)));
-    RTPS_TRY_HIP(hipMalloc(&s->mc_offs, cubes * sizeof(uint32_t)));
-    RTPS_TRY_HIP(hipMalloc(&s->mc_tiles, surface_scan_tiles((long)cubes) * sizeof(uint32_t)));
+    RTPS_TRY_HIP(hipMalloc(&s->mc_tiles, (surface_scan_tiles((long)cubes) + 1) * sizeof(uint32_t)));
     s->cf_res = res;
     return RTPS_OK;
 }
@@ -1084,10 +1081,10 @@ int color_field(rtps_sph* s, int res) {
 int surface(rtps_sph* s, int res, float iso) {
     int rc = color_field(s, res);
     if (rc) return rc;
-    RTPS_TRY_HIP(launch_mc_count(res, iso, s->cf_field, s->mc_ntri, s->mc_cases, s->mc_counts, s->mc_offs,
-                                 s->mc_tiles, s->mc_total, s->stream));
+    RTPS_TRY_HIP(launch_mc_count(res, iso, s->cf_field, s->mc_ntri, s->mc_cases, s->mc_tiles, s->stream));
+    const long m = res - 1;
     uint32_t total = 0;
-    RTPS_TRY_HIP(hipMemcpyAsync(&total, s->mc_total, sizeof(total), hipMemcpyDeviceToHost, s->stream));
+    RTPS_TRY_HIP(hipMemcpyAsync(&total, s->mc_tiles + surface_scan_tiles(m * m * m), sizeof(total), hipMemcpyDeviceToHost, s->stream));
     RTPS_TRY_HIP(hipStreamSynchronize(s->stream));
     if ((long)total > s->mesh_cap) {
         if (s->mesh_v) RTPS_TRY_HIP(hipFree(s->mesh_v));
@@ -1101,7 +1098,7 @@ int surface(rtps_sph* s, int res, float iso) {
     }
     s->mesh_ntri = (int)total;
     if (total > 0)
-        RTPS_TRY_HIP(launch_mc_emit(res, iso, s->cf_field, s->mc_cases, s->mc_counts, s->mc_offs, s->mc_tiles,
+        RTPS_TRY_HIP(launch_mc_emit(res, iso, s->cf_field, s->mc_cases, s->mc_ntri, s->mc_tiles,
                                     s->mc_words, s->gp.bnd_min, s->gp.bnd_max, s->opt_frame, s->mesh_cap, s->mesh_v,
                                     s->mesh_n,
                                     s->stream));
