@@ -52,6 +52,7 @@ struct rtps_badj {
     std::vector<BState> ck_state;      // checkpoints
     std::vector<BRecord> rec;          // records of one segment's steps (or of as many as fit)
     uint32_t *keys = nullptr, *start = nullptr, *end = nullptr, *sub = nullptr;   // of the step at hand
+    bool by_cell = false;   // sorted by cell_sort.hip's counting sort
     void* sort_tmp = nullptr;
     float4 *lam_x[2] = {}, *lam_v[2] = {}, *lam_e[2] = {};
     float4 *ga = nullptr, *gX = nullptr, *lxp = nullptr, *gx2 = nullptr, *ge = nullptr;
@@ -107,13 +108,21 @@ hipError_t alloc_records(rtps_badj* a, int want) {
 // left in r; force: also the SPH force, which only the adjoint reads.
 int forward_step(rtps_badj* a, const BState& in, const BState& out, BRecord& r, bool force, hipStream_t st) {
     const int T = a->T;
-    RTPS_TRY_HIP(launch_hash_b(T, a->sid, a->scenes, a->d_num, in.pos, a->keys, r.idx, a->start, a->C, st));
-    uint32_t *ks, *is;
-    RTPS_TRY_HIP(sort_pairs_passes(T, a->L.shifts, a->L.widths, a->L.npasses, a->keys, r.idx, a->sort_tmp, st, &ks,
-                                   &is));
-    if (is != r.idx) RTPS_TRY_HIP(hipMemcpyAsync(r.idx, is, (size_t)T * 4, hipMemcpyDeviceToDevice, st));
-    RTPS_TRY_HIP(launch_cellindices_b(T, ks, a->scenes, a->start, a->end, st, a->sub));
-    RTPS_TRY_HIP(launch_permute(T, nullptr, r.idx, in.pos, in.vel, in.ve, r.pos_s, r.vel_s, r.ve_s, st));
+    uint32_t* ks = a->keys;
+    if (a->by_cell) {
+        RTPS_TRY_HIP(cell_sort_place_b(T, a->sid, a->scenes, a->d_num, in.pos, a->C, a->keys, r.idx, a->start, a->end,
+                                       a->sort_tmp, st));
+        RTPS_TRY_HIP(cell_sort_finish_b(T, a->sid, a->scenes, a->d_num, a->C, a->start, a->end, a->sub, a->keys,
+                                        r.idx, in.pos, in.vel, in.ve, r.pos_s, r.vel_s, r.ve_s, a->sort_tmp, st));
+    } else {
+        RTPS_TRY_HIP(launch_hash_b(T, a->sid, a->scenes, a->d_num, in.pos, a->keys, r.idx, a->start, a->C, st));
+        uint32_t* is;
+        RTPS_TRY_HIP(sort_pairs_passes(T, a->L.shifts, a->L.widths, a->L.npasses, a->keys, r.idx, a->sort_tmp, st, &ks,
+                                       &is));
+        if (is != r.idx) RTPS_TRY_HIP(hipMemcpyAsync(r.idx, is, (size_t)T * 4, hipMemcpyDeviceToDevice, st));
+        RTPS_TRY_HIP(launch_cellindices_b(T, ks, a->scenes, a->start, a->end, st, a->sub));
+        RTPS_TRY_HIP(launch_permute(T, nullptr, r.idx, in.pos, in.vel, in.ve, r.pos_s, r.vel_s, r.ve_s, st));
+    }
     for (int mode : {kPairsDensity, kPairsForceStep})
         RTPS_TRY_HIP(launch_pairs_split_b(mode, a->n_items64, a->items64, a->scenes, r.pos_s, a->start, a->end, ks,
                                           r.ve_s, r.vel_s, r.idx, out.pos, out.vel, out.ve,
@@ -178,7 +187,9 @@ int rtps_badj_create(int num_scenes, const int* n_settings, const char* const* k
         RTPS_TRY_HIP(a->alloc(&a->end, C));
         if (C * kSubCells * sizeof(uint32_t) <= ((size_t)2 << 30))   // as the batched system's
             RTPS_TRY_HIP(a->alloc(&a->sub, C * kSubCells));
-        RTPS_TRY_HIP(a->alloc((char**)&a->sort_tmp, sort_temp_bytes((int)N, 32)));
+        a->by_cell = cell_sort_fits_b((long)N, (long)C);
+        RTPS_TRY_HIP(a->alloc((char**)&a->sort_tmp, a->by_cell ? cell_sort_temp_bytes((int)N, (int)C - 1)
+                                                               : sort_temp_bytes((int)N, 32)));
         RTPS_TRY_HIP(a->alloc(&a->ga, N));
         RTPS_TRY_HIP(a->alloc(&a->gX, N));
         RTPS_TRY_HIP(a->alloc(&a->lxp, N));
@@ -206,7 +217,8 @@ int rtps_badj_create(int num_scenes, const int* n_settings, const char* const* k
         RTPS_TRY_HIP(hipMemcpy(a->item_first, a->L.item_first.data(), sizeof(int) * (num_scenes + 1),
                                hipMemcpyHostToDevice));
         RTPS_TRY_HIP(hipMemcpy(a->scenes, a->L.scenes.data(), sizeof(SceneDev) * num_scenes, hipMemcpyHostToDevice));
-        RTPS_TRY_HIP(sort_clear_temp(a->sort_tmp, (int)N, nullptr));
+        RTPS_TRY_HIP(a->by_cell ? cell_sort_clear_temp(a->sort_tmp, (int)C - 1, nullptr)
+                                : sort_clear_temp(a->sort_tmp, (int)N, nullptr));
         RTPS_TRY_HIP(launch_fill_u32(a->end, 0u, (long)C, nullptr));
         RTPS_TRY_HIP(hipDeviceSynchronize());
         *out = a.release();

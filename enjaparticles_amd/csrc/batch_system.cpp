@@ -51,6 +51,7 @@ struct rtps_batch {
     int opt_autotune = 1;
     bool tuned = false;
     int* queues = nullptr;
+    bool by_cell = false;      // sorted by cell_sort.hip's counting sort
     void* sort_tmp = nullptr;
     uint32_t* sub = nullptr;   // sub-cell starts of the windowed rows, 16 per cell
     // neighbour rows the density kernel records for the force kernel: 9 rows
@@ -129,6 +130,18 @@ int launch_force_b(rtps_batch* b, const PairsCfg& c) {
 }
 
 int launch_front_b(rtps_batch* b) {
+    if (b->by_cell) {
+        mark(b, B_HASH);
+        mark(b, B_SORT);
+        RTPS_TRY_HIP(cell_sort_place_b(b->T, b->sid, b->scenes, b->d_num, b->pos_u, b->total_cells, b->keys, b->idx,
+                                       b->start, b->end, b->sort_tmp, b->stream));
+        mark(b, B_CELL);
+        mark(b, B_PERMUTE);
+        RTPS_TRY_HIP(cell_sort_finish_b(b->T, b->sid, b->scenes, b->d_num, b->total_cells, b->start, b->end, b->sub,
+                                        b->keys, b->idx, b->pos_u, b->vel_u, b->veleval_u, b->pos_s, b->vel_s,
+                                        b->ve_s, b->sort_tmp, b->stream));
+        return RTPS_OK;
+    }
     mark(b, B_HASH);
     RTPS_TRY_HIP(launch_hash_b(b->T, b->sid, b->scenes, b->d_num, b->pos_u, b->keys, b->idx, b->start,
                                b->total_cells, b->stream));
@@ -374,7 +387,7 @@ int build_batch_layout(int num_scenes, const int* n_settings, const char* const*
         d.collision = 1;
         gravity_sources_of(st, d.gsrc);
         T += cap;
-        cells += gp.nb_cells + 1;
+        cells += gp.nb_cells + 2;
         max_cells = std::max(max_cells, gp.nb_cells);
         if (T >= (1L << 31) - 1) return set_error(RTPS_ERR_ARG, "too many particle slots");
     }
@@ -470,7 +483,9 @@ int rtps_batch_create(int num_scenes, const int* n_settings, const char* const* 
         RTPS_TRY_HIP(hipMalloc((void**)&b->items128, sizeof(BatchItem) * L.items128.size()));
         RTPS_TRY_HIP(hipMalloc((void**)&b->items64, sizeof(BatchItem) * L.items64.size()));
         RTPS_TRY_HIP(hipMalloc((void**)&b->queues, kTileQueueWords * sizeof(int)));
-        RTPS_TRY_HIP(hipMalloc(&b->sort_tmp, sort_temp_bytes((int)T, 32)));
+        b->by_cell = cell_sort_fits_b(T, cells);
+        RTPS_TRY_HIP(hipMalloc(&b->sort_tmp, b->by_cell ? cell_sort_temp_bytes((int)T, (int)cells - 1)
+                                                        : sort_temp_bytes((int)T, 32)));
         RTPS_TRY_HIP(hipMalloc((void**)&b->rows, NT * 27 * 4));
         RTPS_TRY_HIP(hipMemcpyAsync(b->scenes, b->scenes_h.data(), sizeof(SceneDev) * num_scenes,
                                     hipMemcpyHostToDevice, b->stream));
@@ -485,7 +500,8 @@ int rtps_batch_create(int num_scenes, const int* n_settings, const char* const* 
         RTPS_TRY_HIP(hipMemsetAsync(b->queues, 0, kTileQueueWords * sizeof(int), b->stream));
         RTPS_TRY_HIP(launch_fill_u32(b->start, 666u, cells, b->stream));
         RTPS_TRY_HIP(launch_fill_u32(b->end, 666u, cells, b->stream));
-        RTPS_TRY_HIP(sort_clear_temp(b->sort_tmp, (int)T, b->stream));
+        RTPS_TRY_HIP(b->by_cell ? cell_sort_clear_temp(b->sort_tmp, (int)cells - 1, b->stream)
+                                : sort_clear_temp(b->sort_tmp, (int)T, b->stream));
         b->keys_sorted = b->keys;
         b->idx_sorted = b->idx;
         for (auto& e : b->ev) RTPS_TRY_HIP(hipEventCreateWithFlags(&e, kTimingEvent));

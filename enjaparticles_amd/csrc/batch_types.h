@@ -23,7 +23,8 @@ struct SceneDev {
     float dt;
     int off;                     // first slot of the scene in the particle arrays
     int cap;                     // slots of the scene (its max_num_particles)
-    int cell_base;               // first entry of the scene's cell table
+    int cell_base;               // first entry of the scene's cell table (nb_cells + 2 entries: the cells, the
+                                 // particles outside the grid, the unused slots)
     int collision;               // wall collision on
     GravitySources gsrc;         // point sources of gravity.cl (n = 0: none)
 };
@@ -37,6 +38,19 @@ hipError_t launch_hash_b(int T, const uint16_t* sid, const SceneDev* scenes, con
 // sub (optional): sub-cell start table, 16 entries per cell of every scene
 hipError_t launch_cellindices_b(int T, const uint32_t* keys, const SceneDev* scenes, uint32_t* start, uint32_t* end,
                                 hipStream_t st, uint32_t* sub = nullptr);
+// The counting sort of cell_sort.hip over the scenes' cells, in place of
+// launch_hash_b, the key sort, launch_cellindices_b and the permute; temp from
+// cell_sort_temp_bytes(T, total_cells - 1), cleared by cell_sort_clear_temp
+// before the first sort.  cell_sort_fits_b: where it is the faster one.  place: keys and idx are scratch; finish writes both
+// sorted, and pos, vel and veleval in that order.
+bool cell_sort_fits_b(long T, long total_cells);
+hipError_t cell_sort_place_b(int T, const uint16_t* sid, const SceneDev* scenes, const int* d_num,
+                             const float4* pos_u, int total_cells, uint32_t* keys, uint32_t* idx, uint32_t* start,
+                             uint32_t* end, void* temp, hipStream_t st);
+hipError_t cell_sort_finish_b(int T, const uint16_t* sid, const SceneDev* scenes, const int* d_num, int total_cells,
+                              const uint32_t* start, const uint32_t* end, uint32_t* sub, uint32_t* keys,
+                              uint32_t* idx, const float4* pu, const float4* vu, const float4* eu, float4* ps,
+                              float4* vs, float4* es, void* temp, hipStream_t st);
 constexpr int kPairsDensity = 0, kPairsForceStep = 1;
 // Launch configuration of a persistent pair kernel: `block` threads per block
 // (= slots per work item: 64, 128 or 256) and the register budget of `waves`

@@ -25,6 +25,7 @@
 
 #include <algorithm>
 
+#include "batch_types.h"
 #include "rtps_internal.h"
 #include "sort_layout.h"
 #include "sph_device.h"
@@ -71,6 +72,14 @@ hipError_t cell_sort_clear_temp(void* temp, int nb_cells, hipStream_t st) {
 // Grids with many more cells than particles take a sort of the keys instead:
 // the scan reads every cell's counter.
 bool cell_sort_fits(int n, int nb_cells) { return n <= kCellSortMax && (long)nb_cells <= 16L * n + (1 << 20); }
+
+// Batches: the other way there is hash, four or five digit passes, cellindices
+// and permute, nine launches in all.  Measured for all of it (us, digits /
+// counting; settled scenes, then at rest): 43 / 25 and 41 / 24 at 2,574 slots,
+// 76 / 57 and 72 / 41 at 216,557, 97 / 82 and 87 / 52 at 420,738, 132 / 125 and
+// 112 / 78 at 840,154, 187 / 187 and 159 / 122 at 1,356,782, 378 / 416 and 296 /
+// 278 at 3,534,703.  The line, 2^20 slots, is where settled scenes still gain.
+bool cell_sort_fits_b(long T, long total_cells) { return T <= 1 << 20 && total_cells <= 16 * T + (1 << 20); }
 
 __global__ __launch_bounds__(kCsThreads) void k_cell_count(int num_host, const int* __restrict__ d_num,
                                                            const float4* __restrict__ pos_u, Grid g,
@@ -183,6 +192,42 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_place(int num_host, const i
     if (at < (uint32_t)num) pairs[at] = make_uint2(key, (uint32_t)i);
 }
 
+// How many of the cell's pairs [a, b) precede kv (by x sixteenth, then index),
+// and the x sixteenth of the last of them in `prev_xq`.
+__device__ __forceinline__ uint32_t rank_in_cell(const uint2* __restrict__ pairs, uint2 kv, uint32_t a, uint32_t b,
+                                                 uint32_t& prev_xq) {
+    // x sixteenth and index as one number: the order inside a cell
+    auto order = [](const uint2& q) { return (q.x << 28) | q.y; };
+    const uint32_t mine = order(kv);
+    uint32_t before = 0u, prev = 0u;   // pairs that precede this one; the last of them
+    auto member = [&](uint32_t o) {
+        const bool less = o < mine;
+        before += less ? 1u : 0u;
+        prev = max(prev, less ? o : 0u);
+    };
+    uint32_t j = a;
+    for (; j + 4 <= b; j += 4) {
+        uint2 q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[k] = pairs[j + k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) member(order(q[k]));
+    }
+    for (; j < b; ++j) member(order(pairs[j]));
+    prev_xq = prev >> 28;
+    return before;
+}
+
+// The cell's sub-cell starts that the pair at `to` writes: entry q = first
+// index of the cell with x sixteenth >= q (the cell's end when none), each
+// written by the pair that starts it.
+__device__ __forceinline__ void write_sub_starts(uint32_t* __restrict__ row, uint32_t xq, uint32_t before,
+                                                 uint32_t prev_xq, uint32_t to, uint32_t b) {
+    for (uint32_t q = before ? prev_xq + 1u : 0u; q <= xq; ++q) row[q] = to;
+    if (to + 1 == b)
+        for (uint32_t q = xq + 1; q < (uint32_t)kSubCells; ++q) row[q] = b;
+}
+
 __global__ __launch_bounds__(kCsThreads) void k_cell_finish(int n, int num_host, const int* __restrict__ d_num,
                                                             uint32_t pad_key, const uint2* __restrict__ pairs,
                                                             int nb_cells, const uint32_t* __restrict__ start,
@@ -206,24 +251,8 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_finish(int n, int num_host,
     const uint2 kv = pairs[i];
     const float4 p = pu[kv.y], v = vu[kv.y], e = eu[kv.y];
     const uint32_t cell = kv.x >> kSubBits, a = start[cell], b = end[cell];
-    // x sixteenth and index as one number: the order inside a cell
-    auto order = [](const uint2& q) { return (q.x << 28) | q.y; };
-    const uint32_t mine = order(kv);
-    uint32_t before = 0u, prev = 0u;   // pairs that precede this one; the last of them
-    auto member = [&](uint32_t o) {
-        const bool less = o < mine;
-        before += less ? 1u : 0u;
-        prev = max(prev, less ? o : 0u);
-    };
-    uint32_t j = a;
-    for (; j + 4 <= b; j += 4) {
-        uint2 q[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) q[k] = pairs[j + k];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) member(order(q[k]));
-    }
-    for (; j < b; ++j) member(order(pairs[j]));
+    uint32_t prev_xq;
+    const uint32_t before = rank_in_cell(pairs, kv, a, b, prev_xq);
     const uint32_t to = a + before;
     keys[to] = kv.x;
     idx[to] = kv.y;
@@ -232,16 +261,124 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_finish(int n, int num_host,
     es[to] = e;
     if (cu) cs[to] = cu[kv.y];   // permute.cl:41 (colours, when the system keeps them)
     if (left && cell >= (uint32_t)nb_cells) *left = 1;
-    if (sub && cell < (uint32_t)nb_cells) {
-        // sub-cell starts: entry q = first index of the cell with x sixteenth
-        // >= q (the cell's end when none); each is written by the pair that
-        // starts it
-        const uint32_t xq = kv.x & (kSubCells - 1);
-        uint32_t* row = sub + (size_t)cell * kSubCells;
-        for (uint32_t q = before ? (prev >> 28) + 1u : 0u; q <= xq; ++q) row[q] = to;
-        if (to + 1 == b)
-            for (uint32_t q = xq + 1; q < (uint32_t)kSubCells; ++q) row[q] = b;
+    if (sub && cell < (uint32_t)nb_cells)
+        write_sub_starts(sub + (size_t)cell * kSubCells, kv.x & (kSubCells - 1), before, prev_xq, to, b);
+}
+
+// The same for the scenes of a batch: the cells of all scenes, counted
+// together, each scene's followed by one more that counts its unused slots (so
+// that every scene starts at its own slots).  Keys (scene << 24) | cell << 4 | x
+// sixteenth; unused slots keep their place and get (scene << 24) | 0xFFFFFF.
+constexpr uint32_t kPadLocal = (1u << kSceneShift) - 1u;
+
+__device__ __forceinline__ uint32_t cell_of_key(const SceneDev& S, uint32_t key) {
+    return (uint32_t)S.cell_base + ((key & kPadLocal) >> kSubBits);
+}
+
+__global__ __launch_bounds__(kCsThreads) void k_cell_count_b(int T, const uint16_t* __restrict__ sid,
+                                                             const SceneDev* __restrict__ scenes,
+                                                             const int* __restrict__ d_num,
+                                                             const float4* __restrict__ pos_u,
+                                                             uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                                                             uint32_t* __restrict__ count,
+                                                             unsigned long long* __restrict__ status) {
+    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    if (i < kScanBlocks) status[i] = 0ull;
+    if (i >= T) return;
+    const int s = sid[i];
+    const SceneDev& S = scenes[s];
+    const int num = d_num[s], at = i - S.off;
+    if (at >= num) {
+        if (at == num) count[S.cell_base + S.g.nb_cells + 1] = (uint32_t)(S.cap - num);
+        return;
     }
+    const uint32_t key = ((uint32_t)s << kSceneShift) | hash_key(pos_u[i], S.g, kSubBits);
+    keys[i] = key;
+    rank[i] = atomicAdd(&count[cell_of_key(S, key)], 1u);
+}
+
+__global__ __launch_bounds__(kCsThreads) void k_cell_place_b(int T, const uint16_t* __restrict__ sid,
+                                                             const SceneDev* __restrict__ scenes,
+                                                             const int* __restrict__ d_num,
+                                                             const uint32_t* __restrict__ keys,
+                                                             const uint32_t* __restrict__ rank,
+                                                             const uint32_t* __restrict__ start,
+                                                             uint2* __restrict__ pairs) {
+    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    if (i >= T) return;
+    const int s = sid[i];
+    const SceneDev& S = scenes[s];
+    if (i - S.off >= d_num[s]) return;
+    const uint32_t key = keys[i], at = start[cell_of_key(S, key)] + rank[i];
+    if (at < (uint32_t)T) pairs[at] = make_uint2(key, (uint32_t)i);
+}
+
+__global__ __launch_bounds__(kCsThreads) void k_cell_finish_b(int T, const uint16_t* __restrict__ sid,
+                                                              const SceneDev* __restrict__ scenes,
+                                                              const int* __restrict__ d_num,
+                                                              const uint2* __restrict__ pairs,
+                                                              const uint32_t* __restrict__ start,
+                                                              const uint32_t* __restrict__ end,
+                                                              uint32_t* __restrict__ sub, uint32_t* __restrict__ keys,
+                                                              uint32_t* __restrict__ idx,
+                                                              const float4* __restrict__ pu,
+                                                              const float4* __restrict__ vu,
+                                                              const float4* __restrict__ eu, float4* __restrict__ ps,
+                                                              float4* __restrict__ vs, float4* __restrict__ es) {
+    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    if (i >= T) return;
+    const int s = sid[i];
+    const SceneDev& S = scenes[s];
+    uint2 kv = make_uint2(((uint32_t)s << kSceneShift) | kPadLocal, (uint32_t)i);
+    uint32_t to = (uint32_t)i;
+    if (i - S.off < d_num[s]) {
+        kv = pairs[i];
+        const uint32_t cell = cell_of_key(S, kv.x), a = start[cell], b = end[cell];
+        uint32_t prev_xq;
+        const uint32_t before = rank_in_cell(pairs, kv, a, b, prev_xq);
+        to = a + before;
+        if (sub && cell < (uint32_t)(S.cell_base + S.g.nb_cells))
+            write_sub_starts(sub + (size_t)cell * kSubCells, kv.x & (kSubCells - 1), before, prev_xq, to, b);
+    }
+    const float4 p = pu[kv.y], v = vu[kv.y], e = eu[kv.y];
+    keys[to] = kv.x;
+    idx[to] = kv.y;
+    ps[to] = p;
+    vs[to] = v;
+    es[to] = e;
+}
+
+static void launch_cell_scan(int n_cells, const CellTemp& t, uint32_t* start, uint32_t* end, hipStream_t st) {
+    const int want = std::min(kScanBlocks, (n_cells + kScanTile - 1) / kScanTile);
+    const int chunk = ((n_cells + want - 1) / want + 3) & ~3;
+    k_cell_scan<<<(n_cells + chunk - 1) / chunk, kScanThreads, 0, st>>>(n_cells, chunk, t.count, start, end, t.status);
+}
+
+hipError_t cell_sort_place_b(int T, const uint16_t* sid, const SceneDev* scenes, const int* d_num,
+                             const float4* pos_u, int total_cells, uint32_t* keys, uint32_t* idx, uint32_t* start,
+                             uint32_t* end, void* temp, hipStream_t st) {
+    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
+    if (T <= 0) return hipSuccess;
+    CellTemp t;
+    cell_layout(T, total_cells - 1, &t, (char*)temp);
+    k_cell_count_b<<<cs_blocks(std::max(T, kScanBlocks)), kCsThreads, 0, st>>>(T, sid, scenes, d_num, pos_u, keys,
+                                                                               idx, t.count, t.status);
+    launch_cell_scan(total_cells, t, start, end, st);
+    k_cell_place_b<<<cs_blocks(T), kCsThreads, 0, st>>>(T, sid, scenes, d_num, keys, idx, start, t.pairs);
+    return hipGetLastError();
+}
+
+hipError_t cell_sort_finish_b(int T, const uint16_t* sid, const SceneDev* scenes, const int* d_num, int total_cells,
+                              const uint32_t* start, const uint32_t* end, uint32_t* sub, uint32_t* keys,
+                              uint32_t* idx, const float4* pu, const float4* vu, const float4* eu, float4* ps,
+                              float4* vs, float4* es, void* temp, hipStream_t st) {
+    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
+    if (T <= 0) return hipSuccess;
+    CellTemp t;
+    cell_layout(T, total_cells - 1, &t, (char*)temp);
+    k_cell_finish_b<<<cs_blocks(T), kCsThreads, 0, st>>>(T, sid, scenes, d_num, t.pairs, start, end, sub, keys, idx,
+                                                         pu, vu, eu, ps, vs, es);
+    return hipGetLastError();
 }
 
 hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* pos_u, const Grid& g,
@@ -253,10 +390,7 @@ hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* 
     cell_layout(n, g.nb_cells, &t, (char*)temp);
     k_cell_count<<<cs_blocks(std::max(n, kScanBlocks)), kCsThreads, 0, st>>>(num_host, d_num, pos_u, g, keys, idx,
                                                                              t.count, t.status);
-    const int n_cells = g.nb_cells + 1;
-    const int want = std::min(kScanBlocks, (n_cells + kScanTile - 1) / kScanTile);
-    const int chunk = ((n_cells + want - 1) / want + 3) & ~3;
-    k_cell_scan<<<(n_cells + chunk - 1) / chunk, kScanThreads, 0, st>>>(n_cells, chunk, t.count, start, end, t.status);
+    launch_cell_scan(g.nb_cells + 1, t, start, end, st);
     k_cell_place<<<cs_blocks(n), kCsThreads, 0, st>>>(num_host, d_num, keys, idx, start, t.pairs);
     return hipGetLastError();
 }
