@@ -61,6 +61,7 @@ struct rtps_badj {
     double* sums = nullptr;            // and their sums: [step][scene]
     std::vector<double> sums_h;
     bool have_forward = false;
+    int rec_lo = 0, rec_hi = 0;   // rec[0..] hold the steps rec_lo..rec_hi-1 of the last forward run
 
     ~rtps_badj() {
         (void)hipDeviceSynchronize();
@@ -269,6 +270,10 @@ int rtps_badj_forward(rtps_badj* a, const rtps_float4* pos0, const rtps_float4* 
         RTPS_TRY_HIP(launch_fill_u32((uint32_t*)s0.ve, 0u, (long)a->T * 4, st));   // veleval starts at zero
     }
     RTPS_TRY_HIP(launch_fill_u32((uint32_t*)a->left_grid, 0u, 1, st));
+    // The last segment's steps are recorded on the way: the adjoint starts
+    // there, and its replay begins with the segment before.
+    const int last_first = (nsteps - 1) / a->ck * a->ck, rec_lo = std::max(last_first, nsteps - (int)a->rec.size());
+    a->rec_lo = a->rec_hi = 0;
     for (int n = 0; n < nsteps; ++n) {
         const BState& in = n % a->ck == 0 ? a->ck_state[n / a->ck] : a->slot[n & 1];
         BState out = (n + 1) % a->ck == 0 && n + 1 < nsteps ? a->ck_state[(n + 1) / a->ck] : a->slot[(n + 1) & 1];
@@ -276,7 +281,7 @@ int rtps_badj_forward(rtps_badj* a, const rtps_float4* pos0, const rtps_float4* 
             if (aligned16(pos_T)) out.pos = (float4*)pos_T;
             if (vel_T && aligned16(vel_T)) out.vel = (float4*)vel_T;
         }
-        int rc = forward_step(a, in, out, a->rec[0], false, st);
+        int rc = forward_step(a, in, out, a->rec[std::max(n - rec_lo, 0)], n >= rec_lo, st);
         if (rc) return rc;
         if (n + 1 < nsteps) continue;
         if (!aligned16(pos_T)) RTPS_TRY_HIP(hipMemcpyAsync(pos_T, out.pos, nb, hipMemcpyDeviceToDevice, st));
@@ -286,6 +291,8 @@ int rtps_badj_forward(rtps_badj* a, const rtps_float4* pos0, const rtps_float4* 
     RTPS_TRY_HIP(hipMemcpyAsync(&left, a->left_grid, sizeof(int), hipMemcpyDeviceToHost, st));
     RTPS_TRY_HIP(hipStreamSynchronize(st));
     a->have_forward = true;
+    a->rec_lo = rec_lo;
+    a->rec_hi = nsteps;
     if (left) return set_error(RTPS_ERR_STATE, "particles left the grid during the forward run (no deletion path in "
                                                "the adjoint)");
     return RTPS_OK;
@@ -316,11 +323,16 @@ int rtps_badj_backward(rtps_badj* a, const rtps_float4* dL_dpos_T, const rtps_fl
         for (int hi = last, lo; hi > first; hi = lo) {
             lo = std::max(first, hi - R);
             // replay the segment from its checkpoint, recording the steps lo..hi-1
-            for (int s = first; s < hi; ++s) {
+            // (unless they are the ones recorded last)
+            const bool recorded = a->rec_lo == lo && a->rec_hi == hi;
+            if (!recorded) a->rec_lo = a->rec_hi = 0;
+            for (int s = recorded ? hi : first; s < hi; ++s) {
                 const BState& in = s == first ? a->ck_state[c] : a->slot[s & 1];
                 int rc = forward_step(a, in, a->slot[(s + 1) & 1], a->rec[s < lo ? 0 : s - lo], s >= lo, st);
                 if (rc) return rc;
             }
+            a->rec_lo = lo;
+            a->rec_hi = hi;
             for (int s = hi - 1; s >= lo; --s) {
                 const BRecord& r = a->rec[s - lo];
                 float4 *lv_out = a->lam_v[1 - L], *lx_out = a->lam_x[1 - L], *le_out = a->lam_e[1 - L];
