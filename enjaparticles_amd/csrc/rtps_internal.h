@@ -72,6 +72,17 @@ hipError_t launch_force_fused(int num, int* d_num, const float4* pos_s, const fl
                               const GravitySources& gsrc, int collision, const rtps_grid_params& gps, float dt,
                               float4* pos_u, float4* vel_u, float4* veleval_u, hipStream_t st,
                               const float4* color_s = nullptr, float4* color_u = nullptr);
+// The same for small launches on recorded rows, nine waves per 64 particles
+// (row_tiles.hip); the split order (Win::split) where the caller asks for it.
+hipError_t launch_density_rows(int num, const int* d_num, const float4* pos_s, const uint32_t* start,
+                               const uint32_t* end, const rtps_sph_params& sp, const Grid& g, const Win& win,
+                               float4* packed, hipStream_t st);
+hipError_t launch_force_rows(int num, int* d_num, const float4* pos_s, const float4* ve, const uint32_t* start,
+                             const rtps_sph_params& sp, const Grid& g, const Win& win, float4* force, float4* xsph,
+                             bool fused, const float4* vel_s, const uint32_t* idx, const GravitySources& gsrc,
+                             int collision, const rtps_float4& bmin, const rtps_float4& bmax, float dt, float4* pos_u,
+                             float4* vel_u, float4* veleval_u, const float4* color_s, float4* color_u,
+                             hipStream_t st);
 hipError_t launch_count_pairs(int num, const int* d_num, const float4* pos_s, const uint32_t* start,
                               const uint32_t* end, const rtps_sph_params& sp, const Grid& g, const Win& win,
                               unsigned long long* out, hipStream_t st);

@@ -779,6 +779,16 @@ static inline int nbr_block(const Win& w) { return w.block > 0 && w.block <= kBl
 static inline bool nbr_split(int num, const Win& w, int most) {
     return w.split == Win::kAlways || (w.split == Win::kSmall && num <= most);
 }
+// Small launches on recorded rows go to row_tiles.hip.  Where the lines lie (us,
+// tiles here / rows there; at rest, then settled): density 18 / 7 and 19 / 9 at
+// 2,048 particles, 18 / 8 and 22 / 13 at 16,384, 21 / 10 and 23 / 15 at 32,768,
+// 22 / 16 and 25 / 24 at 50,021, 22 / 21 and 25 / 30 at 65,536; force 15 / 9 and
+// 25 / 14, 17 / 10 and 31 / 22, 20 / 18 and 32 / 34, 20 / 30 and 39 / 56.  Split
+// tiles: a rollout's forward step takes 35.5 us at 2,048 particles, 32.8 with the
+// one and 32.9 with the other there, 41.9, 40.2 and 43.7 at 32,768, 44.2, 45.2
+// and 51.6 at 49,152.
+constexpr int kRowsMaxDensity = 5 << 13, kRowsMaxForce = 3 << 13;
+static inline bool by_rows(int num, const Win& w, int most) { return w.rows && !w.tq && num <= most; }
 static inline int nbr_variant(const Win& w) {
     const int v = w.variant >= 0 ? w.variant : g_force_variant;
     return v == kLoopStaged || v == kLoopStagedBits ? v : kLoopDirect;
@@ -874,6 +884,8 @@ hipError_t launch_density(int num, const int* d_num, const float4* pos_s, const 
     const bool stage = g_density_stage != 0;
     const size_t lds = stage ? (size_t)(bs / 64) * kStageCap * sizeof(float4) : 0;
     if (win_in.rows && win_in.rows_stride < (uint32_t)num) return hipErrorInvalidValue;
+    if (by_rows(num, win_in, kRowsMaxDensity) && packed && stage)
+        return launch_density_rows(num, d_num, pos_s, start, end, sp, g, win_in, packed, st);
     Win win = win_in;
     win.ntiles = nb;
 #define RTPS_DENS(S, P, T, E)                                                                                       \
@@ -924,6 +936,9 @@ hipError_t launch_force(int num, int* d_num, const float4* pos_s, const float* d
     const size_t lds = force_lds(loop, bs);
     GravitySources none{};
     rtps_float4 z{0, 0, 0, 0};
+    if (loop == kLoopShared && packed && by_rows(num, win_in, kRowsMaxForce))
+        return launch_force_rows(num, d_num, pos_s, ve, start, sp, g, win_in, force, xsph, false, nullptr, nullptr,
+                                 none, 0, z, z, 0.f, nullptr, nullptr, nullptr, nullptr, nullptr, st);
     Win win = win_in;
     win.ntiles = nb;
 #define RTPS_FORCE_Q(S, P, L, Q, SP, GRID)                                                                          \
@@ -967,6 +982,10 @@ hipError_t launch_force_fused(int num, int* d_num, const float4* pos_s, const fl
     const int loop = force_loop(win_in);
     if (win_in.rows && win_in.rows_stride < (uint32_t)num) return hipErrorInvalidValue;
     const size_t lds = force_lds(loop, bs);
+    if (loop == kLoopShared && by_rows(num, win_in, kRowsMaxForce))
+        return launch_force_rows(num, d_num, pos_s, ve_packed, start, sp, g, win_in, force, xsph, true, vel_s, idx,
+                                 gsrc, collision, gps.bnd_min, gps.bnd_max, dt, pos_u, vel_u, veleval_u, color_s,
+                                 color_u, st);
     Win win = win_in;
     win.ntiles = nb;
 #define RTPS_FFUSED_Q(S, L, Q, SP, GRID)                                                                            \
