@@ -62,6 +62,10 @@ struct rtps_batch {
     int opt_graph = 1, opt_timers = 0;
     hipGraphExec_t gexec = nullptr;
     bool graph_valid = false;
+    // kChainSteps steps in one graph, while the one-step graph it repeats is
+    // valid (as rtps_sph's: no idle time between them)
+    hipGraphExec_t gexec_chain = nullptr;
+    bool chain_valid = false, chain_failed = false;
     hipEvent_t ev[B_N + 1] = {};
     double stage_ms[B_N] = {};
     long stage_cnt[B_N] = {};
@@ -69,6 +73,7 @@ struct rtps_batch {
     ~rtps_batch() {
         if (stream) (void)hipStreamSynchronize(stream);
         if (gexec) (void)hipGraphExecDestroy(gexec);
+        if (gexec_chain) (void)hipGraphExecDestroy(gexec_chain);
         void* bufs[] = {scenes, d_num, sid, pos_u, vel_u, veleval_u, pos_s, vel_s, ve_s, keys, idx,
                         start, end, items, items128, items64, queues, sort_tmp, sub, rows};
         for (void* b : bufs)
@@ -316,16 +321,17 @@ int autotune_step_b(rtps_batch* b, bool measure) {
     return RTPS_OK;
 }
 
-int capture(rtps_batch* b) {
-    if (b->gexec) {
-        (void)hipGraphExecDestroy(b->gexec);
-        b->gexec = nullptr;
+int capture(rtps_batch* b, int steps, hipGraphExec_t* out) {
+    if (*out) {
+        (void)hipGraphExecDestroy(*out);
+        *out = nullptr;
     }
     hipGraph_t graph = nullptr;
     RTPS_TRY_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     const int timers = b->opt_timers;
     b->opt_timers = 0;
-    int rc = launch_step(b);
+    int rc = RTPS_OK;
+    for (int k = 0; k < steps && !rc; ++k) rc = launch_step(b);
     b->opt_timers = timers;
     hipError_t e = hipStreamEndCapture(b->stream, &graph);
     if (rc) {
@@ -333,12 +339,13 @@ int capture(rtps_batch* b) {
         return rc;
     }
     if (e != hipSuccess) return hip_error(e, "hipStreamEndCapture");
-    e = hipGraphInstantiate(&b->gexec, graph, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(out, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     if (e != hipSuccess) return hip_error(e, "hipGraphInstantiate");
-    b->graph_valid = true;
     return RTPS_OK;
 }
+
+constexpr int kChainSteps = 4;
 
 }  // namespace
 
@@ -578,11 +585,22 @@ int rtps_batch_step(rtps_batch* b, int nsteps) {
         return RTPS_OK;
     }
     if (b->opt_graph) {
-        if (!b->graph_valid) {
-            int rc = capture(b);
+        const bool kept = b->graph_valid;
+        if (!kept) {
+            b->chain_valid = false;
+            int rc = capture(b, 1, &b->gexec);
             if (rc) return rc;
+            b->graph_valid = true;
         }
-        for (int k = 0; k < nsteps; ++k) RTPS_TRY_HIP(hipGraphLaunch(b->gexec, b->stream));
+        int k = 0;
+        if (b->chain_valid)
+            for (; k + kChainSteps <= nsteps; k += kChainSteps) RTPS_TRY_HIP(hipGraphLaunch(b->gexec_chain, b->stream));
+        for (; k < nsteps; ++k) RTPS_TRY_HIP(hipGraphLaunch(b->gexec, b->stream));
+        // the chain is captured by a later call than the step's graph, its own steps under way
+        if (kept && !b->chain_valid && !b->chain_failed && nsteps >= kChainSteps) {
+            b->chain_valid = capture(b, kChainSteps, &b->gexec_chain) == RTPS_OK;
+            b->chain_failed = !b->chain_valid;
+        }
         return RTPS_OK;
     }
     for (int k = 0; k < nsteps; ++k) {
