@@ -120,8 +120,8 @@ int forward_step(rtps_adj* a, const State& in, const State& out, Record& r, bool
     const int n = a->N;
     const uint32_t* keys = a->keys;
     if (cell_sort_fits(n, a->nb_cells)) {
-        RTPS_TRY_HIP(cell_sort_place(n, n, nullptr, in.pos, a->g, a->keys, r.idx, a->start, a->end, a->sort_tmp, st));
-        RTPS_TRY_HIP(cell_sort_finish(n, n, nullptr, a->pad_key, a->nb_cells, a->start, a->end, a->sub, a->keys, r.idx,
+        RTPS_TRY_HIP(cell_sort_place(n, n, nullptr, in.pos, a->g, a->pad_key, a->keys, r.idx, a->start, a->end, a->sort_tmp, st));
+        RTPS_TRY_HIP(cell_sort_finish(n, n, nullptr, a->pad_key, a->g, a->start, a->end, a->sub, a->keys, r.idx,
                                       in.pos, in.vel, in.ve, r.pos_s, r.vel_s, r.ve_s, a->sort_tmp, st, nullptr,
                                       nullptr, a->left_grid));
     } else {

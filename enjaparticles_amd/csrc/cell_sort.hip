@@ -4,6 +4,8 @@
 // the grid's cells.  The order is the stable sort's: keys (cell << 4 | x
 // sixteenth) ascending, equal keys by particle index.
 //
+// Up to 4,096 particles k_cell_sort_one makes the order, above these three do:
+//
 //   k_cell_count    the key of every particle (hash_key) and its arrival rank
 //                   in its cell: one atomic on the cell's counter.
 //   k_cell_scan     counters to cell starts and ends (the start/end tables of
@@ -265,6 +267,105 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_finish(int n, int num_host,
         write_sub_starts(sub + (size_t)cell * kSubCells, kv.x & (kSubCells - 1), before, prev_xq, to, b);
 }
 
+// The order in one block, for small launches: the counters (16 bits each, two to
+// a word) and the order inside the cells in LDS, the particles' keys and ranks in
+// registers; launch_cells_permute does the rest.  Up to some thousand particles
+// the count, the scan and the placing each do little but start and wait for
+// memory; one CU alone takes 4 to 8 us for them.  A step takes (us, one block /
+// three launches; settled pools) 23 / 27 with 100 particles, 34 / 38 with 1,000,
+// 41 / 45 with 2,048, 46 / 48 with 4,096, 55 / 53 with 6,000, 61 / 55 with 8,192.
+constexpr int kOneThreads = 1024, kOnePer = kCellSortOneMax / kOneThreads;
+constexpr size_t kOneLds = 63 << 10;   // dynamic; the waves' sums come on top
+static size_t one_lds(int n, int nb_cells) {   // counters of nb_cells + 1 cells and the end, then the orders
+    return (((size_t)nb_cells + 3) / 2 + (size_t)n) * 4;
+}
+static bool one_block(int n, int nb_cells) { return n <= kCellSortOneMax && one_lds(n, nb_cells) <= kOneLds; }
+
+__global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_host, const int* __restrict__ d_num,
+                                                               const float4* __restrict__ pu, Grid g,
+                                                               uint32_t pad_key, uint32_t* __restrict__ start,
+                                                               uint32_t* __restrict__ keys,
+                                                               uint32_t* __restrict__ idx) {
+    extern __shared__ uint32_t lds[];
+    __shared__ uint32_t wsum[kOneThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int nc = g.nb_cells + 1, words = (nc + 2) / 2;   // the last entry: the end of the last cell
+    uint32_t* order = lds + words;
+    const int num = min(d_num ? *d_num : num_host, n);
+    auto at = [&](uint32_t c) { return (lds[c >> 1] >> (16u * (c & 1u))) & 0xFFFFu; };
+    for (int q = tid; q < words; q += kOneThreads) lds[q] = 0u;
+    uint32_t key[kOnePer], rank[kOnePer];
+    float3 p[kOnePer];
+#pragma unroll
+    for (int k = 0; k < kOnePer; ++k) {
+        const float4 q = pu[min(tid + k * kOneThreads, max(num - 1, 0))];   // no branch: the loads are issued together
+        p[k] = make_float3(q.x, q.y, q.z);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kOnePer; ++k) {
+        const int i = tid + k * kOneThreads;
+        if (i < num) {
+            key[k] = hash_key(make_float4(p[k].x, p[k].y, p[k].z, 0.f), g, kSubBits);
+            const uint32_t c = key[k] >> kSubBits, sh = 16u * (c & 1u);
+            rank[k] = (atomicAdd(&lds[c >> 1], 1u << sh) >> sh) & 0xFFFFu;   // counts stay below 2^16: no carry
+        }
+    }
+    __syncthreads();
+    // exclusive scan of the counters in place: an odd run of words per thread (LDS banks)
+    const int per = ((words + kOneThreads - 1) / kOneThreads) | 1, w0 = min(tid * per, words), w1 = min(w0 + per, words);
+    uint32_t sum = 0;
+    for (int q = w0; q < w1; ++q) sum += (lds[q] & 0xFFFFu) + (lds[q] >> 16);
+    const uint32_t inc = wave_incl_scan(sum);
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    uint32_t run = inc - sum;
+#pragma unroll
+    for (int q = 0; q < kOneThreads / 64; ++q) run += q < w ? wsum[q] : 0u;
+    for (int q = w0; q < w1; ++q) {
+        const uint32_t v = lds[q], mid = run + (v & 0xFFFFu);
+        lds[q] = run | mid << 16;
+        run = mid + (v >> 16);
+    }
+    __syncthreads();
+    auto order_of = [](uint32_t key, int i) { return key << 28 | (uint32_t)i; };   // x sixteenth, then index
+#pragma unroll
+    for (int k = 0; k < kOnePer; ++k) {
+        const int i = tid + k * kOneThreads;
+        if (i < num) order[at(key[k] >> kSubBits) + rank[k]] = order_of(key[k], i);
+    }
+    for (int c = tid; c < nc; c += kOneThreads) start[c] = kEmpty;   // the occupied ones follow (launch_cells_permute)
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kOnePer; ++k) {
+        const int i = tid + k * kOneThreads;
+        if (i >= num) {
+            if (i < n) {   // slots past the device's count: the pad key, as the stable sort leaves them
+                keys[i] = pad_key;
+                idx[i] = (uint32_t)i;
+            }
+            continue;
+        }
+        const uint32_t cell = key[k] >> kSubBits, a = at(cell), b = at(cell + 1), mine = order_of(key[k], i);
+        uint32_t before = 0u;   // of the cell
+        uint32_t j = a;
+        for (; j + 8 <= b; j += 8) {
+            uint32_t o[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) o[u] = order[j + u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) before += o[u] < mine ? 1u : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < 7; ++u) {   // past the cell's end: not counted
+            const uint32_t o = order[min(j + u, b - 1u)];
+            before += j + u < b && o < mine ? 1u : 0u;
+        }
+        keys[a + before] = key[k];
+        idx[a + before] = (uint32_t)i;
+    }
+}
+
 // The same for the scenes of a batch: the cells of all scenes, counted
 // together, each scene's followed by one more that counts its unused slots (so
 // that every scene starts at its own slots).  Keys (scene << 24) | cell << 4 | x
@@ -382,10 +483,15 @@ hipError_t cell_sort_finish_b(int T, const uint16_t* sid, const SceneDev* scenes
 }
 
 hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* pos_u, const Grid& g,
-                           uint32_t* keys, uint32_t* idx, uint32_t* start, uint32_t* end, void* temp,
+                           uint32_t pad_key, uint32_t* keys, uint32_t* idx, uint32_t* start, uint32_t* end, void* temp,
                            hipStream_t st) {
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     if (n <= 0) return hipSuccess;
+    if (one_block(n, g.nb_cells)) {
+        k_cell_sort_one<<<1, kOneThreads, one_lds(n, g.nb_cells), st>>>(n, num_host, d_num, pos_u, g, pad_key, start,
+                                                                       keys, idx);
+        return hipGetLastError();
+    }
     CellTemp t;
     cell_layout(n, g.nb_cells, &t, (char*)temp);
     k_cell_count<<<cs_blocks(std::max(n, kScanBlocks)), kCsThreads, 0, st>>>(num_host, d_num, pos_u, g, keys, idx,
@@ -395,15 +501,18 @@ hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* 
     return hipGetLastError();
 }
 
-hipError_t cell_sort_finish(int n, int num_host, const int* d_num, uint32_t pad_key, int nb_cells,
-                            const uint32_t* start, const uint32_t* end, uint32_t* sub, uint32_t* keys, uint32_t* idx,
+hipError_t cell_sort_finish(int n, int num_host, const int* d_num, uint32_t pad_key, const Grid& g,
+                            uint32_t* start, uint32_t* end, uint32_t* sub, uint32_t* keys, uint32_t* idx,
                             const float4* pu, const float4* vu, const float4* eu, float4* ps, float4* vs, float4* es,
                             void* temp, hipStream_t st, const float4* cu, float4* cs, int* left) {
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     if (n <= 0) return hipSuccess;
+    if (one_block(n, g.nb_cells))   // place has made the order
+        return launch_cells_permute(num_host, d_num, keys, g.nb_cells, start, end, kSubBits, sub, idx, pu, vu, eu, ps,
+                                    vs, es, st, cu, cs, left);
     CellTemp t;
-    cell_layout(n, nb_cells, &t, (char*)temp);
-    k_cell_finish<<<cs_blocks(n), kCsThreads, 0, st>>>(n, num_host, d_num, pad_key, t.pairs, nb_cells, start, end, sub,
+    cell_layout(n, g.nb_cells, &t, (char*)temp);
+    k_cell_finish<<<cs_blocks(n), kCsThreads, 0, st>>>(n, num_host, d_num, pad_key, t.pairs, g.nb_cells, start, end, sub,
                                                        keys, idx, pu, vu, eu, ps, vs, es, cu, cs, left);
     return hipGetLastError();
 }

@@ -7,10 +7,10 @@
 // particles the chip has no second wave on a SIMD to cover that.  Here the nine
 // rows wait at the same time: each wave looks its row's window up (or reads its
 // record), copies the candidates to LDS, tests them and works out the first
-// kKeep terms of every particle into registers.  Then the rows take turns in
+// terms of every particle into registers.  Then the rows take turns in
 // their order, each adding its terms to the sums it takes over from the row
 // before, through LDS: the additions are those of one wave walking the rows, at
-// a few instructions per term.  Terms beyond kKeep are worked out in the turn.
+// a few instructions per term.  Terms beyond those are worked out in the turn.
 
 #include <hip/hip_runtime.h>
 
@@ -23,8 +23,11 @@ namespace {
 
 constexpr int kRowWaves = 9, kRowBlock = 64 * kRowWaves;
 constexpr int kRowCap = 192;        // candidates per LDS copy of a row; more are read from memory
-constexpr int kKeepDensity = 20;    // a row of resting particles has 14 to 20 candidates
-constexpr int kKeepForce = 8;       // and up to 7 neighbours
+constexpr int kAheadDensity = 20;    // a row of resting particles has 14 to 20 candidates
+// and up to 7 neighbours, of a settled pool's up to 14: what 168 registers hold
+// (three waves on one of the CU's SIMDs), fewer where positions are scaled or
+// there are three chains
+constexpr int keep_force(bool scaled, bool planes) { return scaled || planes ? 8 : 12; }
 constexpr int kChunk = 32;          // candidates per word of rejection bits
 
 // Turn of a wave and the chain of sums it belongs to: one chain over the nine
@@ -100,11 +103,11 @@ __global__ __launch_bounds__(kRowBlock) void k_density_rows(int num_host, const 
         if (SCALED) { pj.x *= scale; pj.y *= scale; pj.z *= scale; }
         return h2_minus_r2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z, h2);
     };
-    float t[kKeepDensity];
+    float t[kAheadDensity];
     uint32_t rej = 0u;
     auto tests = [&](auto&& at) {   // at(k): candidate k of the window
 #pragma unroll
-        for (int k0 = 0; k0 < kKeepDensity; k0 += 4) {
+        for (int k0 = 0; k0 < kAheadDensity; k0 += 4) {
             if ((uint32_t)k0 < nmax) {
                 float4 p[4];
 #pragma unroll
@@ -118,11 +121,11 @@ __global__ __launch_bounds__(kRowBlock) void k_density_rows(int num_host, const 
                 }
             }
         }
-        for (uint32_t k = kKeepDensity; k < n; ++k) rej = rej_bit(rej, u_of(at(k)));
+        for (uint32_t k = kAheadDensity; k < n; ++k) rej = rej_bit(rej, u_of(at(k)));
     };
     float sum = 0.0f;
     auto rest = [&](auto&& at) {
-        for (uint32_t k = kKeepDensity; k < n; ++k) {
+        for (uint32_t k = kAheadDensity; k < n; ++k) {
             const float v = fmaxf(u_of(at(k)), 0.0f);
             sum = fmaf(v * v, v, sum);
         }
@@ -137,12 +140,12 @@ __global__ __launch_bounds__(kRowBlock) void k_density_rows(int num_host, const 
             sum = s ? chain[T::chain(w)][lane] : 0.0f;
             if (B > A) {
 #pragma unroll
-                for (int k0 = 0; k0 < kKeepDensity; k0 += 4)
+                for (int k0 = 0; k0 < kAheadDensity; k0 += 4)
                     if ((uint32_t)k0 < nmax) {
 #pragma unroll
                         for (int k = k0; k < k0 + 4; ++k) sum = fmaf(t[k] * t[k], t[k], sum);
                     }
-                if (nmax > (uint32_t)kKeepDensity) {
+                if (nmax > (uint32_t)kAheadDensity) {
                     if (staged) rest([&](uint32_t k) { return lds[k]; });
                     else rest([&](uint32_t k) { return mem[k]; });
                 }
@@ -236,6 +239,7 @@ __global__ __launch_bounds__(kRowBlock) void k_force_rows(int num_host, int* d_n
                                                           const float4* __restrict__ color_s,
                                                           float4* __restrict__ color_u) {
     using T = Turn<PLANES>;
+    constexpr int kKeep = keep_force(SCALED, PLANES);
     __shared__ float4 stage[kRowWaves][2 * kRowCap];   // positions (1 / density in w), then veleval|density
     __shared__ float chain[T::kChains][9][64];
     const int lane = (int)threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -303,28 +307,34 @@ __global__ __launch_bounds__(kRowBlock) void k_force_rows(int num_host, int* d_n
                                 inv_w ? pq.w : fast_rcp(vj.w));
     };
     const uint32_t n0 = a < b ? ((b - a - 1u) & (uint32_t)(kChunk - 1)) + 1u : 0u;
-    uint32_t m = 0u, kept = 0u;   // the first chunk's accepted candidates not yet worked out
-    PairTerms keep[kKeepForce];
-    // All of a wave's first kKeepForce pairs at once, without branches: their
+    uint32_t m = 0u, kept = 0u, kmax = 0u;   // the first chunk's accepted candidates not yet worked out
+    PairTerms keep[kKeep];
+    // A wave's first kKeep pairs four at a time, without branches: their
     // reads are issued together and their arithmetic overlaps.
     auto work = [&](auto&& pos, auto&& vel, bool inv_w, uint32_t idle) {   // idle: a particle to read in place of none
         if (n0) m = accepted(a, n0, pos);
-        kept = min((uint32_t)__builtin_popcount(m), (uint32_t)kKeepForce);
-        float4 p[kKeepForce], e[kKeepForce];
+        kept = min((uint32_t)__builtin_popcount(m), (uint32_t)kKeep);
+        kmax = __ockl_wfred_max_u32(kept);
 #pragma unroll
-        for (int k = 0; k < kKeepForce; ++k) {
-            const uint32_t j = m != 0u ? a + (uint32_t)__builtin_ctz(m) : idle;
-            p[k] = pos(j);
-            e[k] = vel(j);
-            m &= m - 1u;
-        }
+        for (int k0 = 0; k0 < kKeep; k0 += 4) {
+            if ((uint32_t)k0 >= kmax) break;
+            float4 p[4], e[4];
 #pragma unroll
-        for (int k = 0; k < kKeepForce; ++k) {
-            const PairTerms q = terms(p[k], e[k], inv_w);
-            const bool in = (uint32_t)k < kept;   // idle slots add nothing, whatever the row's first particle holds
-            keep[k].rx = in ? q.rx : 0.f; keep[k].ry = in ? q.ry : 0.f; keep[k].rz = in ? q.rz : 0.f;
-            keep[k].dvx = in ? q.dvx : 0.f; keep[k].dvy = in ? q.dvy : 0.f; keep[k].dvz = in ? q.dvz : 0.f;
-            keep[k].kern = in ? q.kern : 0.f; keep[k].lv = in ? q.lv : 0.f; keep[k].w6 = in ? q.w6 : 0.f;
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t j = m != 0u ? a + (uint32_t)__builtin_ctz(m) : idle;
+                p[k] = pos(j);
+                e[k] = vel(j);
+                m &= m - 1u;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const PairTerms q = terms(p[k], e[k], inv_w);
+                const bool in = (uint32_t)(k0 + k) < kept;   // idle slots add nothing, whatever was read
+                PairTerms& t = keep[k0 + k];
+                t.rx = in ? q.rx : 0.f; t.ry = in ? q.ry : 0.f; t.rz = in ? q.rz : 0.f;
+                t.dvx = in ? q.dvx : 0.f; t.dvy = in ? q.dvy : 0.f; t.dvz = in ? q.dvz : 0.f;
+                t.kern = in ? q.kern : 0.f; t.lv = in ? q.lv : 0.f; t.w6 = in ? q.w6 : 0.f;
+            }
         }
     };
     ForceAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -348,14 +358,13 @@ __global__ __launch_bounds__(kRowBlock) void k_force_rows(int num_host, int* d_n
         if (staged) work(ldsp, ldsv, true, 0u - base);
         else work(memp, memv, false, A);
     }
-    const uint32_t kmax = __ockl_wfred_max_u32(kept);
     const bool more = __ballot(m != 0u || (a < b && b - a > (uint32_t)kChunk)) != 0ull;
     for (int s = 0; s < T::kTurns; ++s) {
         if (T::turn(w) == s) {
             if (s) acc = load_acc(chain[T::chain(w)], lane);
             if (B > A) {
 #pragma unroll
-                for (int k = 0; k < kKeepForce; ++k)
+                for (int k = 0; k < kKeep; ++k)
                     if ((uint32_t)k < kmax) add_pair(acc, keep[k]);
                 if (more) {
                     if (staged) rest(ldsp, ldsv, true);

@@ -210,7 +210,8 @@ hipError_t sort_segments(int batch, int length, int dir, uint32_t* dkeys, uint32
                          const uint32_t* svals, void* temp, hipStream_t st);
 
 // ---- counting sort of the step's particles by cell (cell_sort.hip) ----
-constexpr int kCellSortMax = 5 << 16;   // particles
+constexpr int kCellSortMax = 5 << 16;      // particles
+constexpr int kCellSortOneMax = 1 << 12;   // particles that one block sorts
 // True when cell_sort_place takes n particles on a grid of nb_cells cells.
 bool cell_sort_fits(int n, int nb_cells);
 size_t cell_sort_temp_bytes(int n, int nb_cells);   // for every count up to n
@@ -219,10 +220,10 @@ hipError_t cell_sort_clear_temp(void* temp, int nb_cells, hipStream_t st);   // 
 // are written); then that order (keys, idx: hash_sort_pairs's result), the
 // sub-cell table (may be null) and the permute, as launch_cells_permute.
 hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* pos_u, const Grid& g,
-                           uint32_t* keys, uint32_t* idx, uint32_t* start, uint32_t* end, void* temp,
+                           uint32_t pad_key, uint32_t* keys, uint32_t* idx, uint32_t* start, uint32_t* end, void* temp,
                            hipStream_t st);
-hipError_t cell_sort_finish(int n, int num_host, const int* d_num, uint32_t pad_key, int nb_cells,
-                            const uint32_t* start, const uint32_t* end, uint32_t* sub, uint32_t* keys, uint32_t* idx,
+hipError_t cell_sort_finish(int n, int num_host, const int* d_num, uint32_t pad_key, const Grid& g,
+                            uint32_t* start, uint32_t* end, uint32_t* sub, uint32_t* keys, uint32_t* idx,
                             const float4* pu, const float4* vu, const float4* eu, float4* ps, float4* vs, float4* es,
                             void* temp, hipStream_t st, const float4* cu = nullptr, float4* cs = nullptr,
                             int* left = nullptr);

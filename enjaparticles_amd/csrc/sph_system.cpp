@@ -222,7 +222,7 @@ int launch_front(rtps_sph* s, StageTimer& t) {
     t.mark(ST_SORT);
     const bool by_cell = s->opt_bucket && cell_sort_fits(n, s->nb_cells);
     if (by_cell) {
-        RTPS_TRY_HIP(cell_sort_place(n, n, s->d_num, s->pos_u, s->g, s->keys, s->idx, s->start, s->end, s->cell_tmp,
+        RTPS_TRY_HIP(cell_sort_place(n, n, s->d_num, s->pos_u, s->g, s->pad_key, s->keys, s->idx, s->start, s->end, s->cell_tmp,
                                      s->stream));
         s->keys_sorted = s->keys;
         s->idx_sorted = s->idx;
@@ -241,7 +241,7 @@ int launch_front(rtps_sph* s, StageTimer& t) {
     // "permute" stage is empty
     t.mark(ST_CELL);
     if (by_cell)
-        RTPS_TRY_HIP(cell_sort_finish(n, n, s->d_num, s->pad_key, s->nb_cells, s->start, s->end, sub_table_to_write(s),
+        RTPS_TRY_HIP(cell_sort_finish(n, n, s->d_num, s->pad_key, s->g, s->start, s->end, sub_table_to_write(s),
                                       s->keys, s->idx, s->pos_u, s->vel_u, s->veleval_u, s->pos_s, s->vel_s, s->ve_s,
                                       s->cell_tmp, s->stream, col_u(s), col_s(s)));
     else
