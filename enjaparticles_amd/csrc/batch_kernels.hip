@@ -402,7 +402,8 @@ __device__ __forceinline__ void pairs_one(int i, int s, const SceneDev& S, bool 
 template <int MODE, int BLOCK, int WAVES, bool ROWS>
 __global__ __launch_bounds__(BLOCK, WAVES) void k_pairs_b(const BatchItem* __restrict__ items, int n_items,
                                                      int* __restrict__ queue, const SceneDev* __restrict__ scenes,
-                                                     const int* __restrict__ d_num, const float4* __restrict__ pos_s,
+                                                     int* d_num, int* __restrict__ num_seen,
+                                                     const float4* __restrict__ pos_s,
                                                      const uint32_t* __restrict__ start,
                                                      const uint32_t* __restrict__ end,
                                                      const uint32_t* __restrict__ keys, float4* __restrict__ ve,
@@ -422,6 +423,14 @@ __global__ __launch_bounds__(BLOCK, WAVES) void k_pairs_b(const BatchItem* __res
         const SceneDev& S = scenes[s];
         int num;
         const bool deleted = scene_num(S, d_num[s], start, num);
+        // The scene's count after the step, for the next one and in host memory
+        // (a read of it costs the wait for the step, not a transfer of 20 us).
+        // Blocks that read d_num after this store get the same count: that of
+        // the committed one is itself.
+        if (MODE == kPairsForceStep && I.first == S.off && threadIdx.x == 0) {
+            d_num[s] = num;
+            num_seen[s] = num;
+        }
         const int i = I.first + (int)threadIdx.x;
         if ((int)threadIdx.x < I.count && i - S.off < num)
             pairs_one<MODE, ROWS>(i, s, S, deleted, pos_s, start, end, keys, ve, vel_s, idx, pos_u, vel_u, veleval_u,
@@ -495,17 +504,6 @@ __global__ __launch_bounds__(192, 5) void k_pairs_split_b(const BatchItem* __res
     }
 }
 
-// The scenes' counts after the step, on the device and in host memory (a read
-// of a count then costs the wait for the step, not a transfer of 20 us).
-__global__ void k_commit_b(int S, const SceneDev* __restrict__ scenes, int* __restrict__ d_num,
-                           int* __restrict__ num_seen, const uint32_t* __restrict__ start) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= S) return;
-    int num;
-    if (scene_num(scenes[s], d_num[s], start, num)) d_num[s] = num;
-    num_seen[s] = num;
-}
-
 hipError_t launch_hash_b(int T, const uint16_t* sid, const SceneDev* scenes, const int* d_num, const float4* pos_u,
                          uint32_t* keys, uint32_t* idx, uint32_t* start, int n_cells, hipStream_t st) {
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
@@ -532,10 +530,10 @@ bool pairs_cfg_valid(int mode, const PairsCfg& c) {
 PairsCfg pairs_default_cfg(int mode) { return mode == kPairsDensity ? PairsCfg{256, 5} : PairsCfg{256, 4}; }
 
 hipError_t launch_pairs_b(int mode, const PairsCfg& cfg, int grid, const BatchItem* items, int n_items, int* queue,
-                          const SceneDev* scenes, const int* d_num, const float4* pos_s, const uint32_t* start,
-                          const uint32_t* end, const uint32_t* keys, float4* ve, const float4* vel_s,
-                          const uint32_t* idx, float4* pos_u, float4* vel_u, float4* veleval_u, hipStream_t st,
-                          const uint32_t* sub, uint32_t* rows, uint32_t rows_stride) {
+                          const SceneDev* scenes, int* d_num, int* num_seen, const float4* pos_s,
+                          const uint32_t* start, const uint32_t* end, const uint32_t* keys, float4* ve,
+                          const float4* vel_s, const uint32_t* idx, float4* pos_u, float4* vel_u, float4* veleval_u,
+                          hipStream_t st, const uint32_t* sub, uint32_t* rows, uint32_t rows_stride) {
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     if (rows && rows_stride == 0) return hipErrorInvalidValue;
     if (!pairs_cfg_valid(mode, cfg)) return hipErrorInvalidValue;
@@ -544,12 +542,12 @@ hipError_t launch_pairs_b(int mode, const PairsCfg& cfg, int grid, const BatchIt
     auto go = [&](auto m, auto b, auto w) {
         constexpr int M = decltype(m)::value, BL = decltype(b)::value, W = decltype(w)::value;
         if (rows)
-            k_pairs_b<M, BL, W, true><<<grid, BL, 0, st>>>(items, n_items, queue, scenes, d_num, pos_s, start, end,
-                                                           keys, ve, vel_s, idx, pos_u, vel_u, veleval_u, sub, rows,
+            k_pairs_b<M, BL, W, true><<<grid, BL, 0, st>>>(items, n_items, queue, scenes, d_num, num_seen, pos_s, start,
+                                                           end, keys, ve, vel_s, idx, pos_u, vel_u, veleval_u, sub, rows,
                                                            rows_stride);
         else
-            k_pairs_b<M, BL, W, false><<<grid, BL, 0, st>>>(items, n_items, queue, scenes, d_num, pos_s, start, end,
-                                                            keys, ve, vel_s, idx, pos_u, vel_u, veleval_u, sub,
+            k_pairs_b<M, BL, W, false><<<grid, BL, 0, st>>>(items, n_items, queue, scenes, d_num, num_seen, pos_s, start,
+                                                            end, keys, ve, vel_s, idx, pos_u, vel_u, veleval_u, sub,
                                                             nullptr, 0u);
     };
     auto by_waves = [&](auto m, auto b) {
@@ -592,13 +590,6 @@ hipError_t launch_pairs_split_b(int mode, int n_items64, const BatchItem* items6
     if (mode == kPairsDensity) go(std::integral_constant<int, kPairsDensity>{});
     else if (mode == kPairsForceStep) go(std::integral_constant<int, kPairsForceStep>{});
     else return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-
-hipError_t launch_commit_b(int S, const SceneDev* scenes, int* d_num, int* num_seen, const uint32_t* start,
-                           hipStream_t st) {
-    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    k_commit_b<<<(S + 63) / 64, 64, 0, st>>>(S, scenes, d_num, num_seen, start);
     return hipGetLastError();
 }
 

@@ -35,7 +35,7 @@ struct rtps_batch {
     hipStream_t stream = nullptr;
     SceneDev* scenes = nullptr;
     int* d_num = nullptr;
-    int* num_seen = nullptr;   // d_num in pinned host memory, as of the last finished step (commit writes both)
+    int* num_seen = nullptr;   // d_num in pinned host memory, as of the last finished step (the force step writes both)
     uint16_t* sid = nullptr;
     float4 *pos_u = nullptr, *vel_u = nullptr, *veleval_u = nullptr, *pos_s = nullptr, *vel_s = nullptr,
            *ve_s = nullptr;
@@ -120,7 +120,7 @@ uint32_t* rows_of(const rtps_batch* b) { return b->opt_rows ? b->rows : nullptr;
 
 int launch_density_b(rtps_batch* b, const PairsCfg& c) {
     RTPS_TRY_HIP(launch_pairs_b(kPairsDensity, c, grid_of(b, c), items_of(b, c), nitems_of(b, c), b->queues,
-                                b->scenes, b->d_num, b->pos_s, b->start, b->end, b->keys_sorted, b->ve_s, b->vel_s,
+                                b->scenes, b->d_num, b->num_seen, b->pos_s, b->start, b->end, b->keys_sorted, b->ve_s, b->vel_s,
                                 b->idx_sorted, b->pos_u, b->vel_u, b->veleval_u, b->stream, b->sub,
                                 rows_of(b), (uint32_t)b->T));
     return RTPS_OK;
@@ -128,7 +128,7 @@ int launch_density_b(rtps_batch* b, const PairsCfg& c) {
 
 int launch_force_b(rtps_batch* b, const PairsCfg& c) {
     RTPS_TRY_HIP(launch_pairs_b(kPairsForceStep, c, grid_of(b, c), items_of(b, c), nitems_of(b, c),
-                                b->queues, b->scenes, b->d_num, b->pos_s, b->start, b->end,
+                                b->queues, b->scenes, b->d_num, b->num_seen, b->pos_s, b->start, b->end,
                                 b->keys_sorted, b->ve_s, b->vel_s, b->idx_sorted, b->pos_u, b->vel_u, b->veleval_u,
                                 b->stream, b->sub, rows_of(b), (uint32_t)b->T));
     return RTPS_OK;
@@ -170,7 +170,6 @@ int launch_step(rtps_batch* b) {
     mark(b, B_FORCE);
     rc = launch_force_b(b, b->cfg_force);
     if (rc) return rc;
-    RTPS_TRY_HIP(launch_commit_b(b->S, b->scenes, b->d_num, b->num_seen, b->start, b->stream));
     mark(b, B_N);
     return RTPS_OK;
 }
@@ -314,10 +313,9 @@ int autotune_step_b(rtps_batch* b, bool measure) {
     b->tuned = true;
     b->graph_valid = false;
     btune_put(key, best[0], best[1]);
-    // finish the step: the force step with the chosen configuration, then the count commit
+    // finish the step: the force step with the chosen configuration, which commits the counts
     rc = launch_force_b(b, b->cfg_force);
     if (rc) return rc;
-    RTPS_TRY_HIP(launch_commit_b(b->S, b->scenes, b->d_num, b->num_seen, b->start, b->stream));
     return RTPS_OK;
 }
 

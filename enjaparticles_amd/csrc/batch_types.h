@@ -68,10 +68,12 @@ struct PairsCfg {
 int pairs_blocks_per_cu(const PairsCfg& c);
 bool pairs_cfg_valid(int mode, const PairsCfg& c);
 PairsCfg pairs_default_cfg(int mode);
+// The force step also commits the scenes' counts to d_num and num_seen (pinned host memory).
 hipError_t launch_pairs_b(int mode, const PairsCfg& cfg, int grid, const BatchItem* items, int n_items, int* queue,
-                          const SceneDev* scenes, const int* d_num, const float4* pos_s, const uint32_t* start,
-                          const uint32_t* end, const uint32_t* keys, float4* ve, const float4* vel_s,
-                          const uint32_t* idx, float4* pos_u, float4* vel_u, float4* veleval_u, hipStream_t st,
+                          const SceneDev* scenes, int* d_num, int* num_seen, const float4* pos_s,
+                          const uint32_t* start, const uint32_t* end, const uint32_t* keys, float4* ve,
+                          const float4* vel_s, const uint32_t* idx, float4* pos_u, float4* vel_u, float4* veleval_u,
+                          hipStream_t st,
                           const uint32_t* sub = nullptr, uint32_t* rows = nullptr, uint32_t rows_stride = 0);
 // The same step with one block per 64-slot item, split over three waves
 // (recorded steps: every slot holds a particle, no deletion; rows required).
@@ -82,7 +84,5 @@ hipError_t launch_pairs_split_b(int mode, int n_items64, const BatchItem* items6
                                 const uint32_t* keys, float4* ve, const float4* vel_s, const uint32_t* idx,
                                 float4* pos_u, float4* vel_u, float4* veleval_u, float4* force_out, int* left,
                                 const uint32_t* sub, uint32_t* rows, uint32_t rows_stride, hipStream_t st);
-hipError_t launch_commit_b(int S, const SceneDev* scenes, int* d_num, int* num_seen, const uint32_t* start,
-                           hipStream_t st);
 
 }  // namespace rtps
