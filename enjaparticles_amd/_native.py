@@ -81,6 +81,7 @@ SIGNATURES = {
     "rtps_mc_geometry": (_i, [P, P]),
     "rtps_batch_autotune": (_i, [P, _i, P, P, P, P]),
     "rtps_cellindices": (_i, [_i, P, _i, P, P, P, P]),
+    "rtps_max_i32": (_i, [_i, P, P, P]),
     "rtps_permute": (_i, [_i, P, P, P, P, P, P, P, P]),
     "rtps_density": (_i, [_i, P, P, P, P, P, P, P]),
     "rtps_force": (_i, [_i, P, P, P, P, P, P, P, P, P, P]),

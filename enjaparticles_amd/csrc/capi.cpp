@@ -3,6 +3,7 @@
 // given stream and reports failures through a status code plus
 // rtps_last_error(); no exception leaves this file.
 
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -107,6 +108,29 @@ int rtps_cellindices(int num, const uint32_t* keys, int nb_cells, uint32_t* star
     RTPS_HIP(launch_fill_u32(start, kEmpty, (long)nb_cells + 1, S(stream)));
     RTPS_HIP(launch_cellindices(num, nullptr, keys, nb_cells, start, end, 0, S(stream)));
     if (nc) RTPS_HIP(launch_read_nc(start, nb_cells, nc, S(stream)));
+    return RTPS_OK;
+}
+
+int rtps_max_i32(int n, const int32_t* v, int32_t* max, void* stream) {
+    RTPS_CHECK(n >= 0 && max, "rtps_max_i32: bad arguments");
+    *max = INT32_MIN;
+    if (n == 0) return RTPS_OK;
+    RTPS_CHECK(v, "rtps_max_i32: null buffer");
+    // The kernel's blocks leave their maxima in pinned host memory, one page per
+    // calling thread (it waits below, so it is the only user), given back with it.
+    struct Page {
+        int32_t* p = nullptr;
+        ~Page() {
+            if (p) (void)hipHostFree(p);
+        }
+    };
+    static thread_local Page page;
+    if (!page.p)
+        RTPS_HIP(hipHostMalloc((void**)&page.p, kMaxBlocks * sizeof(int32_t), hipHostMallocPortable));
+    int blocks = 0;
+    RTPS_HIP(launch_max_i32(n, v, page.p, &blocks, S(stream)));
+    RTPS_HIP(hipStreamSynchronize(S(stream)));
+    for (int b = 0; b < blocks; ++b) *max = std::max(*max, page.p[b]);
     return RTPS_OK;
 }
 

@@ -12,6 +12,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -90,6 +91,20 @@ __global__ __launch_bounds__(kBlock) void k_cellindices(int num_host, const int*
 
 __global__ void k_read_nc(const uint32_t* __restrict__ start, int nb_cells, int* __restrict__ nc) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *nc = (int)start[nb_cells];
+}
+
+// Maximum of an index array, for the host's check of it.
+__global__ __launch_bounds__(kBlock) void k_max_i32(int n, const int32_t* __restrict__ v, int32_t* __restrict__ out) {
+    __shared__ int32_t part[kBlock / 64];
+    int32_t m = INT32_MIN;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) m = max(m, v[i]);
+    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_down(m, o, 64));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) m = max(m, part[w]);
+        out[blockIdx.x] = m;
+    }
 }
 
 // a5: permute.cl:10-46 (pos, vel, veleval).
@@ -833,6 +848,13 @@ hipError_t launch_read_nc(const uint32_t* start, int nb_cells, int* nc, hipStrea
 }
 
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, long n, hipStream_t st);
+
+hipError_t launch_max_i32(int n, const int32_t* v, int32_t* out, int* blocks, hipStream_t st) {
+    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
+    *blocks = std::min(blocks_for(n), kMaxBlocks);
+    k_max_i32<<<*blocks, kBlock, 0, st>>>(n, v, out);
+    return hipGetLastError();
+}
 
 hipError_t launch_permute(int num, const int* d_num, const uint32_t* idx, const float4* pu, const float4* vu,
                           const float4* eu, float4* ps, float4* vs, float4* es, hipStream_t st, const float4* cu,

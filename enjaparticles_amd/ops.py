@@ -32,6 +32,15 @@ def _u32(t: torch.Tensor, n: int, name: str) -> None:
         raise ValueError(f"{name} must be a 32-bit integer vector of length >= {n}")
 
 
+def _max_index(idx: torch.Tensor, num: int) -> int:
+    """Largest of the first num entries, on the host."""
+    if idx.dtype == torch.int32 and idx.is_cuda and idx.dim() == 1 and idx.is_contiguous() and idx.shape[0] >= num:
+        out = C.c_int32()
+        N.check(N.lib().rtps_max_i32(num, idx.data_ptr(), C.byref(out), _stream()))
+        return out.value
+    return int(idx[:num].max().item())
+
+
 def hash(pos_u: torch.Tensor, gp: N.GridParams, num: int | None = None, n_pad: int | None = None):
     num = pos_u.shape[0] if num is None else num
     n_pad = num if n_pad is None else n_pad
@@ -87,7 +96,7 @@ def permute(idx, pos_u, vel_u, veleval_u, num: int | None = None):
         _f4(t, 1, nm)
     _u32(idx, num, "idx")
     n_u = min(pos_u.shape[0], vel_u.shape[0], veleval_u.shape[0])
-    if num and int(idx[:num].max().item()) >= n_u:
+    if num and _max_index(idx, num) >= n_u:
         raise ValueError("idx points outside the unsorted arrays")
     ps, vs, es = (torch.empty((num, 4), dtype=torch.float32, device=idx.device) for _ in range(3))
     N.check(N.lib().rtps_permute(num, _ptr(idx), _ptr(pos_u), _ptr(vel_u), _ptr(veleval_u), _ptr(ps), _ptr(vs),
@@ -159,7 +168,7 @@ def collision_triangles(pos_s, vel_s, force_s, triangles, sphp):
 def leapfrog(pos_s, vel_s, force_s, xsph_s, idx, sphp, dt, pos_u, vel_u, veleval_u):
     """Returns updated clones of (pos_u, vel_u, veleval_u)."""
     num = pos_s.shape[0]
-    if num and int(idx[:num].max().item()) >= pos_u.shape[0]:
+    if num and _max_index(idx, num) >= pos_u.shape[0]:
         raise ValueError("idx points outside the unsorted arrays")
     pu, vu, eu = pos_u.clone(), vel_u.clone(), veleval_u.clone()
     N.check(N.lib().rtps_leapfrog(num, _ptr(pos_s), _ptr(vel_s), _ptr(force_s), _ptr(xsph_s), _ptr(idx),

@@ -122,6 +122,10 @@ int rtps_sort_segments(int batch, int array_length, int dir, uint32_t* dst_keys 
 int rtps_cellindices(int num, const uint32_t* keys /*dev*/, int nb_cells, uint32_t* start /*dev*/,
                      uint32_t* end /*dev*/, int* nc /*dev, may be NULL*/, void* stream);
 
+/* The largest of n signed 32-bit integers on the device (INT32_MIN for n = 0), to
+ * check an index array before rtps_permute or rtps_leapfrog: waits for the stream. */
+int rtps_max_i32(int n, const int32_t* v, int32_t* max, void* stream);
+
 /* a5. Permute::execute (rtpslib/system/common/Permute.h:46-79, permute.cl:10-46):
  * X_s[i] = X_u[idx[i]] for position, velocity and veleval. */
 int rtps_permute(int num, const uint32_t* idx, const rtps_float4* pos_u, const rtps_float4* vel_u,
