@@ -62,10 +62,7 @@ struct rtps_batch {
     int opt_graph = 1, opt_timers = 0;
     hipGraphExec_t gexec = nullptr;
     bool graph_valid = false;
-    // kChainSteps steps in one graph, while the one-step graph it repeats is
-    // valid (as rtps_sph's: no idle time between them)
-    hipGraphExec_t gexec_chain = nullptr;
-    bool chain_valid = false, chain_failed = false;
+    StepRuns runs;   // of several steps, while that graph is valid
     hipEvent_t ev[B_N + 1] = {};
     double stage_ms[B_N] = {};
     long stage_cnt[B_N] = {};
@@ -73,7 +70,7 @@ struct rtps_batch {
     ~rtps_batch() {
         if (stream) (void)hipStreamSynchronize(stream);
         if (gexec) (void)hipGraphExecDestroy(gexec);
-        if (gexec_chain) (void)hipGraphExecDestroy(gexec_chain);
+        runs.drop();
         void* bufs[] = {scenes, d_num, sid, pos_u, vel_u, veleval_u, pos_s, vel_s, ve_s, keys, idx,
                         start, end, items, items128, items64, queues, sort_tmp, sub, rows};
         for (void* b : bufs)
@@ -343,8 +340,6 @@ int capture(rtps_batch* b, int steps, hipGraphExec_t* out) {
     return RTPS_OK;
 }
 
-constexpr int kChainSteps = 4;
-
 }  // namespace
 
 namespace rtps {
@@ -585,20 +580,14 @@ int rtps_batch_step(rtps_batch* b, int nsteps) {
     if (b->opt_graph) {
         const bool kept = b->graph_valid;
         if (!kept) {
-            b->chain_valid = false;
+            b->runs.drop();
             int rc = capture(b, 1, &b->gexec);
             if (rc) return rc;
             b->graph_valid = true;
         }
-        int k = 0;
-        if (b->chain_valid)
-            for (; k + kChainSteps <= nsteps; k += kChainSteps) RTPS_TRY_HIP(hipGraphLaunch(b->gexec_chain, b->stream));
-        for (; k < nsteps; ++k) RTPS_TRY_HIP(hipGraphLaunch(b->gexec, b->stream));
-        // the chain is captured by a later call than the step's graph, its own steps under way
-        if (kept && !b->chain_valid && !b->chain_failed && nsteps >= kChainSteps) {
-            b->chain_valid = capture(b, kChainSteps, &b->gexec_chain) == RTPS_OK;
-            b->chain_failed = !b->chain_valid;
-        }
+        RTPS_TRY_HIP(b->runs.replay(b->gexec, kept, nsteps, b->stream, [b](int steps, hipGraphExec_t* out) {
+            return capture(b, steps, out);
+        }));
         return RTPS_OK;
     }
     for (int k = 0; k < nsteps; ++k) {

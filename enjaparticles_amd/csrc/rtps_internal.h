@@ -27,6 +27,50 @@ struct Win;
 int set_error(int code, const std::string& msg);
 int hip_error(hipError_t e, const char* where);
 
+// ---- runs of steps (sph_system.cpp, batch_system.cpp) ----
+// Between two graph launches the device is idle for 8 to 10 us, a fifth of a step
+// of 2,048 particles; so runs of four and of two steps are graphs, too, next to a
+// handle's graph of one.  Each is captured by a call that could use it and finds
+// the one-step graph of an earlier call still valid (not where options change
+// from call to call), once that call's own steps are under way.
+class StepRuns {
+public:
+    StepRuns() = default;
+    StepRuns(const StepRuns&) = delete;
+    StepRuns& operator=(const StepRuns&) = delete;
+    ~StepRuns() { drop(); }
+    void drop() {   // the one-step graph has changed
+        for (hipGraphExec_t& e : run_) {
+            if (e) (void)hipGraphExecDestroy(e);
+            e = nullptr;
+        }
+        failed_ = false;
+    }
+    // nsteps steps: runs where they are there, the rest by `one`; kept: it is an
+    // earlier call's.  capture(steps, &exec) captures that many steps (RTPS_OK).
+    template <class Capture>
+    hipError_t replay(hipGraphExec_t one, bool kept, int nsteps, hipStream_t st, Capture&& capture) {
+        int left = nsteps;
+        for (int r = 0; r < 2; ++r)
+            for (; run_[r] && left >= kSteps[r]; left -= kSteps[r]) {
+                const hipError_t e = hipGraphLaunch(run_[r], st);
+                if (e != hipSuccess) return e;
+            }
+        for (; left > 0; --left) {
+            const hipError_t e = hipGraphLaunch(one, st);
+            if (e != hipSuccess) return e;
+        }
+        for (int r = 0, n = nsteps; r < 2 && kept && !failed_; n %= kSteps[r], ++r)
+            if (!run_[r] && n >= kSteps[r]) failed_ = capture(kSteps[r], &run_[r]) != 0;   // then by the others
+        return hipSuccess;
+    }
+
+private:
+    static constexpr int kSteps[2] = {4, 2};
+    hipGraphExec_t run_[2] = {};
+    bool failed_ = false;
+};
+
 // ---- parameter derivation (params.cpp) ----
 // SPH::calculate (SPHSettings.cpp:30-144) on `s` (writes the derived keys),
 // then SPH::updateParams (:149-201) and System::setupDomain (System.cpp:294-329).

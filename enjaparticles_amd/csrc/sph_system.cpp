@@ -72,8 +72,7 @@ struct rtps_sph {
     bool tuned = false;
     hipGraphExec_t gexec = nullptr;
     bool graph_valid = false;
-    hipGraphExec_t gexec_chain = nullptr;   // kChainSteps steps, while the one-step graph it repeats is valid
-    bool chain_valid = false, chain_failed = false;
+    StepRuns runs;   // of several steps, while that graph is valid
     // Timers: two event sets alternate between steps (set k & 1 for step k),
     // each recorded by its own captured step graph when graphs are on.
     hipGraphExec_t gexec_t[2] = {};
@@ -106,7 +105,7 @@ struct rtps_sph {
         for (rtps_hose* h : hoses) rtps_hose_destroy(h);
         if (stream) (void)hipStreamSynchronize(stream);
         if (gexec) (void)hipGraphExecDestroy(gexec);
-        if (gexec_chain) (void)hipGraphExecDestroy(gexec_chain);
+        runs.drop();
         for (auto& g : gexec_t)
             if (g) (void)hipGraphExecDestroy(g);
         void* bufs[] = {pos_u, vel_u, veleval_u, pos_s, vel_s, ve_s,  force_s,  xsph_s,   color_u,
@@ -349,34 +348,22 @@ int capture_step(rtps_sph* s, bool timed, int set, hipGraphExec_t* out, int step
 }
 
 int capture_graph(rtps_sph* s) {
-    s->chain_valid = false;
+    s->runs.drop();
     int rc = capture_step(s, false, 0, &s->gexec);
     if (rc) return rc;
     s->graph_valid = true;
     return RTPS_OK;
 }
 
-// nsteps steps by graphs.  Between two graphs the device is idle for 8 to 10 us,
-// a fifth of a step of 2,048 particles, so runs of kChainSteps steps are one
-// graph.  It is captured by the first call of as many steps that finds the
-// one-step graph of an earlier call still valid (not where options change from
-// call to call), once that call's own steps are under way.
-constexpr int kChainSteps = 4;
-
-int replay_steps(rtps_sph* s, int nsteps) {
+int replay_steps(rtps_sph* s, int nsteps) {   // by graphs
     const bool kept = s->graph_valid;
     if (!kept) {
         int rc = capture_graph(s);
         if (rc) return rc;
     }
-    int k = 0;
-    if (s->chain_valid)
-        for (; k + kChainSteps <= nsteps; k += kChainSteps) RTPS_TRY_HIP(hipGraphLaunch(s->gexec_chain, s->stream));
-    for (; k < nsteps; ++k) RTPS_TRY_HIP(hipGraphLaunch(s->gexec, s->stream));
-    if (kept && !s->chain_valid && !s->chain_failed && nsteps >= kChainSteps) {
-        s->chain_valid = capture_step(s, false, 0, &s->gexec_chain, kChainSteps) == RTPS_OK;
-        s->chain_failed = !s->chain_valid;   // no room for it: one graph per step as before
-    }
+    RTPS_TRY_HIP(s->runs.replay(s->gexec, kept, nsteps, s->stream, [s](int steps, hipGraphExec_t* out) {
+        return capture_step(s, false, 0, out, steps);
+    }));
     return RTPS_OK;
 }
 
