@@ -1,6 +1,6 @@
 // Batched scenes handle (rtps_batch): S independent SPH systems, each with
 // its own settings (viscosity, gas constant, box, capacity ...), stepped with
-// one launch per stage and one hipGraph per step.  No reference counterpart:
+// one launch per stage, replayed from hipGraphs.  No reference counterpart:
 // every scene computes what a single rtps_sph system with the same settings
 // and particles computes.
 

@@ -9,9 +9,9 @@
 //   start/end                                u32[nb_cells + 1]
 //   d_num                                    the particle count, on the device
 // The step never synchronises with the host: the per-step clear of start[]
-// is fused into the hash kernel, nc stays on the device and the deletion
-// path's new count is committed by a one-thread kernel, so rtps_sph_step can
-// replay one captured hipGraph per step.
+// is fused into the sort, nc stays on the device and the deletion
+// path's new count is committed by the force kernel, so rtps_sph_step can
+// replay captured hipGraphs.
 
 #include <hip/hip_runtime.h>
 

@@ -238,7 +238,7 @@ class SPH:
         return v, nn
 
     def step(self, nsteps: int = 1) -> None:
-        """nsteps x (update + integrate), fused kernels, one hipGraph replay per step."""
+        """nsteps x (update + integrate), fused kernels, replayed from hipGraphs."""
         N.check(N.lib().rtps_sph_step(self._h, int(nsteps)))
 
     def synchronize(self) -> None:
