@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kBBlock) void k_cellindices_b(int T, const uint32_t
                                                            const SceneDev* __restrict__ scenes,
                                                            uint32_t* __restrict__ start, uint32_t* __restrict__ end,
                                                            uint32_t* __restrict__ sub) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (i >= T) return;
     uint32_t g;
     if (!cell_of(keys[i], scenes, g)) return;

@@ -77,10 +77,10 @@ bool cell_sort_fits(int n, int nb_cells) { return n <= kCellSortMax && (long)nb_
 
 // Batches: the other way there is hash, four or five digit passes, cellindices
 // and permute, nine launches in all.  Measured for all of it (us, digits /
-// counting; settled scenes, then at rest): 43 / 25 and 41 / 24 at 2,574 slots,
-// 76 / 57 and 72 / 41 at 216,557, 97 / 82 and 87 / 52 at 420,738, 132 / 125 and
-// 112 / 78 at 840,154, 187 / 187 and 159 / 122 at 1,356,782, 378 / 416 and 296 /
-// 278 at 3,534,703.  The line, 2^20 slots, is where settled scenes still gain.
+// counting; settled scenes, then at rest): 43 / 27 and 41 / 25 at 2,574 slots,
+// 76 / 51 and 70 / 39 at 216,557, 110 / 105 and 110 / 76 at 840,154, 155 / 159 and
+// 159 / 125 at 1,356,782, 331 / 389 and 301 / 290 at 3,534,703.  The line, 2^20
+// slots, is where settled scenes still gain.
 bool cell_sort_fits_b(long T, long total_cells) { return T <= 1 << 20 && total_cells <= 16 * T + (1 << 20); }
 
 __global__ __launch_bounds__(kCsThreads) void k_cell_count(int num_host, const int* __restrict__ d_num,
@@ -370,6 +370,9 @@ __global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_ho
 // together, each scene's followed by one more that counts its unused slots (so
 // that every scene starts at its own slots).  Keys (scene << 24) | cell << 4 | x
 // sixteenth; unused slots keep their place and get (scene << 24) | 0xFFFFFF.
+// The blocks go over the slots in XCD order (xcd_tile): a scene's gathers and its
+// counters stay in one L2, which its pair kernels' items use as well.  finish at
+// 216,557 settled slots: 16 -> 11 us, 48 -> 26 at 840,154.
 constexpr uint32_t kPadLocal = (1u << kSceneShift) - 1u;
 
 __device__ __forceinline__ uint32_t cell_of_key(const SceneDev& S, uint32_t key) {
@@ -383,7 +386,7 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_count_b(int T, const uint16
                                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
                                                              uint32_t* __restrict__ count,
                                                              unsigned long long* __restrict__ status) {
-    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    const int i = xcd_tile(blockIdx.x, gridDim.x) * kCsThreads + threadIdx.x;
     if (i < kScanBlocks) status[i] = 0ull;
     if (i >= T) return;
     const int s = sid[i];
@@ -405,7 +408,7 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_place_b(int T, const uint16
                                                              const uint32_t* __restrict__ rank,
                                                              const uint32_t* __restrict__ start,
                                                              uint2* __restrict__ pairs) {
-    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    const int i = xcd_tile(blockIdx.x, gridDim.x) * kCsThreads + threadIdx.x;
     if (i >= T) return;
     const int s = sid[i];
     const SceneDev& S = scenes[s];
@@ -426,7 +429,7 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_finish_b(int T, const uint1
                                                               const float4* __restrict__ vu,
                                                               const float4* __restrict__ eu, float4* __restrict__ ps,
                                                               float4* __restrict__ vs, float4* __restrict__ es) {
-    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    const int i = xcd_tile(blockIdx.x, gridDim.x) * kCsThreads + threadIdx.x;
     if (i >= T) return;
     const int s = sid[i];
     const SceneDev& S = scenes[s];
