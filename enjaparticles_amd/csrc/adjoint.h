@@ -7,6 +7,13 @@
 
 namespace rtps {
 
+// Tile order (remap_tile) of the recorded steps and of B2 and B3: one contiguous
+// eighth of the particles per XCD, whose L2 then serves its tiles' rows; for larger
+// runs chunks of 16 tiles in turn, as a pool's dense bottom would make one XCD's
+// eighth the slowest (force at 150,001 settled particles: 52 us in plain order and in chunks, 66 in
+// eighths; 43 and 42 at 65,536).  A gradient over 20 steps of 65,536 particles
+// takes 2.41 ms in plain order, 2.31 in eighths.
+__host__ __device__ inline int adj_remap(int num) { return num <= 1 << 16 ? 1 : 16; }
 int adjoint_tiles(int num);   // tiles of B2 (shares of dL/dmu, dL/dK it writes)
 // A state's copy at the start of a run: pos and vel copied, veleval zero.
 hipError_t launch_adj_start(int num, const float4* pos, const float4* vel, float4* pos_out, float4* vel_out,

@@ -53,8 +53,8 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_b2(int num, const float4* _
                                                         rtps_sph_params sp, float4* __restrict__ gx2_s,
                                                         float4* __restrict__ ge_s, float* __restrict__ grho_s,
                                                         float2* __restrict__ partial) {
-    const int i = (int)blockIdx.x * 64 + ((int)threadIdx.x & 63);
-    adj_b2_tile(i, i < num, pos_s, ve_s, ga_s, gX_s, rows, sp, gx2_s, ge_s, grho_s, partial + blockIdx.x);
+    const int tile = remap_tile(adj_remap(num), blockIdx.x, gridDim.x), i = tile * 64 + ((int)threadIdx.x & 63);
+    adj_b2_tile(i, i < num, pos_s, ve_s, ga_s, gX_s, rows, sp, gx2_s, ge_s, grho_s, partial + tile);
 }
 
 __global__ __launch_bounds__(kAdjThreads) void k_adj_b3(int num, const uint32_t* __restrict__ idx,
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_b3(int num, const uint32_t*
                                                         const float4* __restrict__ ge_s, AdjRows rows,
                                                         rtps_sph_params sp, float4* __restrict__ lam_x_out,
                                                         float4* __restrict__ lam_e_out) {
-    const int i = (int)blockIdx.x * 64 + ((int)threadIdx.x & 63);
+    const int i = remap_tile(adj_remap(num), blockIdx.x, gridDim.x) * 64 + ((int)threadIdx.x & 63);
     adj_b3_tile(i, i < num, idx, pos_s, grho_s, lxp_s, gx2_s, ge_s, rows, sp, lam_x_out, lam_e_out);
 }
 

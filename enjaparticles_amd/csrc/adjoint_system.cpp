@@ -139,7 +139,7 @@ int forward_step(rtps_adj* a, const State& in, const State& out, Record& r, bool
         keys = ks;
     }
     // force loop 5 on recorded rows, which the adjoint reads as well
-    Win w{keys, a->gps.grid_res.x, a->gps.grid_res.y, a->gps.grid_res.z, 0, 0, 5};
+    Win w{keys, a->gps.grid_res.x, a->gps.grid_res.y, a->gps.grid_res.z, adj_remap(n), 0, 5};
     w.sub = a->sub;
     w.rows = r.rows;
     w.rows_stride = (uint32_t)n;

@@ -25,7 +25,7 @@ struct ItemCtx {
 };
 
 __device__ __forceinline__ ItemCtx item_ctx(const BatchItem* __restrict__ items) {
-    const BatchItem it = items[blockIdx.x];
+    const BatchItem it = items[xcd_tile(blockIdx.x, gridDim.x)];
     ItemCtx c;
     c.s = __builtin_amdgcn_readfirstlane(it.scene);
     c.i = it.first + (int)threadIdx.x;
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kBABlock) void k_badj_b1(const BatchItem* __restric
 
 // The 64-slot item of a block of B2 or B3: slot of the calling lane.
 __device__ __forceinline__ ItemCtx item64_ctx(const BatchItem* __restrict__ items) {
-    const BatchItem it = items[blockIdx.x];
+    const BatchItem it = items[xcd_tile(blockIdx.x, gridDim.x)];
     const int lane = (int)threadIdx.x & 63;
     return ItemCtx{__builtin_amdgcn_readfirstlane(it.scene), it.first + lane, lane < it.count};
 }
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_badj_b2(const BatchItem* __rest
                                                          float* __restrict__ grho_s, float2* __restrict__ partial) {
     const ItemCtx c = item64_ctx(items);
     adj_b2_tile(c.i, c.valid, pos_s, ve_s, ga_s, gX_s, rows, scenes[c.s].sp, gx2_s, ge_s, grho_s,
-                partial + blockIdx.x);
+                partial + xcd_tile(blockIdx.x, gridDim.x));
 }
 
 __global__ __launch_bounds__(kAdjThreads) void k_badj_b3(const BatchItem* __restrict__ items,

@@ -461,7 +461,9 @@ __global__ __launch_bounds__(192, 5) void k_pairs_split_b(const BatchItem* __res
                                                        const uint32_t* __restrict__ sub, uint32_t* __restrict__ rows,
                                                        uint32_t rows_stride) {
     __shared__ float4 stage_b[3][2 * kBStageCap];
-    const BatchItem I = items64[blockIdx.x];
+    // in XCD order: a scene's rows from one L2 (20 scenes' gradient: 2.43 -> 2.28 ms,
+    // with the adjoint's kernels)
+    const BatchItem I = items64[xcd_tile(blockIdx.x, gridDim.x)];
     const int s = __builtin_amdgcn_readfirstlane(I.scene);
     const SceneDev& S = scenes[s];
     const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
