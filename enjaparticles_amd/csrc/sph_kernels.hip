@@ -97,7 +97,8 @@ __global__ void k_read_nc(const uint32_t* __restrict__ start, int nb_cells, int*
 __global__ __launch_bounds__(kBlock) void k_max_i32(int n, const int32_t* __restrict__ v, int32_t* __restrict__ out) {
     __shared__ int32_t part[kBlock / 64];
     int32_t m = INT32_MIN;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) m = max(m, v[i]);
+    // 64-bit: the stride goes past INT_MAX at counts within kMaxBlocks * kBlock of 2^31
+    for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long)gridDim.x * kBlock) m = max(m, v[i]);
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_down(m, o, 64));
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
     __syncthreads();
