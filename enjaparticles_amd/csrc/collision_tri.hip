@@ -165,7 +165,8 @@ TriBins bin_triangles(const std::vector<TriPrep>& prep, float dist) {
 
 hipError_t TriDevice::load(const std::vector<TriPrep>& prep, float dist, hipStream_t st) {
     set = TriSet{};
-    if (prep.empty()) return hipSuccess;
+    // a hit needs dist - |pos - tp| > 1e-6: none at a distance that is negative, zero, infinite or not a number
+    if (prep.empty() || !(dist > 0.f) || !std::isfinite(dist)) return hipSuccess;
     const TriBins B = bin_triangles(prep, dist);
     if (B.start.empty()) return hipSuccess;   // no finite triangle
     // one allocation and one copy: spheres in list order, records, cell starts, lists
