@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <exception>
 #include <string>
 #include <vector>
 
@@ -208,7 +209,7 @@ int rtps_collision_wall(int num, const rtps_float4* pos_s, const rtps_float4* ve
 }
 
 int rtps_collision_triangles(int num, const rtps_float4* pos_s, const rtps_float4* vel_s, rtps_float4* force,
-                             const rtps_triangle* tris, int n, const rtps_sph_params* sphp, void* stream) {
+                             const rtps_triangle* tris, int n, const rtps_sph_params* sphp, void* stream) try {
     RTPS_CHECK(num >= 0 && n >= 0 && sphp && (tris || n == 0), "rtps_collision_triangles: bad arguments");
     if (num == 0 || n == 0) return RTPS_OK;
     RTPS_CHECK(pos_s && vel_s && force, "rtps_collision_triangles: null buffer");
@@ -221,6 +222,8 @@ int rtps_collision_triangles(int num, const rtps_float4* pos_s, const rtps_float
                                 &dev.set, nullptr, nullptr, nullptr, nullptr, S(stream)));
     RTPS_HIP(hipStreamSynchronize(S(stream)));   // the triangle memory goes with dev
     return RTPS_OK;
+} catch (const std::exception& e) {
+    return set_error(RTPS_ERR_ARG, std::string("rtps_collision_triangles: ") + e.what());
 }
 
 int rtps_leapfrog(int num, const rtps_float4* pos_s, const rtps_float4* vel_s, const rtps_float4* force,

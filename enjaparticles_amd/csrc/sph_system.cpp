@@ -171,11 +171,14 @@ hipError_t dalloc(T** p, size_t count) {
 void load_gravity_sources(rtps_sph* s) { gravity_sources_of(s->settings, s->gsrc); }
 
 // Triangles in the current simulation scale and boundary distance, on the device.
-hipError_t upload_triangles(rtps_sph* s) {
+hipError_t upload_triangles(rtps_sph* s) try {
     std::vector<TriPrep> prep = prepare_triangles(s->triangles.data(), (int)s->triangles.size(),
                                                   s->sp.simulation_scale);
     set_triangle_reach(prep, s->sp.boundary_distance);
     return s->tri.load(prep, s->sp.boundary_distance, s->stream);
+} catch (const std::exception&) {   // no host memory
+    s->tri.set = TriSet{};
+    return hipErrorOutOfMemory;
 }
 
 void apply_settings(rtps_sph* s) {
@@ -837,11 +840,15 @@ int rtps_sph_refill_hose(rtps_sph* s, int index, int refill) {
 
 int rtps_sph_load_triangles(rtps_sph* s, const rtps_triangle* tris, int n) {
     if (!s || n < 0 || (n > 0 && !tris)) return set_error(RTPS_ERR_ARG, "rtps_sph_load_triangles: bad arguments");
-    s->triangles.assign(tris, tris + n);
+    s->graph_valid = false;   // also where the load fails: the captured steps' triangles are gone
+    s->timed_graph_valid = false;
+    try {
+        s->triangles.assign(tris, tris + n);
+    } catch (const std::exception& e) {
+        return set_error(RTPS_ERR_ARG, std::string("rtps_sph_load_triangles: ") + e.what());
+    }
     maybe_update_params(s);
     RTPS_TRY_HIP(upload_triangles(s));
-    s->graph_valid = false;
-    s->timed_graph_valid = false;
     return RTPS_OK;
 }
 
