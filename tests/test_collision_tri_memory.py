@@ -37,7 +37,7 @@ def test_system_without_device_memory(cuda):
     from enjaparticles_amd.rtps import RTPS
     sc = scenes.dam_custom(12, 12, 8, seed=3)
     sheet = np.array([[[0, 0, 0.1], [1, 0, 0.1], [0, 1, 0.1]]], np.float32)
-    many = np.random.default_rng(4).uniform(0, 1, (600000, 3, 3)).astype(np.float32)   # 48 MB of records alone
+    many = np.random.default_rng(4).uniform(0, 1, (3000000, 3, 3)).astype(np.float32)   # 300 MB of records and lists
     out = []
     for fails in (True, False):
         with RTPS.generateSystemInstance(sc.settings) as s:
@@ -48,7 +48,15 @@ def test_system_without_device_memory(cuda):
             s.synchronize()
             if fails:
                 torch.cuda.empty_cache()
-                spare = torch.empty(torch.cuda.mem_get_info()[0] - (32 << 20), dtype=torch.uint8, device=cuda)
+                # the device filled but for 64 MB (it gives out somewhat more than it reports as free)
+                spare = [torch.empty(torch.cuda.mem_get_info()[0] - (64 << 20), dtype=torch.uint8, device=cuda)]
+                try:
+                    while len(spare) < 64:
+                        spare.append(torch.empty(32 << 20, dtype=torch.uint8, device=cuda))
+                except torch.OutOfMemoryError:
+                    pass
+                del spare[-2:]
+                torch.cuda.empty_cache()
                 with pytest.raises(RTPSError):
                     s.loadTriangles(many)
                 del spare
