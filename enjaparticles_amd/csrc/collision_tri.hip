@@ -19,13 +19,28 @@
 
 #include <algorithm>
 #include <cmath>
-#include <cstring>
+#include <limits>
 #include <vector>
 
 #include "obstacles_device.h"
 #include "rtps_internal.h"
 
 namespace rtps {
+
+namespace {
+
+constexpr int kBlockTri = 256;
+// The spheres of the triangles in list order.
+__global__ __launch_bounds__(kBlockTri) void k_list_spheres(uint32_t n, const uint32_t* __restrict__ list,
+                                                            const TriPrep* __restrict__ tris,
+                                                            float4* __restrict__ sphere) {
+    const uint32_t q = blockIdx.x * kBlockTri + threadIdx.x;
+    if (q >= n) return;
+    const TriPrep& T = tris[list[q]];
+    sphere[q] = make_float4(T.cx, T.cy, T.cz, T.reach2);
+}
+
+}  // namespace
 
 std::vector<TriPrep> prepare_triangles(const rtps_triangle* tris, int n, float scale) {
 #pragma clang fp contract(off)
@@ -75,7 +90,31 @@ namespace {
 struct TriBins {
     float min[3] = {}, inv = 0.f;
     int n[3] = {};
-    std::vector<uint32_t> start, list;
+    std::vector<uint32_t> start;
+    struct Box {
+        float lo[3], hi[3];   // around triangle id
+        uint32_t id;
+    };
+    std::vector<Box> box;   // finite triangles
+    double wide = 0.0;      // added to them on each side
+    // cell(c) for every cell that box b may meet
+    template <typename Cell>
+    void each(const Box& b, Cell&& cell) const {
+        int f[3], t[3];
+        range(b, f, t);
+        for (int z = f[2]; z <= t[2]; ++z)
+            for (int y = f[1]; y <= t[1]; ++y)
+                for (int x = f[0]; x <= t[0]; ++x) cell(((size_t)z * n[1] + y) * n[0] + x);
+    }
+    size_t range(const Box& b, int (&f)[3], int (&t)[3]) const {   // those cells, and their number
+        size_t m = 1;
+        for (int k = 0; k < 3; ++k) {   // no box begins below min
+            f[k] = std::min((int)((b.lo[k] - (min[k] + wide)) * inv), n[k] - 1);
+            t[k] = std::min((int)((b.hi[k] - (min[k] - wide)) * inv), n[k] - 1);
+            m *= (size_t)(t[k] - f[k] + 1);
+        }
+        return m;
+    }
 };
 
 // Cells about as large as the triangles: a triangle then lies in a few cells
@@ -85,78 +124,62 @@ struct TriBins {
 // every triangle once.
 constexpr size_t kTriLists = 16, kTriCells = 1 << 18;
 
+// The grid and its cells' starts in the lists (start[c + 1] holds the number
+// before it, to be filled from there on).
 TriBins bin_triangles(const std::vector<TriPrep>& prep, float dist) {
     TriBins B;
-    struct Box {
-        double lo[3], hi[3];
-    };
-    std::vector<Box> box;
-    std::vector<uint32_t> id;
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300}, edge = 0.0, most = 0.0;
-    for (const TriPrep& P : prep)   // the largest coordinate: the scale of the particle side's roundings
-        for (float v : {P.ax, P.ay, P.az, P.bx, P.by, P.bz, P.qx, P.qy, P.qz})
-            if (std::isfinite(v)) most = std::max(most, (double)std::fabs(v));
+    constexpr double top = std::numeric_limits<float>::max();
+    float first[3] = {(float)top, (float)top, (float)top}, last[3] = {(float)-top, (float)-top, (float)-top};
+    double edge = 0.0;
+    B.box.reserve(prep.size());
     for (size_t q = 0; q < prep.size(); ++q) {
         const TriPrep& P = prep[q];
         const float v[3][3] = {{P.ax, P.bx, P.qx}, {P.ay, P.by, P.qy}, {P.az, P.bz, P.qz}};
-        Box b;
-        bool finite = true;
+        TriBins::Box b;
+        b.id = (uint32_t)q;
+        float none = 0.f, side = 0.f;
         for (int k = 0; k < 3; ++k) {
-            const double l = std::min({v[k][0], v[k][1], v[k][2]}), h = std::max({v[k][0], v[k][1], v[k][2]});
-            finite = finite && std::isfinite(v[k][0]) && std::isfinite(v[k][1]) && std::isfinite(v[k][2]);
-            // wider than the roundings of the particle's side (its cell index, tp, the
-            // distance), each below 1e-6 of the largest coordinate
-            const double w = dist * (1.0 + 1e-5) + 1e-6 + 1e-5 * most;
-            b.lo[k] = l - w;
-            b.hi[k] = h + w;
+            b.lo[k] = std::min(v[k][0], std::min(v[k][1], v[k][2]));
+            b.hi[k] = std::max(v[k][0], std::max(v[k][1], v[k][2]));
+            none += (v[k][0] - v[k][0]) + (v[k][1] - v[k][1]) + (v[k][2] - v[k][2]);
+            side = std::max(side, b.hi[k] - b.lo[k]);
         }
-        if (!finite) continue;   // no comparison of its test can hold
+        if (!(none == 0.f)) continue;   // infinite or not a number: no comparison of its test can hold
         for (int k = 0; k < 3; ++k) {
-            lo[k] = std::min(lo[k], b.lo[k]);
-            hi[k] = std::max(hi[k], b.hi[k]);
+            first[k] = std::min(first[k], b.lo[k]);
+            last[k] = std::max(last[k], b.hi[k]);
         }
-        edge += std::max({b.hi[0] - b.lo[0], b.hi[1] - b.lo[1], b.hi[2] - b.lo[2]});
-        box.push_back(b);
-        id.push_back((uint32_t)q);
+        edge += side;
+        B.box.push_back(b);
     }
-    if (box.empty()) return B;
-    const double extent = std::max({hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]});
-    edge /= (double)box.size();
-    for (int k = 0; k < 3; ++k) B.min[k] = (float)lo[k];
+    if (B.box.empty()) return B;
+    double most = 0.0, extent = 0.0, size[3];   // the largest coordinate: the scale of the particle side's roundings
+    for (int k = 0; k < 3; ++k) most = std::max({most, std::fabs((double)first[k]), std::fabs((double)last[k])});
+    // wider than the roundings of the particle's side (its cell index, tp, the
+    // distance), each below 1e-6 of the largest coordinate
+    B.wide = dist * (1.0 + 1e-5) + 1e-6 + 1e-5 * most;
+    for (int k = 0; k < 3; ++k) {
+        B.min[k] = (float)std::max(first[k] - B.wide, -top);
+        size[k] = last[k] + B.wide - B.min[k];
+        extent = std::max(extent, size[k]);
+    }
+    edge = edge / (double)B.box.size() + 2.0 * B.wide;
     for (;; edge *= 2.0) {
         const bool one = !(edge < extent);
         B.inv = one ? 0.f : (float)(1.0 / edge);   // one cell: every index is 0
         size_t cells = 1;
         for (int k = 0; k < 3; ++k) {
-            B.n[k] = one ? 1 : (int)std::min(1e6, std::floor((hi[k] - lo[k]) / edge) + 2.0);
+            B.n[k] = one ? 1 : (int)std::min(1e6, std::floor(size[k] / edge) + 2.0);
             cells *= (size_t)B.n[k];
         }
         if (!one && cells > kTriCells) continue;
-        auto range = [&](const Box& b, int (&f)[3], int (&t)[3]) {   // the cells the box may meet
-            size_t m = 1;
-            for (int k = 0; k < 3; ++k) {
-                f[k] = std::clamp((int)std::floor((b.lo[k] - B.min[k]) * B.inv), 0, B.n[k] - 1);
-                t[k] = std::clamp((int)std::floor((b.hi[k] - B.min[k]) * B.inv), 0, B.n[k] - 1);
-                m *= (size_t)(t[k] - f[k] + 1);
-            }
-            return m;
-        };
         int f[3], t[3];
         size_t total = 0;
-        for (const Box& b : box) total += range(b, f, t);
-        if (!one && total > kTriLists * box.size()) continue;
-        B.start.assign(cells + 1, 0);
-        B.list.resize(total);
-        auto each = [&](const Box& b, auto&& cell) {
-            range(b, f, t);
-            for (int z = f[2]; z <= t[2]; ++z)
-                for (int y = f[1]; y <= t[1]; ++y)
-                    for (int x = f[0]; x <= t[0]; ++x) cell(((size_t)z * B.n[1] + y) * B.n[0] + x);
-        };
-        for (const Box& b : box) each(b, [&](size_t c) { ++B.start[c + 1]; });
-        for (size_t c = 0; c < cells; ++c) B.start[c + 1] += B.start[c];
-        std::vector<uint32_t> at(B.start.begin(), B.start.end() - 1);
-        for (size_t q = 0; q < box.size(); ++q) each(box[q], [&](size_t c) { B.list[at[c]++] = id[q]; });
+        for (const TriBins::Box& b : B.box) total += B.range(b, f, t);
+        if (!one && total > kTriLists * B.box.size()) continue;
+        B.start.assign(cells + 2, 0);
+        for (const TriBins::Box& b : B.box) B.each(b, [&](size_t c) { ++B.start[c + 2]; });
+        for (size_t c = 0; c < cells; ++c) B.start[c + 2] += B.start[c + 1];
         return B;
     }
 }
@@ -164,23 +187,20 @@ TriBins bin_triangles(const std::vector<TriPrep>& prep, float dist) {
 }  // namespace
 
 hipError_t TriDevice::load(const std::vector<TriPrep>& prep, float dist, hipStream_t st) {
+    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
     set = TriSet{};
     // a hit needs dist - |pos - tp| > 1e-6: none at a distance that is negative, zero, infinite or not a number
     if (prep.empty() || !(dist > 0.f) || !std::isfinite(dist)) return hipSuccess;
-    const TriBins B = bin_triangles(prep, dist);
+    TriBins B = bin_triangles(prep, dist);
     if (B.start.empty()) return hipSuccess;   // no finite triangle
-    // one allocation and one copy: spheres in list order, records, cell starts, lists
-    const size_t o_tri = B.list.size() * sizeof(float4), o_start = o_tri + prep.size() * sizeof(TriPrep),
-                 o_list = o_start + B.start.size() * 4, bytes = o_list + B.list.size() * 4;
-    std::vector<char> host(bytes);
-    for (size_t q = 0; q < B.list.size(); ++q) {
-        const TriPrep& P = prep[B.list[q]];
-        const float sphere[4] = {P.cx, P.cy, P.cz, P.reach2};
-        std::memcpy(&host[q * sizeof(float4)], sphere, sizeof(sphere));
-    }
-    std::memcpy(&host[o_tri], prep.data(), prep.size() * sizeof(TriPrep));
-    std::memcpy(&host[o_start], B.start.data(), B.start.size() * 4);
-    std::memcpy(&host[o_list], B.list.data(), B.list.size() * 4);
+    // one allocation: spheres in list order, records, cell starts, lists
+    const size_t listed = B.start.back(), cells = B.start.size() - 2;
+    std::vector<uint32_t> host(cells + 1 + listed);
+    uint32_t* const list = host.data() + cells + 1;
+    for (const TriBins::Box& b : B.box) B.each(b, [&](size_t c) { list[B.start[c + 1]++] = b.id; });
+    std::copy_n(B.start.begin(), cells + 1, host.begin());
+    const size_t o_tri = listed * sizeof(float4), o_start = o_tri + prep.size() * sizeof(TriPrep),
+                 o_list = o_start + (cells + 1) * 4, bytes = o_list + listed * 4;
     hipError_t e = hipStreamSynchronize(st);   // launches that read the former triangles
     if (e == hipSuccess && bytes > cap) {
         if (mem) e = hipFree(mem);
@@ -190,8 +210,14 @@ hipError_t TriDevice::load(const std::vector<TriPrep>& prep, float dist, hipStre
         if (e != hipSuccess) return e;
         cap = bytes;
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(mem, host.data(), bytes, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = hipMemcpyAsync(mem + o_tri, prep.data(), o_start - o_tri, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(mem + o_start, host.data(), bytes - o_start, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) {
+        k_list_spheres<<<(uint32_t)((listed + kBlockTri - 1) / kBlockTri), kBlockTri, 0, st>>>(
+            (uint32_t)listed, (const uint32_t*)(mem + o_list), (const TriPrep*)(mem + o_tri), (float4*)mem);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(st);   // the host arrays are read
     if (e != hipSuccess) return e;
     set.n = (int)prep.size();
     set.sphere = (const float4*)mem;
