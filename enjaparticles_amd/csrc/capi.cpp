@@ -215,12 +215,8 @@ int rtps_collision_triangles(int num, const rtps_float4* pos_s, const rtps_float
     RTPS_CHECK(pos_s && vel_s && force, "rtps_collision_triangles: null buffer");
     std::vector<TriPrep> prep = prepare_triangles(tris, n, sphp->simulation_scale);
     set_triangle_reach(prep, sphp->boundary_distance);
-    TriDevice dev;
-    RTPS_HIP(dev.load(prep, sphp->boundary_distance, S(stream)));
-    RTPS_HIP(launch_after_force(num, nullptr, nullptr, 0, (const float4*)pos_s, (const float4*)vel_s, nullptr,
-                                (float4*)force, nullptr, nullptr, *sphp, AfterForce{}, GravitySources{}, Grid{},
-                                &dev.set, nullptr, nullptr, nullptr, nullptr, S(stream)));
-    RTPS_HIP(hipStreamSynchronize(S(stream)));   // the triangle memory goes with dev
+    RTPS_HIP(collision_triangles(num, (const float4*)pos_s, (const float4*)vel_s, (float4*)force, prep, *sphp,
+                                 S(stream)));
     return RTPS_OK;
 } catch (const std::exception& e) {
     return set_error(RTPS_ERR_ARG, std::string("rtps_collision_triangles: ") + e.what());

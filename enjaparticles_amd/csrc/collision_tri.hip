@@ -1,6 +1,6 @@
-// Triangle collision: the loaded triangles on the device, for
-// CollisionTriangle::execute (Collision_triangle.cpp, collision_tri.cl:120-231
-// and 418-470; the device side is tri_forces in obstacles_device.h).
+// Triangle collision, CollisionTriangle::execute (Collision_triangle.cpp,
+// collision_tri.cl:120-231 and 418-470; one particle and one triangle are
+// tri_add in obstacles_device.h).
 //
 // Per triangle the host prepares, in the simulation scale, its vertices
 // a, b, c (= v * scale), n = (b - a) x (c - a), the unit normal n / |n| and a
@@ -8,12 +8,18 @@
 // centre cannot get a hit closer than dist (tp lies in the triangle), so it
 // skips the test; that changes no result.
 //
-// A particle visits only the triangles listed in its cell of a grid laid over
-// them (bin_triangles): those whose box, widened by dist, meets the cell, in
-// triangle order.  Culling blocks of particles against the triangles instead
-// leaves the blocks that span a change of row or plane with most of them:
-// 97 us for 150,001 particles and 1,152 triangles, of which the sheet in the
-// pool touches a fraction.
+// A system's triangles are loaded once and met in every step: a particle
+// visits only those listed in its cell of a grid laid over them
+// (bin_triangles), whose box, widened by dist, meets the cell, in triangle
+// order.  Culling blocks of particles against the triangles instead leaves the
+// blocks that span a change of row or plane with most of them: 97 us a step for
+// 150,001 particles and 1,152 triangles, of which the sheet in the pool touches
+// a fraction.
+//
+// The stage operator's triangles are met once, where making the lists costs
+// the host more than they save: k_collision_tri culls by block.  Only for few
+// particles, whose blocks leave most of the chip idle while each goes through
+// all triangles, the lists are made there, too (kListParticles).
 
 #include <hip/hip_runtime.h>
 
@@ -30,6 +36,102 @@ namespace rtps {
 namespace {
 
 constexpr int kBlockTri = 256;
+constexpr int kWavesTri = kBlockTri / 64;
+constexpr int kTriChunk = 256;   // triangles tested per chunk (one per thread); 20 KiB of TriPrep in LDS
+
+__device__ __forceinline__ float wave_min(float v) {
+    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
+    return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+    return v;
+}
+
+// Blocks of consecutive sorted particles are compact in space: per chunk of
+// triangles, each thread tests one triangle's sphere (centre, reach squared)
+// against the block's bounding box, and those that meet it are compacted into
+// LDS in triangle order (ballot ranks, then per-wave offsets).
+__global__ __launch_bounds__(kBlockTri) void k_collision_tri(int num, const float4* __restrict__ pos_s,
+                                                             const float4* __restrict__ vel_s,
+                                                             float4* __restrict__ force,
+                                                             const TriPrep* __restrict__ tris,
+                                                             const float4* __restrict__ sphere, int ntri,
+                                                             rtps_sph_params sp) {
+    __shared__ TriPrep lt[kTriChunk];
+    __shared__ float box[kWavesTri][6];
+    __shared__ int wave_n[kWavesTri];
+    const int i = blockIdx.x * kBlockTri + threadIdx.x;
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    const bool live = i < num;
+    const float s = sp.simulation_scale;
+    float4 p = make_float4(0.f, 0.f, 0.f, 0.f), v = p;
+    if (live) {
+        p = pos_s[i];
+        v = vel_s[i];
+    }
+    const float px = p.x * s, py = p.y * s, pz = p.z * s;
+    // bounding box of the block's live particles
+    {
+        const float inf = __builtin_inff();
+        const float lo[3] = {live ? px : inf, live ? py : inf, live ? pz : inf};
+        const float hi[3] = {live ? px : -inf, live ? py : -inf, live ? pz : -inf};
+        for (int c = 0; c < 3; ++c) {
+            const float a = wave_min(lo[c]), b = wave_max(hi[c]);
+            if (lane == 0) {
+                box[wave][c] = a;
+                box[wave][3 + c] = b;
+            }
+        }
+    }
+    __syncthreads();
+    float bl[3], bh[3];
+    for (int c = 0; c < 3; ++c) {
+        bl[c] = box[0][c];
+        bh[c] = box[0][3 + c];
+        for (int w = 1; w < kWavesTri; ++w) {
+            bl[c] = fminf(bl[c], box[w][c]);
+            bh[c] = fmaxf(bh[c], box[w][3 + c]);
+        }
+    }
+    float3 f = make_float3(0.f, 0.f, 0.f);
+    for (int c0 = 0; c0 < ntri; c0 += kTriChunk) {
+        const int t = c0 + (int)threadIdx.x;
+        bool cand = false;
+        if (t < ntri) {
+            const float4 r = sphere[t];
+            const float dx = fmaxf(fmaxf(bl[0] - r.x, r.x - bh[0]), 0.f);
+            const float dy = fmaxf(fmaxf(bl[1] - r.y, r.y - bh[1]), 0.f);
+            const float dz = fmaxf(fmaxf(bl[2] - r.z, r.z - bh[2]), 0.f);
+            cand = dx * dx + dy * dy + dz * dz <= r.w;
+        }
+        const unsigned long long m = __ballot(cand);
+        const int rank = __popcll(m & ((1ull << lane) - 1ull));
+        __syncthreads();   // the previous chunk's triangles are no longer read
+        if (lane == 0) wave_n[wave] = __popcll(m);
+        __syncthreads();
+        int base = 0, total = 0;
+        for (int w = 0; w < kWavesTri; ++w) {
+            if (w < wave) base += wave_n[w];
+            total += wave_n[w];
+        }
+        if (cand) lt[base + rank] = tris[t];
+        __syncthreads();
+        if (!live) continue;
+        for (int q = 0; q < total; ++q) {
+            const TriPrep& T = lt[q];
+            const float cx = px - T.cx, cy = py - T.cy, cz = pz - T.cz;
+            if (!(cx * cx + cy * cy + cz * cz > T.reach2)) tri_add(f, px, py, pz, v, T, sp);
+        }
+    }
+    if (!live) return;
+    float4 F = force[i];
+    F.x += f.x;
+    F.y += f.y;
+    F.z += f.z;
+    force[i] = F;
+}
+
 // The spheres of the triangles in list order.
 __global__ __launch_bounds__(kBlockTri) void k_list_spheres(uint32_t n, const uint32_t* __restrict__ list,
                                                             const TriPrep* __restrict__ tris,
@@ -41,6 +143,50 @@ __global__ __launch_bounds__(kBlockTri) void k_list_spheres(uint32_t n, const ui
 }
 
 }  // namespace
+
+// Where the lists pay for one call.  Measured for the operator (us, lists /
+// blocks): 59 / 40 with 2 triangles and 86 / 74 with 128 (1,000 particles and
+// more); with 1,152, 5,000 and 20,000 triangles 194 / 264, 422 / 845 and
+// 1,475 / 2,380 at 1,000 particles, 147 / 172, 348 / 494 and 1,208 / 1,618 at
+// 10,000, 134 / 125, 333 / 290 and 1,149 / 819 at 50,000, 137 / 154, 341 / 360
+// and 1,165 / 1,014 at 600,000; with 180,000 14.9 / 22.0, 13.8 / 15.6,
+// 13.0 / 6.2 and 9.8 / 7.9 ms.
+constexpr int kListParticles = 1 << 14;
+constexpr size_t kListTriangles = 1 << 10;
+
+hipError_t collision_triangles(int num, const float4* pos_s, const float4* vel_s, float4* force,
+                               const std::vector<TriPrep>& prep, const rtps_sph_params& sp, hipStream_t st) {
+    (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
+    if (num <= 0 || prep.empty()) return hipSuccess;
+    if (num <= kListParticles && prep.size() >= kListTriangles) {
+        TriDevice dev;
+        hipError_t e = dev.load(prep, sp.boundary_distance, st);
+        if (e == hipSuccess)
+            e = launch_after_force(num, nullptr, nullptr, 0, pos_s, vel_s, nullptr, force, nullptr, nullptr, sp,
+                                   AfterForce{}, GravitySources{}, Grid{}, &dev.set, nullptr, nullptr, nullptr,
+                                   nullptr, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);   // the triangle memory goes with dev
+        return e;
+    }
+    std::vector<float4> sphere(prep.size());
+    for (size_t q = 0; q < prep.size(); ++q)
+        sphere[q] = make_float4(prep[q].cx, prep[q].cy, prep[q].cz, prep[q].reach2);
+    TriPrep* dev = nullptr;
+    hipError_t e = hipMalloc((void**)&dev, prep.size() * (sizeof(TriPrep) + sizeof(float4)));
+    if (e != hipSuccess) return e;
+    float4* dev_sphere = reinterpret_cast<float4*>(dev + prep.size());
+    e = hipMemcpyAsync(dev, prep.data(), prep.size() * sizeof(TriPrep), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(dev_sphere, sphere.data(), sphere.size() * sizeof(float4), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) {
+        k_collision_tri<<<(num + kBlockTri - 1) / kBlockTri, kBlockTri, 0, st>>>(num, pos_s, vel_s, force, dev,
+                                                                               dev_sphere, (int)prep.size(), sp);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(st);   // the triangles are freed below
+    (void)hipFree(dev);
+    return e;
+}
 
 std::vector<TriPrep> prepare_triangles(const rtps_triangle* tris, int n, float scale) {
 #pragma clang fp contract(off)

@@ -9,16 +9,64 @@
 
 namespace rtps {
 
-// Triangle collision of collision_tri.cl:120-231, 418-470 for one particle
-// (p, v unscaled).  For every triangle of the particle's cell, the segment
-// pos +- dist * v/|v| (dist = boundary_distance) is intersected with the
-// triangle (Ericson, Real-Time Collision Detection, pp. 191-192); on a hit at
-// tp, penetration = dist - |pos - tp| and, when it exceeds 1e-6, the repulsion
+// Triangle collision of collision_tri.cl:120-231, 418-470 for one particle at
+// px, py, pz (scaled) with velocity v and one triangle: the segment
+// pos +- dist * v/|v| (dist = boundary_distance) is intersected with it
+// (Ericson, Real-Time Collision Detection, pp. 191-192); on a hit at tp,
+// penetration = dist - |pos - tp| and, when it exceeds 1e-6, the repulsion
 // and friction of cl_sph_collision.h:31-73 along the triangle's unit normal
-// are added, in triangle order.
+// are added to f.
+__device__ __forceinline__ void tri_add(float3& f, float px, float py, float pz, float4 v, const TriPrep& T,
+                                        const rtps_sph_params& sp) {
+    const float dist = sp.boundary_distance, k = sp.boundary_stiffness, damp = sp.boundary_dampening;
+    // v3normalize (collision_tri.cl:46-50): NaN for v = 0, and then no hit
+    const float mag = __builtin_sqrtf(v.x * v.x + v.y * v.y + v.z * v.z);
+    const float vnx = v.x / mag, vny = v.y / mag, vnz = v.z / mag;
+    // segment ends p = pos - vn dist, q = pos + vn dist (collision_tri.cl:135-137)
+    const float sx = px - vnx * dist, sy = py - vny * dist, sz = pz - vnz * dist;
+    const float qx = px + vnx * dist, qy = py + vny * dist, qz = pz + vnz * dist;
+    const float qpx = sx - qx, qpy = sy - qy, qpz = sz - qz;
+    // Ericson segment-triangle test (collision_tri.cl:120-170)
+    const float d = qpx * T.nx + qpy * T.ny + qpz * T.nz;
+    if (d <= 0.0f) return;
+    const float apx = sx - T.ax, apy = sy - T.ay, apz = sz - T.az;
+    float tt = apx * T.nx + apy * T.ny + apz * T.nz;
+    if (tt < 0.0f || tt > d) return;
+    const float ex = qpy * apz - qpz * apy, ey = qpz * apx - qpx * apz, ez = qpx * apy - qpy * apx;
+    const float abx = T.bx - T.ax, aby = T.by - T.ay, abz = T.bz - T.az;
+    const float acx = T.qx - T.ax, acy = T.qy - T.ay, acz = T.qz - T.az;
+    float vv = acx * ex + acy * ey + acz * ez;
+    if (vv < 0.0f || vv > d) return;
+    float ww = -(abx * ex + aby * ey + abz * ez);
+    if (ww < 0.0f || vv + ww > d) return;
+    const float ood = 1.0f / d;
+    vv *= ood;
+    ww *= ood;
+    const float uu = 1.0f - vv - ww;
+    const float tx = uu * T.ax + vv * T.bx + ww * T.qx;   // tp = u a + v b + w c
+    const float ty = uu * T.ay + vv * T.by + ww * T.qy;
+    const float tz = uu * T.az + vv * T.bz + ww * T.qz;
+    const float ddx = px - tx, ddy = py - ty, ddz = pz - tz;
+    const float pen = dist - __builtin_sqrtf(ddx * ddx + ddy * ddy + ddz * ddz);
+    if (!(pen > 1e-6f)) return;   // collision_tri.cl:196
+    // calculateRepulsionForce + calculateFrictionForce (zero coefficients)
+    const float ndv = T.ux * v.x + T.uy * v.y + T.uz * v.z;
+    const float m2 = k * pen - damp * ndv;
+    f.x += m2 * T.ux;
+    f.y += m2 * T.uy;
+    f.z += m2 * T.uz;
+    const float vtx = v.x - v.x * ndv, vty = v.y - v.y * ndv, vtz = v.z - v.z * ndv;
+    if ((vtx + vty + vtz) / 3.0f > 0.0f) {
+        f.x -= vtx;
+        f.y -= vty;
+        f.z -= vtz;
+    }
+}
+
+// The forces of the triangles listed in the particle's cell (p, v unscaled),
+// in triangle order.
 __device__ __forceinline__ float3 tri_forces(float4 p, float4 v, const TriSet& S, const rtps_sph_params& sp) {
-    const float s = sp.simulation_scale, dist = sp.boundary_distance;
-    const float k = sp.boundary_stiffness, damp = sp.boundary_dampening;
+    const float s = sp.simulation_scale;
     const float px = p.x * s, py = p.y * s, pz = p.z * s;
     float3 f = make_float3(0.f, 0.f, 0.f);
     const float ux = (px - S.min.x) * S.inv, uy = (py - S.min.y) * S.inv, uz = (pz - S.min.z) * S.inv;
@@ -38,52 +86,8 @@ __device__ __forceinline__ float3 tri_forces(float4 p, float4 v, const TriSet& S
             const bool outside = cx * cx + cy * cy + cz * cz > r.w;   // no hit within dist
             meet |= !outside && q0 + g < q1 ? 1u << g : 0u;
         }
-        for (; meet != 0u; meet &= meet - 1u) {
-            const uint32_t t = S.list[q0 + (uint32_t)__builtin_ctz(meet)];
-            const TriPrep& T = S.tris[t];
-            // v3normalize (collision_tri.cl:46-50): NaN for v = 0, and then no hit
-            const float mag = __builtin_sqrtf(v.x * v.x + v.y * v.y + v.z * v.z);
-            const float vnx = v.x / mag, vny = v.y / mag, vnz = v.z / mag;
-            // segment ends p = pos - vn dist, q = pos + vn dist (collision_tri.cl:135-137)
-            const float sx = px - vnx * dist, sy = py - vny * dist, sz = pz - vnz * dist;
-            const float qx = px + vnx * dist, qy = py + vny * dist, qz = pz + vnz * dist;
-            const float qpx = sx - qx, qpy = sy - qy, qpz = sz - qz;
-            // Ericson segment-triangle test (collision_tri.cl:120-170)
-            const float d = qpx * T.nx + qpy * T.ny + qpz * T.nz;
-            if (d <= 0.0f) continue;
-            const float apx = sx - T.ax, apy = sy - T.ay, apz = sz - T.az;
-            float tt = apx * T.nx + apy * T.ny + apz * T.nz;
-            if (tt < 0.0f || tt > d) continue;
-            const float ex = qpy * apz - qpz * apy, ey = qpz * apx - qpx * apz, ez = qpx * apy - qpy * apx;
-            const float abx = T.bx - T.ax, aby = T.by - T.ay, abz = T.bz - T.az;
-            const float acx = T.qx - T.ax, acy = T.qy - T.ay, acz = T.qz - T.az;
-            float vv = acx * ex + acy * ey + acz * ez;
-            if (vv < 0.0f || vv > d) continue;
-            float ww = -(abx * ex + aby * ey + abz * ez);
-            if (ww < 0.0f || vv + ww > d) continue;
-            const float ood = 1.0f / d;
-            vv *= ood;
-            ww *= ood;
-            const float uu = 1.0f - vv - ww;
-            const float tx = uu * T.ax + vv * T.bx + ww * T.qx;   // tp = u a + v b + w c
-            const float ty = uu * T.ay + vv * T.by + ww * T.qy;
-            const float tz = uu * T.az + vv * T.bz + ww * T.qz;
-            const float ddx = px - tx, ddy = py - ty, ddz = pz - tz;
-            const float pen = dist - __builtin_sqrtf(ddx * ddx + ddy * ddy + ddz * ddz);
-            if (!(pen > 1e-6f)) continue;   // collision_tri.cl:196
-            // calculateRepulsionForce + calculateFrictionForce (zero coefficients)
-            const float ndv = T.ux * v.x + T.uy * v.y + T.uz * v.z;
-            const float m2 = k * pen - damp * ndv;
-            f.x += m2 * T.ux;
-            f.y += m2 * T.uy;
-            f.z += m2 * T.uz;
-            const float vtx = v.x - v.x * ndv, vty = v.y - v.y * ndv, vtz = v.z - v.z * ndv;
-            if ((vtx + vty + vtz) / 3.0f > 0.0f) {
-                f.x -= vtx;
-                f.y -= vty;
-                f.z -= vtz;
-            }
-        }
+        for (; meet != 0u; meet &= meet - 1u)
+            tri_add(f, px, py, pz, v, S.tris[S.list[q0 + (uint32_t)__builtin_ctz(meet)]], sp);
     }
     return f;
 }

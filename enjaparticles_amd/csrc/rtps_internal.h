@@ -149,6 +149,9 @@ struct TriPrep {
 };
 std::vector<TriPrep> prepare_triangles(const rtps_triangle* tris, int n, float scale);
 void set_triangle_reach(std::vector<TriPrep>& t, float dist);
+// Adds the triangles' forces to force, once (waits for the stream).
+hipError_t collision_triangles(int num, const float4* pos_s, const float4* vel_s, float4* force,
+                               const std::vector<TriPrep>& prep, const rtps_sph_params& sp, hipStream_t st);
 // The triangles on the device, and a grid over them: a particle in cell c can
 // touch the triangles list[q], q in start[c]..start[c + 1] - 1, whose bounding
 // spheres (centre, reach squared) are sphere[q].
