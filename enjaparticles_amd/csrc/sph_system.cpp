@@ -97,6 +97,8 @@ struct rtps_sph {
     std::vector<rtps_hose*> hoses;   // SPH::hoses (SPH.h), sprayed at the start of every update
     std::vector<rtps_triangle> triangles;   // SPH::loadTriangles, world units
     TriDevice tri;
+    bool tri_loaded = false;   // tri holds the triangles, in this scale and boundary distance:
+    float tri_scale = 0.f, tri_dist = 0.f;
     std::vector<rtps_float4> hose_color;
     // rigid-body particle sets of SPH::interact: [0] a moving body, [1] the static boundary
     RigidDev rigid[2];
@@ -172,10 +174,14 @@ void load_gravity_sources(rtps_sph* s) { gravity_sources_of(s->settings, s->gsrc
 
 // Triangles in the current simulation scale and boundary distance, on the device.
 hipError_t upload_triangles(rtps_sph* s) try {
-    std::vector<TriPrep> prep = prepare_triangles(s->triangles.data(), (int)s->triangles.size(),
-                                                  s->sp.simulation_scale);
-    set_triangle_reach(prep, s->sp.boundary_distance);
-    return s->tri.load(prep, s->sp.boundary_distance, s->stream);
+    s->tri_loaded = false;
+    s->tri_scale = s->sp.simulation_scale;
+    s->tri_dist = s->sp.boundary_distance;
+    std::vector<TriPrep> prep = prepare_triangles(s->triangles.data(), (int)s->triangles.size(), s->tri_scale);
+    set_triangle_reach(prep, s->tri_dist);
+    const hipError_t e = s->tri.load(prep, s->tri_dist, s->stream);
+    s->tri_loaded = e == hipSuccess;
+    return e;
 } catch (const std::exception&) {   // no host memory
     s->tri.set = TriSet{};
     return hipErrorOutOfMemory;
@@ -187,7 +193,10 @@ void apply_settings(rtps_sph* s) {
     s->sp.num = s->num_host;
     s->dt = s->settings.GetSettingAs<float>("time_step");
     load_gravity_sources(s);
-    if (!s->triangles.empty()) (void)upload_triangles(s);   // a failure leaves none: reported by the next load
+    // (every push comes here: the triangles are loaded again only where that changes them)
+    if (!s->triangles.empty() &&
+        !(s->tri_loaded && s->tri_scale == s->sp.simulation_scale && s->tri_dist == s->sp.boundary_distance))
+        (void)upload_triangles(s);   // a failure leaves none: reported by the next load
     s->settings.updated();
     s->graph_valid = false;
     s->timed_graph_valid = false;
