@@ -4,7 +4,9 @@
 // the grid's cells.  The order is the stable sort's: keys (cell << 4 | x
 // sixteenth) ascending, equal keys by particle index.
 //
-// Up to 4,096 particles k_cell_sort_one makes the order, above these three do:
+// Up to 4,096 particles on grids whose counters fit LDS (some 24,000 cells at
+// 4,096 particles) k_cell_sort_one makes the order and launch_cells_permute the
+// rest, above these four do:
 //
 //   k_cell_count    the key of every particle (hash_key) and its arrival rank
 //                   in its cell: one atomic on the cell's counter.
@@ -21,7 +23,12 @@
 // between tiles, and writes the cell tables on the way.  A cell holds 8
 // particles at rest and 20 to 40 in a settled pool, so the counting inside a
 // cell is short; a cell of m particles costs m^2 comparisons, 9,000 stacked in
-// one cell 0.3 ms.
+// one cell 0.3 ms, which their pair sums then exceed.  The particles outside the
+// grid, in one cell more, have no pair sums and may be any number: their keys
+// are equal, so their order is that of the indices, and count leaves a bit for
+// each slot that holds one, from which place counts (outside_rank).  A step of
+// which 95% are outside takes 0.15 ms at 327,680 particles and 0.21 in a batch of
+// 400,000; 47 and 78 where they are compared in pairs.
 
 #include <hip/hip_runtime.h>
 
@@ -42,10 +49,11 @@ constexpr int kScanBlocks = 256;              // at most: a block adds up every 
 static inline int cs_blocks(long n) { return (int)((n + kCsThreads - 1) / kCsThreads); }
 
 // Layout of the temp: the counters (zero between sorts), the scan's status
-// words, the pairs.
+// words, the slots' bits of particles outside the grid, the pairs.
 struct CellTemp {
     uint32_t* count;
     unsigned long long* status;
+    uint64_t* outside;
     uint2* pairs;
 };
 static size_t cell_layout(int n, int nb_cells, CellTemp* t, char* p) {
@@ -54,6 +62,8 @@ static size_t cell_layout(int n, int nb_cells, CellTemp* t, char* p) {
     off += (((size_t)nb_cells + 1) * 4 + 255) & ~(size_t)255;
     if (t) t->status = (unsigned long long*)(p + off);
     off += kScanBlocks * sizeof(unsigned long long);
+    if (t) t->outside = (uint64_t*)(p + off);
+    off += (size_t)cs_blocks(std::max(n, kScanBlocks)) * (kCsThreads / 64) * sizeof(uint64_t);   // one per wave of the count
     if (t) t->pairs = (uint2*)(p + off);
     return off + (size_t)std::max(n, 1) * sizeof(uint2);
 }
@@ -83,18 +93,40 @@ bool cell_sort_fits(int n, int nb_cells) { return n <= kCellSortMax && (long)nb_
 // slots, is where settled scenes still gain.
 bool cell_sort_fits_b(long T, long total_cells) { return T <= 1 << 20 && total_cells <= 16 * T + (1 << 20); }
 
+// The place of lane `lane` of a wave over the slots [first, first + 64) among the
+// particles outside the grid of its scene, which begins at slot `off`: those in
+// the scene's slots before it.  same: the wave's lanes that hold one of that
+// scene.  Called by whole waves.
+__device__ __forceinline__ uint32_t outside_rank(const uint64_t* __restrict__ outside, int off, int first, int lane,
+                                                 uint64_t same) {
+    uint32_t before = 0u;
+    for (int w = (off >> 6) + lane; w < first >> 6; w += 64) {
+        const uint64_t m = w == off >> 6 ? ~0ull << (off & 63) : ~0ull;   // the scene's part of its first word
+        before += (uint32_t)__popcll(outside[w] & m);
+    }
+    before = __shfl(wave_incl_scan(before), 63);
+    return before + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+}
+
 __global__ __launch_bounds__(kCsThreads) void k_cell_count(int num_host, const int* __restrict__ d_num,
                                                            const float4* __restrict__ pos_u, Grid g,
                                                            uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
                                                            uint32_t* __restrict__ count,
+                                                           uint64_t* __restrict__ outside,
                                                            unsigned long long* __restrict__ status) {
     const int i = blockIdx.x * kCsThreads + threadIdx.x;
     if (i < kScanBlocks) status[i] = 0ull;
     const int num = d_num ? *d_num : num_host;
-    if (i >= num) return;
-    const uint32_t key = hash_key(pos_u[i], g, kSubBits);
-    keys[i] = key;
-    rank[i] = atomicAdd(&count[key >> kSubBits], 1u);
+    const bool valid = i < num;
+    const uint32_t key = valid ? hash_key(pos_u[i], g, kSubBits) : 0u, cell = key >> kSubBits;
+    const bool out = valid && cell >= (uint32_t)g.nb_cells;
+    const uint64_t outs = __ballot(out);
+    if ((threadIdx.x & 63) == 0) {
+        outside[i >> 6] = outs;
+        if (outs != 0ull) atomicAdd(&count[g.nb_cells], (uint32_t)__popcll(outs));
+    }
+    if (valid) keys[i] = key;
+    if (valid && !out) rank[i] = atomicAdd(&count[cell], 1u);
 }
 
 // Block b scans the cells [b * chunk, (b + 1) * chunk) of the n_cells = nb_cells
@@ -184,13 +216,19 @@ __global__ __launch_bounds__(kScanThreads) void k_cell_scan(int n_cells, int chu
 __global__ __launch_bounds__(kCsThreads) void k_cell_place(int num_host, const int* __restrict__ d_num,
                                                            const uint32_t* __restrict__ keys,
                                                            const uint32_t* __restrict__ rank,
-                                                           const uint32_t* __restrict__ start,
+                                                           const uint32_t* __restrict__ start, int nb_cells,
+                                                           const uint64_t* __restrict__ outside,
                                                            uint2* __restrict__ pairs) {
-    const int i = blockIdx.x * kCsThreads + threadIdx.x;
+    const int i = blockIdx.x * kCsThreads + threadIdx.x, lane = (int)threadIdx.x & 63;
     const int num = d_num ? *d_num : num_host;
-    if (i >= num) return;
-    const uint32_t key = keys[i];
-    const uint32_t at = start[key >> kSubBits] + rank[i];
+    const bool valid = i < num;
+    const uint32_t key = valid ? keys[i] : 0u, cell = key >> kSubBits;
+    const bool out = valid && cell >= (uint32_t)nb_cells;
+    const uint64_t outs = __ballot(out);
+    uint32_t order = 0u;
+    if (outs != 0ull) order = outside_rank(outside, 0, i - lane, lane, outs);
+    if (!valid) return;
+    const uint32_t at = start[cell] + (out ? order : rank[i]);
     if (at < (uint32_t)num) pairs[at] = make_uint2(key, (uint32_t)i);
 }
 
@@ -252,10 +290,16 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_finish(int n, int num_host,
     }
     const uint2 kv = pairs[i];
     const float4 p = pu[kv.y], v = vu[kv.y], e = eu[kv.y];
-    const uint32_t cell = kv.x >> kSubBits, a = start[cell], b = end[cell];
-    uint32_t prev_xq;
-    const uint32_t before = rank_in_cell(pairs, kv, a, b, prev_xq);
-    const uint32_t to = a + before;
+    const uint32_t cell = kv.x >> kSubBits;
+    uint32_t to = (uint32_t)i;   // outside the grid: in order already
+    if (cell < (uint32_t)nb_cells) {
+        const uint32_t a = start[cell], b = end[cell];
+        uint32_t prev_xq;
+        const uint32_t before = rank_in_cell(pairs, kv, a, b, prev_xq);
+        to = a + before;
+        if (sub)
+            write_sub_starts(sub + (size_t)cell * kSubCells, kv.x & (kSubCells - 1), before, prev_xq, to, b);
+    }
     keys[to] = kv.x;
     idx[to] = kv.y;
     ps[to] = p;
@@ -263,8 +307,6 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_finish(int n, int num_host,
     es[to] = e;
     if (cu) cs[to] = cu[kv.y];   // permute.cl:41 (colours, when the system keeps them)
     if (left && cell >= (uint32_t)nb_cells) *left = 1;
-    if (sub && cell < (uint32_t)nb_cells)
-        write_sub_starts(sub + (size_t)cell * kSubCells, kv.x & (kSubCells - 1), before, prev_xq, to, b);
 }
 
 // The order in one block, for small launches: the counters (16 bits each, two to
@@ -287,7 +329,8 @@ __global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_ho
                                                                uint32_t* __restrict__ keys,
                                                                uint32_t* __restrict__ idx) {
     extern __shared__ uint32_t lds[];
-    __shared__ uint32_t wsum[kOneThreads / 64];
+    constexpr int kWaves = kOneThreads / 64;
+    __shared__ uint32_t wsum[kWaves], wout[kOnePer * kWaves];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int nc = g.nb_cells + 1, words = (nc + 2) / 2;   // the last entry: the end of the last cell
     uint32_t* order = lds + words;
@@ -321,7 +364,7 @@ __global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_ho
     __syncthreads();
     uint32_t run = inc - sum;
 #pragma unroll
-    for (int q = 0; q < kOneThreads / 64; ++q) run += q < w ? wsum[q] : 0u;
+    for (int q = 0; q < kWaves; ++q) run += q < w ? wsum[q] : 0u;
     for (int q = w0; q < w1; ++q) {
         const uint32_t v = lds[q], mid = run + (v & 0xFFFFu);
         lds[q] = run | mid << 16;
@@ -335,7 +378,25 @@ __global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_ho
         if (i < num) order[at(key[k] >> kSubBits) + rank[k]] = order_of(key[k], i);
     }
     for (int c = tid; c < nc; c += kOneThreads) start[c] = kEmpty;   // the occupied ones follow (launch_cells_permute)
+    // The particles outside the grid, where they are more than a cell's usual
+    // number: their places by counting the flags in index order.
+    const bool many_out = at((uint32_t)g.nb_cells + 1u) - at((uint32_t)g.nb_cells) > 64u;   // of the block
+    uint32_t out_before[kOnePer];
+    if (many_out) {
+#pragma unroll
+        for (int k = 0; k < kOnePer; ++k) {
+            const bool out = tid + k * kOneThreads < num && key[k] >> kSubBits >= (uint32_t)g.nb_cells;
+            const uint64_t outs = __ballot(out);
+            out_before[k] = (uint32_t)__popcll(outs & ((1ull << lane) - 1ull));
+            if (lane == 0) wout[k * kWaves + w] = (uint32_t)__popcll(outs);
+        }
+    }
     __syncthreads();
+    if (many_out) {
+#pragma unroll
+        for (int k = 0; k < kOnePer; ++k)
+            for (int q = 0; q < k * kWaves + w; ++q) out_before[k] += wout[q];
+    }
 #pragma unroll
     for (int k = 0; k < kOnePer; ++k) {
         const int i = tid + k * kOneThreads;
@@ -347,6 +408,11 @@ __global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_ho
             continue;
         }
         const uint32_t cell = key[k] >> kSubBits, a = at(cell), b = at(cell + 1), mine = order_of(key[k], i);
+        if (many_out && cell >= (uint32_t)g.nb_cells) {
+            keys[a + out_before[k]] = key[k];
+            idx[a + out_before[k]] = (uint32_t)i;
+            continue;
+        }
         uint32_t before = 0u;   // of the cell
         uint32_t j = a;
         for (; j + 8 <= b; j += 8) {
@@ -385,20 +451,28 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_count_b(int T, const uint16
                                                              const float4* __restrict__ pos_u,
                                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
                                                              uint32_t* __restrict__ count,
+                                                             uint64_t* __restrict__ outside,
                                                              unsigned long long* __restrict__ status) {
-    const int i = xcd_tile(blockIdx.x, gridDim.x) * kCsThreads + threadIdx.x;
+    const int i = xcd_tile(blockIdx.x, gridDim.x) * kCsThreads + threadIdx.x, lane = (int)threadIdx.x & 63;
     if (i < kScanBlocks) status[i] = 0ull;
-    if (i >= T) return;
-    const int s = sid[i];
+    const int s = i < T ? sid[i] : 0;
     const SceneDev& S = scenes[s];
     const int num = d_num[s], at = i - S.off;
-    if (at >= num) {
-        if (at == num) count[S.cell_base + S.g.nb_cells + 1] = (uint32_t)(S.cap - num);
-        return;
+    const bool valid = i < T && at < num;
+    if (i < T && at == num) count[S.cell_base + S.g.nb_cells + 1] = (uint32_t)(S.cap - num);
+    const uint32_t key = valid ? ((uint32_t)s << kSceneShift) | hash_key(pos_u[i], S.g, kSubBits) : 0u;
+    const uint32_t cell = cell_of_key(S, key), past = (uint32_t)(S.cell_base + S.g.nb_cells);
+    const bool out = valid && cell >= past;
+    const uint64_t outs = __ballot(out);
+    if (lane == 0) outside[i >> 6] = outs;
+    for (uint64_t left = outs; left != 0ull;) {   // scene by scene
+        const int lead = __builtin_ctzll(left), s0 = __builtin_amdgcn_readlane(s, lead);
+        const uint64_t same = __ballot(out && s == s0);
+        if (lane == lead) atomicAdd(&count[past], (uint32_t)__popcll(same));
+        left &= ~same;
     }
-    const uint32_t key = ((uint32_t)s << kSceneShift) | hash_key(pos_u[i], S.g, kSubBits);
-    keys[i] = key;
-    rank[i] = atomicAdd(&count[cell_of_key(S, key)], 1u);
+    if (valid) keys[i] = key;
+    if (valid && !out) rank[i] = atomicAdd(&count[cell], 1u);
 }
 
 __global__ __launch_bounds__(kCsThreads) void k_cell_place_b(int T, const uint16_t* __restrict__ sid,
@@ -407,13 +481,24 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_place_b(int T, const uint16
                                                              const uint32_t* __restrict__ keys,
                                                              const uint32_t* __restrict__ rank,
                                                              const uint32_t* __restrict__ start,
+                                                             const uint64_t* __restrict__ outside,
                                                              uint2* __restrict__ pairs) {
-    const int i = xcd_tile(blockIdx.x, gridDim.x) * kCsThreads + threadIdx.x;
-    if (i >= T) return;
-    const int s = sid[i];
+    const int i = xcd_tile(blockIdx.x, gridDim.x) * kCsThreads + threadIdx.x, lane = (int)threadIdx.x & 63;
+    const int s = i < T ? sid[i] : 0;
     const SceneDev& S = scenes[s];
-    if (i - S.off >= d_num[s]) return;
-    const uint32_t key = keys[i], at = start[cell_of_key(S, key)] + rank[i];
+    const bool valid = i < T && i - S.off < d_num[s];
+    const uint32_t key = valid ? keys[i] : 0u, cell = cell_of_key(S, key);
+    const bool out = valid && cell >= (uint32_t)(S.cell_base + S.g.nb_cells);
+    uint32_t order = 0u;
+    for (uint64_t left = __ballot(out); left != 0ull;) {   // scene by scene
+        const int lead = __builtin_ctzll(left), s0 = __builtin_amdgcn_readlane(s, lead);
+        const uint64_t same = __ballot(out && s == s0);
+        const uint32_t r = outside_rank(outside, scenes[s0].off, i - lane, lane, same);
+        if ((same >> lane) & 1ull) order = r;
+        left &= ~same;
+    }
+    if (!valid) return;
+    const uint32_t at = start[cell] + (out ? order : rank[i]);
     if (at < (uint32_t)T) pairs[at] = make_uint2(key, (uint32_t)i);
 }
 
@@ -437,12 +522,15 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_finish_b(int T, const uint1
     uint32_t to = (uint32_t)i;
     if (i - S.off < d_num[s]) {
         kv = pairs[i];
-        const uint32_t cell = cell_of_key(S, kv.x), a = start[cell], b = end[cell];
-        uint32_t prev_xq;
-        const uint32_t before = rank_in_cell(pairs, kv, a, b, prev_xq);
-        to = a + before;
-        if (sub && cell < (uint32_t)(S.cell_base + S.g.nb_cells))
-            write_sub_starts(sub + (size_t)cell * kSubCells, kv.x & (kSubCells - 1), before, prev_xq, to, b);
+        const uint32_t cell = cell_of_key(S, kv.x);
+        if (cell < (uint32_t)(S.cell_base + S.g.nb_cells)) {   // outside the grid: in order already
+            const uint32_t a = start[cell], b = end[cell];
+            uint32_t prev_xq;
+            const uint32_t before = rank_in_cell(pairs, kv, a, b, prev_xq);
+            to = a + before;
+            if (sub)
+                write_sub_starts(sub + (size_t)cell * kSubCells, kv.x & (kSubCells - 1), before, prev_xq, to, b);
+        }
     }
     const float4 p = pu[kv.y], v = vu[kv.y], e = eu[kv.y];
     keys[to] = kv.x;
@@ -466,9 +554,10 @@ hipError_t cell_sort_place_b(int T, const uint16_t* sid, const SceneDev* scenes,
     CellTemp t;
     cell_layout(T, total_cells - 1, &t, (char*)temp);
     k_cell_count_b<<<cs_blocks(std::max(T, kScanBlocks)), kCsThreads, 0, st>>>(T, sid, scenes, d_num, pos_u, keys,
-                                                                               idx, t.count, t.status);
+                                                                               idx, t.count, t.outside, t.status);
     launch_cell_scan(total_cells, t, start, end, st);
-    k_cell_place_b<<<cs_blocks(T), kCsThreads, 0, st>>>(T, sid, scenes, d_num, keys, idx, start, t.pairs);
+    k_cell_place_b<<<cs_blocks(T), kCsThreads, 0, st>>>(T, sid, scenes, d_num, keys, idx, start, t.outside,
+                                                            t.pairs);
     return hipGetLastError();
 }
 
@@ -498,9 +587,10 @@ hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* 
     CellTemp t;
     cell_layout(n, g.nb_cells, &t, (char*)temp);
     k_cell_count<<<cs_blocks(std::max(n, kScanBlocks)), kCsThreads, 0, st>>>(num_host, d_num, pos_u, g, keys, idx,
-                                                                             t.count, t.status);
+                                                                             t.count, t.outside, t.status);
     launch_cell_scan(g.nb_cells + 1, t, start, end, st);
-    k_cell_place<<<cs_blocks(n), kCsThreads, 0, st>>>(num_host, d_num, keys, idx, start, t.pairs);
+    k_cell_place<<<cs_blocks(n), kCsThreads, 0, st>>>(num_host, d_num, keys, idx, start, g.nb_cells, t.outside,
+                                                          t.pairs);
     return hipGetLastError();
 }
 

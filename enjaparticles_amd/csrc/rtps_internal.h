@@ -266,9 +266,10 @@ constexpr int kCellSortOneMax = 1 << 12;   // particles that one block sorts
 bool cell_sort_fits(int n, int nb_cells);
 size_t cell_sort_temp_bytes(int n, int nb_cells);   // for every count up to n
 hipError_t cell_sort_clear_temp(void* temp, int nb_cells, hipStream_t st);   // before the first sort
-// hash, sort and cellindices up to the order inside the cells (start and end
-// are written); then that order (keys, idx: hash_sort_pairs's result), the
-// sub-cell table (may be null) and the permute, as launch_cells_permute.
+// hash, sort and cellindices up to the order inside the cells; then that order
+// (keys, idx: hash_sort_pairs's result), the sub-cell table (may be null) and the
+// permute, as launch_cells_permute.  start and end are valid after both (small
+// launches write them in the second).
 hipError_t cell_sort_place(int n, int num_host, const int* d_num, const float4* pos_u, const Grid& g,
                            uint32_t pad_key, uint32_t* keys, uint32_t* idx, uint32_t* start, uint32_t* end, void* temp,
                            hipStream_t st);

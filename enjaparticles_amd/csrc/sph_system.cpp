@@ -929,7 +929,7 @@ int load_rigid(rtps_sph* s, int k, const rtps_float4* pos, const rtps_float4* ve
         void* old[] = {r.pos, r.vel, r.in_pos, r.in_vel, r.mass, r.in_mass, r.keys, r.idx, r.sort_tmp};
         for (void* b : old)
             if (b) RTPS_TRY_HIP(hipFree(b));
-RigidDev kept;   // the cell tables stay
+        RigidDev kept;   // the cell tables stay
         kept.start = r.start;
         kept.end = r.end;
         kept.near = r.near;
