@@ -55,7 +55,7 @@ struct rtps_sph {
     int* d_num = nullptr;
     int* tile_q = nullptr;   // per-XCD tile queue counters of the neighbour kernels (kTileQueueWords)
     void* sort_tmp = nullptr;
-    void* cell_tmp = nullptr;   // the counting sort's (cell_sort.hip)
+    void* cell_tmp = nullptr;   // the counting sort's (cell_sort.hip); null: never used
     // the neighbour rows the density kernel records for force loop 5 (Win::rows):
     // 9 rows x 3 words per particle slot, then 9 x 2 words per wave of 64 slots
     uint32_t* rows = nullptr;
@@ -231,7 +231,7 @@ int launch_front(rtps_sph* s, StageTimer& t) {
     // stage holds both, the "hash" stage is empty
     t.mark(ST_HASH);
     t.mark(ST_SORT);
-    const bool by_cell = s->opt_bucket && cell_sort_fits(n, s->nb_cells);
+    const bool by_cell = s->opt_bucket && s->cell_tmp && cell_sort_fits(n, s->nb_cells);
     if (by_cell) {
         RTPS_TRY_HIP(cell_sort_place(n, n, s->d_num, s->pos_u, s->g, s->pad_key, s->keys, s->idx, s->start, s->end, s->cell_tmp,
                                      s->stream));
@@ -702,8 +702,12 @@ int rtps_sph_create(const char* const* keys, const char* const* vals, int n, rtp
             RTPS_TRY_HIP(dalloc(&s->sub_start, (size_t)s->nb_cells * kSubCells));
         // the bucket sort's temp, a superset of the radix sort's, for every count up to N
         RTPS_TRY_HIP(hipMalloc(&s->sort_tmp, bucket_temp_bytes((int)N, s->key_bits)));
-        RTPS_TRY_HIP(hipMalloc(&s->cell_tmp, cell_sort_temp_bytes(std::min((int)N, kCellSortMax), s->nb_cells)));
-        RTPS_TRY_HIP(cell_sort_clear_temp(s->cell_tmp, s->nb_cells, s->stream));
+        // the counting sort's, where it takes any count (if not the largest, then none)
+        const int by_cell = std::min((int)N, kCellSortMax);
+        if (cell_sort_fits(by_cell, s->nb_cells)) {
+            RTPS_TRY_HIP(hipMalloc(&s->cell_tmp, cell_sort_temp_bytes(by_cell, s->nb_cells)));
+            RTPS_TRY_HIP(cell_sort_clear_temp(s->cell_tmp, s->nb_cells, s->stream));
+        }
         RTPS_TRY_HIP(dalloc(&s->rows, 27 * N + 18 * ((N + 63) / 64)));
         float4* zf[] = {s->pos_u, s->vel_u, s->veleval_u, s->pos_s, s->vel_s, s->ve_s, s->force_s, s->xsph_s};
         for (float4* p : zf) RTPS_TRY_HIP(hipMemsetAsync(p, 0, N * sizeof(float4), s->stream));
