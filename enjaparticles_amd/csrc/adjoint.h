@@ -14,6 +14,31 @@ namespace rtps {
 // eighths; 43 and 42 at 65,536).  A gradient over 20 steps of 65,536 particles
 // takes 2.41 ms in plain order, 2.31 in eighths.
 __host__ __device__ inline int adj_remap(int num) { return num <= 1 << 16 ? 1 : 16; }
+// How many of the `want` step records of a segment, `bytes` each, a handle keeps:
+// what half of the device's free memory holds.  The rest is the caller's (a
+// segment is then replayed once per part, and a record of 177 bytes a particle
+// would otherwise leave 4 of 286 GiB: 4,194,304 particles, segments of 400 steps).
+int adjoint_records(int want, size_t bytes);
+// The parts of a record of n particles in one allocation (the device gives out
+// whole 2 MiB: six of their own took 34 MiB instead of 24 at 131,072 particles).
+struct RecordLayout {
+    size_t idx, rows, pos, vel, ve, force, bytes;
+    RecordLayout(size_t n, size_t row_words) {
+        size_t at = 0;
+        auto part = [&at](size_t size) {
+            const size_t o = at;
+            at += (size + 255) & ~(size_t)255;
+            return o;
+        };
+        idx = part(4 * n);
+        rows = part(4 * row_words);
+        pos = part(16 * n);
+        vel = part(16 * n);
+        ve = part(16 * n);
+        force = part(16 * n);
+        bytes = at;
+    }
+};
 int adjoint_tiles(int num);   // tiles of B2 (shares of dL/dmu, dL/dK it writes)
 // A state's copy at the start of a run: pos and vel copied, veleval zero.
 hipError_t launch_adj_start(int num, const float4* pos, const float4* vel, float4* pos_out, float4* vel_out,

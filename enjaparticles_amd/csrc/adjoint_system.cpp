@@ -47,6 +47,20 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 }  // namespace
 
+namespace rtps {
+
+int adjoint_records(int want, size_t bytes) {
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return want;
+    }
+    bytes = (bytes + (2 << 20) - 1) >> 21 << 21;
+    return std::max(1, (int)std::min((size_t)want, free / 2 / bytes));
+}
+
+}  // namespace rtps
+
 struct rtps_adj {
     RTPSSettings settings;
     rtps_sph_params sp{};
@@ -92,20 +106,26 @@ namespace {
         if (e_ != hipSuccess) return hip_error(e_, #expr); \
     } while (0)
 
-// Records for `want` steps, or half as many while the device has no room.
+// Records for `want` steps or as many as adjoint_records allows, and half as many
+// while the device has no room.
 hipError_t alloc_records(rtps_adj* a, int want) {
     const size_t N = (size_t)a->N;
+    const RecordLayout L(N, 27 * N + 18 * ((N + 63) / 64));
+    want = adjoint_records(want, L.bytes);
     for (;; want = (want + 1) / 2) {
         const size_t before = a->allocs.size();
         a->rec.assign((size_t)want, Record());
         hipError_t e = hipSuccess;
         for (Record& r : a->rec) {
-            if (e == hipSuccess) e = a->alloc(&r.idx, N);
-            if (e == hipSuccess) e = a->alloc(&r.rows, 27 * N + 18 * ((N + 63) / 64));
-            if (e == hipSuccess) e = a->alloc(&r.pos_s, N);
-            if (e == hipSuccess) e = a->alloc(&r.vel_s, N);
-            if (e == hipSuccess) e = a->alloc(&r.ve_s, N);
-            if (e == hipSuccess) e = a->alloc(&r.force_s, N);
+            char* p = nullptr;
+            e = a->alloc(&p, L.bytes);
+            if (e != hipSuccess) break;
+            r.idx = (uint32_t*)(p + L.idx);
+            r.rows = (uint32_t*)(p + L.rows);
+            r.pos_s = (float4*)(p + L.pos);
+            r.vel_s = (float4*)(p + L.vel);
+            r.ve_s = (float4*)(p + L.ve);
+            r.force_s = (float4*)(p + L.force);
         }
         if (e == hipSuccess || e != hipErrorOutOfMemory || want == 1) return e;
         (void)hipGetLastError();
