@@ -127,6 +127,11 @@ hipError_t launch_force_rows(int num, int* d_num, const float4* pos_s, const flo
                              int collision, const rtps_float4& bmin, const rtps_float4& bmax, float dt, float4* pos_u,
                              float4* vel_u, float4* veleval_u, const float4* color_s, float4* color_u,
                              hipStream_t st);
+// Whether launch_density / launch_force (packed) take these (Win::block is then
+// without effect), and how many of the two may at this count.
+bool density_by_rows(int num, const Win& win);
+bool force_by_rows(int num, const Win& win);
+int kernels_by_rows(int num);
 hipError_t launch_count_pairs(int num, const int* d_num, const float4* pos_s, const uint32_t* start,
                               const uint32_t* end, const rtps_sph_params& sp, const Grid& g, const Win& win,
                               unsigned long long* out, hipStream_t st);

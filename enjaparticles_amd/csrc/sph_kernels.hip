@@ -909,7 +909,7 @@ hipError_t launch_density(int num, const int* d_num, const float4* pos_s, const 
     const bool stage = g_density_stage != 0;
     const size_t lds = stage ? (size_t)(bs / 64) * kStageCap * sizeof(float4) : 0;
     if (win_in.rows && win_in.rows_stride < (uint32_t)num) return hipErrorInvalidValue;
-    if (by_rows(num, win_in, kRowsMaxDensity) && packed && stage)
+    if (packed && density_by_rows(num, win_in))
         return launch_density_rows(num, d_num, pos_s, start, end, sp, g, win_in, packed, st);
     Win win = win_in;
     win.ntiles = nb;
@@ -947,6 +947,11 @@ static inline int force_loop(const Win& w) {
     return v == kLoopStagedBits && w.rows ? kLoopShared : v;
 }
 
+bool density_by_rows(int num, const Win& w) { return by_rows(num, w, kRowsMaxDensity) && g_density_stage != 0; }
+bool force_by_rows(int num, const Win& w) { return by_rows(num, w, kRowsMaxForce) && force_loop(w) == kLoopShared; }
+int kernels_by_rows(int num) { return (num <= kRowsMaxDensity ? 1 : 0) + (num <= kRowsMaxForce ? 1 : 0); }
+
+
 hipError_t launch_force(int num, int* d_num, const float4* pos_s, const float* dens, const float4* ve,
                         bool packed, const uint32_t* start, const uint32_t* end, const rtps_sph_params& sp,
                         const Grid& g, const Win& win_in, float4* force, float4* xsph, hipStream_t st) {
@@ -961,7 +966,7 @@ hipError_t launch_force(int num, int* d_num, const float4* pos_s, const float* d
     const size_t lds = force_lds(loop, bs);
     GravitySources none{};
     rtps_float4 z{0, 0, 0, 0};
-    if (loop == kLoopShared && packed && by_rows(num, win_in, kRowsMaxForce))
+    if (packed && force_by_rows(num, win_in))
         return launch_force_rows(num, d_num, pos_s, ve, start, sp, g, win_in, force, xsph, false, nullptr, nullptr,
                                  none, 0, z, z, 0.f, nullptr, nullptr, nullptr, nullptr, nullptr, st);
     Win win = win_in;
@@ -1007,7 +1012,7 @@ hipError_t launch_force_fused(int num, int* d_num, const float4* pos_s, const fl
     const int loop = force_loop(win_in);
     if (win_in.rows && win_in.rows_stride < (uint32_t)num) return hipErrorInvalidValue;
     const size_t lds = force_lds(loop, bs);
-    if (loop == kLoopShared && by_rows(num, win_in, kRowsMaxForce))
+    if (force_by_rows(num, win_in))
         return launch_force_rows(num, d_num, pos_s, ve_packed, start, sp, g, win_in, force, xsph, true, vel_s, idx,
                                  gsrc, collision, gps.bnd_min, gps.bnd_max, dt, pos_u, vel_u, veleval_u, color_s,
                                  color_u, st);

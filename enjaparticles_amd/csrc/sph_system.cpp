@@ -70,6 +70,7 @@ struct rtps_sph {
     // launch configuration of the neighbour kernels (0 / -1 = defaults), set by the autotuner
     int block_density = 0, block_force = 0, force_variant = -1;
     bool tuned = false;
+    int tuned_rows = -1;   // by the autotuner, for this kernels_by_rows(); -1: fixed by the caller
     hipGraphExec_t gexec = nullptr;
     bool graph_valid = false;
     StepRuns runs;   // of several steps, while that graph is valid
@@ -541,7 +542,9 @@ std::string tune_key(const rtps_sph* s) {
     while (n2 < (unsigned long)s->num_host) n2 <<= 1;
     return arch + "/cu" + std::to_string(cus) + "/n" + std::to_string(n2) + "/c" + std::to_string(s->nb_cells) +
            "/w" + std::to_string(s->opt_window) + "/r" + std::to_string(s->opt_remap) + "/q" + std::to_string(s->opt_queues) + "/s" +
-           std::to_string(s->sp.simulation_scale != 1.0f ? 1 : 0) + "/i" + std::to_string(s->integrator);
+           std::to_string(s->sp.simulation_scale != 1.0f ? 1 : 0) + "/i" + std::to_string(s->integrator) +
+           // the row kernels' lines lie inside the size classes
+           (kernels_by_rows(s->num_host) ? "/k" + std::to_string(kernels_by_rows(s->num_host)) : "");
 }
 
 void apply_tune(rtps_sph* s, const Tune& t) {
@@ -549,6 +552,7 @@ void apply_tune(rtps_sph* s, const Tune& t) {
     s->block_force = t.bf;
     s->force_variant = t.var;
     s->tuned = true;
+    s->tuned_rows = kernels_by_rows(s->num_host);
     s->graph_valid = false;
     s->timed_graph_valid = false;
 }
@@ -601,6 +605,7 @@ int autotune_step(rtps_sph* s, bool measure) {
     for (int bs : blocks) {
         Win w = win(s, false);
         w.block = bs;
+        if (bs != blocks[0] && density_by_rows(s->num_host, w)) break;   // block sizes without effect
         const float ms = time_it([&] {
             return launch_density(s->num_host, s->d_num, s->pos_s, s->start, s->end, s->sp, s->gs, w, nullptr,
                                   s->ve_s, s->stream);
@@ -618,6 +623,7 @@ int autotune_step(rtps_sph* s, bool measure) {
             Win w = win(s, true);
             w.block = bs;
             w.variant = var;
+            if (bs != blocks[0] && force_by_rows(s->num_host, w)) break;
             const float ms = time_it([&] {
                 // the euler step stores forces and leaves veleval alone: time the unfused force kernel
                 if (s->integrator == 1)
@@ -987,7 +993,10 @@ namespace {
 // after a push, whose graph would be captured for one replay only)
 int run_steps(rtps_sph* s, int nsteps, bool eager = false) {
     if (s->num_host == 0) return RTPS_OK;
-    if (s->opt_autotune && !s->tuned && nsteps > 0) {   // the first step also tunes the launches
+    // the first step also tunes the launches, and the first one after a push past
+    // a line between kernels that obey the choice and kernels that do not
+    const bool stale = s->tuned_rows >= 0 && s->tuned_rows != kernels_by_rows(s->num_host);
+    if (s->opt_autotune && (!s->tuned || stale) && nsteps > 0) {
         int rc = autotune_step(s, false);
         if (rc) return rc;
         if (--nsteps == 0) return RTPS_OK;
@@ -1353,6 +1362,7 @@ int rtps_sph_set_option(rtps_sph* s, int option, int value) {
             if (option == RTPS_OPT_BLOCK_DENSITY) s->block_density = value; else s->block_force = value;
             s->force_variant = -1;
             s->tuned = true;
+            s->tuned_rows = -1;
             break;
         case RTPS_OPT_DENSITY_STAGE:
             if (value < 0 || value > 1) return set_error(RTPS_ERR_ARG, "density stage option must be 0 or 1");

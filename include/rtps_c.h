@@ -366,7 +366,8 @@ int rtps_sph_set_option(rtps_sph* s, int option, int value);
  * and the fastest density + force pair kept
  * (a candidate tried later must be 5% faster).  The two kernels are idempotent on one sorted state, so the
  * step's result does not depend on the choice.  Choices are cached per
- * process by device and size class (and in the file named by the
+ * process by device, size class and the kernels that small launches go to (and
+ * in the file named by the
  * RTPS_TUNE_CACHE environment variable, when set); measure = 0 takes a cached
  * choice when there is one.  With RTPS_OPT_AUTOTUNE on (default) the first
  * rtps_sph_step does this by itself.  Reports the configuration in use. */
