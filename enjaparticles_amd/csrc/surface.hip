@@ -60,7 +60,7 @@ namespace {
 // Measured on a settled pool of 262,139 particles in a 128^3 lattice (14% of its
 // nodes in the fluid): 81 us, with bricks of 16 x 2 x 2 and 16 x 4 x 1 nodes 86
 // and 91, 8 x 4 x 2 97, 4 x 4 x 4 115; a thread per node that reads its windows
-// from memory 150, in bricks of 4 x 4 x 4 166.
+// from memory 150, in bricks of 4 x 4 x 4 166.  (Coarse lattices: bricks_pay.)
 constexpr int kBrickX = 32, kBrickY = 2, kBrickZ = 1;   // 64 nodes
 constexpr int kFieldCap = 256;   // candidates per LDS copy of a row (4 KB per wave)
 
@@ -162,6 +162,72 @@ __global__ __launch_bounds__(kBlockSurf) void k_color_field(int res, const float
         }
     }
     if (inside) field[((long)r * res + t) * res + s] = sum * sp.mass;
+}
+
+// The same for coarse lattices, a thread per node that reads its nine windows
+// from memory: the nodes of a wave are so far apart there that a brick's rows
+// reach across the box, most of them not its nodes' own.
+template <bool SCALED>
+__global__ __launch_bounds__(kBlockSurf) void k_color_field_nodes(int res, const float4* __restrict__ pos_s,
+                                                                  const float4* __restrict__ ve_s,
+                                                                  const uint32_t* __restrict__ start,
+                                                                  const uint32_t* __restrict__ end,
+                                                                  rtps_sph_params sp, Grid g, Win win,
+                                                                  rtps_float4 bmin, rtps_float4 bmax,
+                                                                  float* __restrict__ field) {
+    const long idx = (long)blockIdx.x * kBlockSurf + threadIdx.x;
+    if (idx >= (long)res * res * res) return;
+    const int s = (int)(idx % res), t = (int)((idx / res) % res), r = (int)(idx / ((long)res * res));
+    const float tmp = 1.0f / (float)(res - 1);
+    const float px = (float)s * tmp * (bmax.x - bmin.x) + bmin.x;
+    const float py = (float)t * tmp * (bmax.y - bmin.y) + bmin.y;
+    const float pz = (float)r * tmp * (bmax.z - bmin.z) + bmin.z;
+    const float scale = sp.simulation_scale;
+    const float h = sp.smoothing_distance, h2 = h * h, eps = sp.EPSILON;
+    const float h6 = h * h * h * h * h * h;
+    const float alpha = 15.0f / 3.14159265f / h6;
+    const int3 c = grid_cell(px, py, pz, g);
+    const WindowCtx wc = window_ctx(px, py, pz, g, c, h, win.keys, win.rx, win.ry, win.rz);
+    float sum = 0.0f;
+    for (int dz = -1; dz <= 1; ++dz)
+        for (int dy = -1; dy <= 1; ++dy) {
+            uint32_t a, b;
+            row_window(wc, c, dy, dz, h2, g, start, end, win.keys, a, b, 0u, win.sub);
+            auto term = [&](float4 pj, uint32_t j) {   // colorfield.cl:63-75
+                if (SCALED) { pj.x *= scale; pj.y *= scale; pj.z *= scale; }
+                const float rx = px - pj.x, ry = py - pj.y, rz = pz - pj.z;
+                const float r2 = rx * rx + ry * ry + rz * rz;
+                if (r2 <= h2) {
+                    const float rlen = fmaxf(__builtin_sqrtf(r2), eps);
+                    const float hr = h - rlen;
+                    sum += alpha * hr * hr * hr / ve_s[j].w;
+                }
+            };
+            uint32_t j = a;
+            for (; j + kGroup <= b; j += kGroup) {   // loads of a group issued together
+                float4 q[kGroup];
+#pragma unroll
+                for (int k = 0; k < kGroup; ++k) q[k] = pos_s[j + k];
+#pragma unroll
+                for (int k = 0; k < kGroup; ++k) term(q[k], j + k);
+            }
+            for (; j < b; ++j) term(pos_s[j], j);
+        }
+    field[idx] = sum * sp.mass;
+}
+
+// Where the bricks pay: from kBrickRes nodes an axis, fewer being too few waves,
+// at a node spacing of at most kBrickSpacing cells.  Measured (us, a thread per
+// node / bricks; settled pools): 21 / 75 at 2 nodes an axis and 64 / 67 at 16 of
+// 23 cells (20,011 particles); 31 / 75, 79 / 102, 139 / 103 and 158 / 96 at 3, 16,
+// 31 and 104 of 52 cells (262,139); 44 / 96, 168 / 202, 204 / 191, 169 / 156 and
+// 771 / 298 at 4, 40, 56, 80 and 159 of 79 cells (1,000,000).
+constexpr int kBrickRes = 28;
+constexpr float kBrickSpacing = 1.8f;
+bool bricks_pay(int res, const Grid& g, const rtps_float4& bmin, const rtps_float4& bmax) {
+    const float per = 1.0f / (float)(res - 1);   // along z a brick is one node
+    return res >= kBrickRes && (bmax.x - bmin.x) * per * g.delta.x <= kBrickSpacing &&
+           (bmax.y - bmin.y) * per * g.delta.y <= kBrickSpacing;
 }
 
 __device__ __forceinline__ float node(const float* __restrict__ f, int res, int x, int y, int z) {
@@ -330,14 +396,13 @@ hipError_t launch_color_field(int res, const float4* pos_s, const float4* ve_s, 
                               hipStream_t st) {
     (void)hipGetLastError();
     if (res < 2) return hipErrorInvalidValue;
+    const bool scaled = sp.simulation_scale != 1.0f, bricks = bricks_pay(res, g, bmin_scaled, bmax_scaled);
     const long bx = (res + kBrickX - 1) / kBrickX, by = (res + kBrickY - 1) / kBrickY, bz = (res + kBrickZ - 1) / kBrickZ;
-    const long n = bx * by * bz * 64;   // one wave per brick
-    if (sp.simulation_scale != 1.0f)
-        k_color_field<true><<<blocks_of(n, kBlockSurf), kBlockSurf, 0, st>>>(res, pos_s, ve_s, start, end, sp, g, win,
-                                                                            bmin_scaled, bmax_scaled, field);
-    else
-        k_color_field<false><<<blocks_of(n, kBlockSurf), kBlockSurf, 0, st>>>(res, pos_s, ve_s, start, end, sp, g, win,
-                                                                             bmin_scaled, bmax_scaled, field);
+    const long n = bricks ? bx * by * bz * 64 : (long)res * res * res;   // one wave per brick, or a thread per node
+    auto* kernel = bricks ? (scaled ? k_color_field<true> : k_color_field<false>)
+                          : (scaled ? k_color_field_nodes<true> : k_color_field_nodes<false>);
+    kernel<<<blocks_of(n, kBlockSurf), kBlockSurf, 0, st>>>(res, pos_s, ve_s, start, end, sp, g, win, bmin_scaled,
+                                                            bmax_scaled, field);
     return hipGetLastError();
 }
 
