@@ -163,6 +163,7 @@ int forward_step(rtps_adj* a, const State& in, const State& out, Record& r, bool
     w.sub = a->sub;
     w.rows = r.rows;
     w.rows_stride = (uint32_t)n;
+    w.rows_share = rows_share_of(a->sp);
     w.split = Win::kAlways;
     RTPS_TRY_HIP(launch_density(n, nullptr, r.pos_s, a->start, a->end, a->sp, a->gs, w, nullptr, r.ve_s, st));
     const GravitySources none{};

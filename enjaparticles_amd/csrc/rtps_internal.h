@@ -131,7 +131,8 @@ hipError_t launch_force_rows(int num, int* d_num, const float4* pos_s, const flo
 // without effect), and how many of the two may at this count.
 bool density_by_rows(int num, const Win& win);
 bool force_by_rows(int num, const Win& win);
-int kernels_by_rows(int num);
+int kernels_by_rows(int num, float share);
+float rows_share_of(const rtps_sph_params& sp);   // Win::rows_share
 hipError_t launch_count_pairs(int num, const int* d_num, const float4* pos_s, const uint32_t* start,
                               const uint32_t* end, const rtps_sph_params& sp, const Grid& g, const Win& win,
                               unsigned long long* out, hipStream_t st);

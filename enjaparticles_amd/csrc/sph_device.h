@@ -163,6 +163,7 @@ struct Win {
     // the neighbourhood (other roundings than the unsplit kernels' single sequence)
     enum Split { kNever, kSmall, kAlways };
     Split split = kNever;
+    float rows_share = 1.f;   // of the counts up to which launches go to row_tiles.hip (rows_share_of)
 };
 
 // Candidates per group in the neighbour loops (loads in flight per lane).

@@ -806,7 +806,22 @@ static inline bool nbr_split(int num, const Win& w, int most) {
 // one and 32.9 with the other there, 41.9, 40.2 and 43.7 at 32,768, 44.2, 45.2
 // and 51.6 at 49,152.
 constexpr int kRowsMaxDensity = 5 << 13, kRowsMaxForce = 3 << 13;
-static inline bool by_rows(int num, const Win& w, int most) { return w.rows && !w.tq && num <= most; }
+static inline bool below(int num, int most, float share) { return (float)num <= (float)most * share; }
+static inline bool by_rows(int num, const Win& w, int most) {
+    return w.rows && !w.tq && below(num, most, w.rows_share);
+}
+// Those lines are for smoothing lengths of two particle spacings, 34 neighbours at
+// rest.  With more of them a row's pairs exceed what its wave works out ahead,
+// and the turns take longer than a wave of its own would.  An update (us, tiles
+// / rows; at rest, then 2.5 times as dense) takes 118 / 88 and 176 / 158 at 12,000
+// particles of 65 neighbours at rest, 123 / 116 and 195 / 205 at 40,000;
+// 121 / 98 and 242 / 246 at 12,000 of 113, 132 / 143 and 304 / 373 at 40,000;
+// 168 / 164 and 325 / 395 at 2,000 of 268.
+float rows_share_of(const rtps_sph_params& sp) {
+    const double h = sp.smoothing_distance, neighbours = 4.0 / 3.0 * 3.14159265 * h * h * h * sp.rest_density / sp.mass;
+    if (!(neighbours > 40.0)) return 1.f;
+    return neighbours <= 120.0 ? (float)(40.0 / neighbours) : 0.f;
+}
 static inline int nbr_variant(const Win& w) {
     const int v = w.variant >= 0 ? w.variant : g_force_variant;
     return v == kLoopStaged || v == kLoopStagedBits ? v : kLoopDirect;
@@ -949,7 +964,9 @@ static inline int force_loop(const Win& w) {
 
 bool density_by_rows(int num, const Win& w) { return by_rows(num, w, kRowsMaxDensity) && g_density_stage != 0; }
 bool force_by_rows(int num, const Win& w) { return by_rows(num, w, kRowsMaxForce) && force_loop(w) == kLoopShared; }
-int kernels_by_rows(int num) { return (num <= kRowsMaxDensity ? 1 : 0) + (num <= kRowsMaxForce ? 1 : 0); }
+int kernels_by_rows(int num, float share) {
+    return (below(num, kRowsMaxDensity, share) ? 1 : 0) + (below(num, kRowsMaxForce, share) ? 1 : 0);
+}
 
 
 hipError_t launch_force(int num, int* d_num, const float4* pos_s, const float* dens, const float4* ve,

@@ -156,6 +156,7 @@ Win win(const rtps_sph* s, bool force = false) {
     if (s->opt_rows && s->rows && var == 5) {
         w.rows = s->rows;
         w.rows_stride = (uint32_t)s->max_num;
+        w.rows_share = rows_share_of(s->sp);
     }
     return w;
 }
@@ -540,11 +541,12 @@ std::string tune_key(const rtps_sph* s) {
     }
     unsigned long n2 = 1;
     while (n2 < (unsigned long)s->num_host) n2 <<= 1;
+    const int by_rows = kernels_by_rows(s->num_host, rows_share_of(s->sp));
     return arch + "/cu" + std::to_string(cus) + "/n" + std::to_string(n2) + "/c" + std::to_string(s->nb_cells) +
            "/w" + std::to_string(s->opt_window) + "/r" + std::to_string(s->opt_remap) + "/q" + std::to_string(s->opt_queues) + "/s" +
            std::to_string(s->sp.simulation_scale != 1.0f ? 1 : 0) + "/i" + std::to_string(s->integrator) +
            // the row kernels' lines lie inside the size classes
-           (kernels_by_rows(s->num_host) ? "/k" + std::to_string(kernels_by_rows(s->num_host)) : "");
+           (by_rows ? "/k" + std::to_string(by_rows) : "");
 }
 
 void apply_tune(rtps_sph* s, const Tune& t) {
@@ -552,7 +554,7 @@ void apply_tune(rtps_sph* s, const Tune& t) {
     s->block_force = t.bf;
     s->force_variant = t.var;
     s->tuned = true;
-    s->tuned_rows = kernels_by_rows(s->num_host);
+    s->tuned_rows = kernels_by_rows(s->num_host, rows_share_of(s->sp));
     s->graph_valid = false;
     s->timed_graph_valid = false;
 }
@@ -995,7 +997,7 @@ int run_steps(rtps_sph* s, int nsteps, bool eager = false) {
     if (s->num_host == 0) return RTPS_OK;
     // the first step also tunes the launches, and the first one after a push past
     // a line between kernels that obey the choice and kernels that do not
-    const bool stale = s->tuned_rows >= 0 && s->tuned_rows != kernels_by_rows(s->num_host);
+    const bool stale = s->tuned_rows >= 0 && s->tuned_rows != kernels_by_rows(s->num_host, rows_share_of(s->sp));
     if (s->opt_autotune && (!s->tuned || stale) && nsteps > 0) {
         int rc = autotune_step(s, false);
         if (rc) return rc;

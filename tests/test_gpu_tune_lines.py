@@ -73,3 +73,40 @@ def test_block_sizes_are_not_timed_where_they_have_no_effect(cuda, tmp_path, mon
         timed.append((err.count("density block"), err.count("force loop 5"), err.count("force loop 4")))
     s.close()
     assert timed == [(1, 1, 3), (1, 3, 3), (3, 3, 3)]
+
+
+def test_the_lines_are_lower_where_particles_have_more_neighbours(cuda, tmp_path, monkeypatch):
+    """A smoothing length of 2.5 spacings, 65 neighbours at rest: 40 / 65 of the
+    counts (15,020 and 25,033); of four, 268 neighbours: no row kernels."""
+    monkeypatch.setenv("RTPS_TUNE_CACHE", str(tmp_path / "choices"))
+    rng = np.random.default_rng(5)
+    pos = np.ones((30000, 4), np.float32)
+    pos[:, :3] = rng.uniform(0.02, 1.3, (30000, 3))
+    want = 0
+    for h, steps in (("0.05", ((10000, 1), (15015, 0), (15030, 1), (25020, 0), (25050, 1))), ("0.08", ((2000, 1), (2040, 0)))):
+        st = dict(scenes.dam_settings(1.32, 48000), smoothing_distance=h)
+        with RTPS.generateSystemInstance(st) as s:
+            at = 0
+            for upto, new in steps:
+                s.pushParticles(pos[at:upto], np.zeros_like(pos[at:upto]))
+                at = upto
+                s.step(1)
+                want += new
+                assert len(_choices(tmp_path)) == want, (h, upto)
+
+
+@pytest.mark.parametrize("h,n", [("0.05", 15000), ("0.05", 15040), ("0.05", 25050), ("0.06", 8000), ("0.08", 2000)])
+def test_both_kinds_of_kernel_give_the_same_bits(cuda, h, n):
+    """The rows and, through the tile queues, the tiles (which the queues always take)."""
+    out = []
+    for queues in (0, 1):
+        sc = scenes.dam_custom(32, 32, 32, seed=8)
+        with RTPS.generateSystemInstance(dict(sc.settings, smoothing_distance=h)) as s:
+            s.setOption(N.OPT_TILE_QUEUES, queues)
+            s.setOption(N.OPT_BLOCK_DENSITY, 64)
+            s.setOption(N.OPT_BLOCK_FORCE, 64)
+            s.pushParticles(sc.pos[:n], sc.vel[:n])
+            s.step(4)
+            out.append([s.read(f) for f in ("pos", "vel", "density")])
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
