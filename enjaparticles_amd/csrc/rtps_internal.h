@@ -137,7 +137,7 @@ hipError_t launch_count_pairs(int num, const int* d_num, const float4* pos_s, co
                               const uint32_t* end, const rtps_sph_params& sp, const Grid& g, const Win& win,
                               unsigned long long* out, hipStream_t st);
 // the maxima of parts of v[0, n) to out[0, *blocks), at most kMaxBlocks of them
-constexpr int kMaxBlocks = 64;
+constexpr int kMaxBlocks = 256;
 hipError_t launch_max_i32(int n, const int32_t* v, int32_t* out, int* blocks, hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, long n, hipStream_t st);
 

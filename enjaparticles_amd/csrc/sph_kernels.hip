@@ -93,12 +93,19 @@ __global__ void k_read_nc(const uint32_t* __restrict__ start, int nb_cells, int*
     if (threadIdx.x == 0 && blockIdx.x == 0) *nc = (int)start[nb_cells];
 }
 
-// Maximum of an index array, for the host's check of it.
+// Maximum of an index array, for the host's check of it: four loads of a thread
+// in flight, up to kMaxBlocks blocks.
 __global__ __launch_bounds__(kBlock) void k_max_i32(int n, const int32_t* __restrict__ v, int32_t* __restrict__ out) {
     __shared__ int32_t part[kBlock / 64];
     int32_t m = INT32_MIN;
-    // 64-bit: the stride goes past INT_MAX at counts within kMaxBlocks * kBlock of 2^31
-    for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long)gridDim.x * kBlock) m = max(m, v[i]);
+    // 64-bit: the stride goes past INT_MAX at counts near 2^31
+    const long stride = (long)gridDim.x * kBlock;
+    for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < n; i += 4 * stride) {
+        int32_t q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[k] = v[i + k * stride < n ? i + k * stride : i];
+        m = max(m, max(max(q[0], q[1]), max(q[2], q[3])));
+    }
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_down(m, o, 64));
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -869,7 +876,7 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t v, long n, hipStream_t st);
 
 hipError_t launch_max_i32(int n, const int32_t* v, int32_t* out, int* blocks, hipStream_t st) {
     (void)hipGetLastError();   // drop a stale error left by unrelated earlier HIP calls
-    *blocks = std::min(blocks_for(n), kMaxBlocks);
+    *blocks = std::min(blocks_for(n, 4 * kBlock), kMaxBlocks);
     k_max_i32<<<*blocks, kBlock, 0, st>>>(n, v, out);
     return hipGetLastError();
 }
