@@ -223,12 +223,15 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_place(int num_host, const i
     const int num = d_num ? *d_num : num_host;
     const bool valid = i < num;
     const uint32_t key = valid ? keys[i] : 0u, cell = key >> kSubBits;
+    uint32_t order = valid ? rank[i] : 0u;   // outside the grid not yet one
     const bool out = valid && cell >= (uint32_t)nb_cells;
     const uint64_t outs = __ballot(out);
-    uint32_t order = 0u;
-    if (outs != 0ull) order = outside_rank(outside, 0, i - lane, lane, outs);
+    if (outs != 0ull) {
+        const uint32_t r = outside_rank(outside, 0, i - lane, lane, outs);
+        order = out ? r : order;
+    }
     if (!valid) return;
-    const uint32_t at = start[cell] + (out ? order : rank[i]);
+    const uint32_t at = start[cell] + order;
     if (at < (uint32_t)num) pairs[at] = make_uint2(key, (uint32_t)i);
 }
 
@@ -371,6 +374,7 @@ __global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_ho
         run = mid + (v >> 16);
     }
     __syncthreads();
+    const uint32_t inside = at((uint32_t)g.nb_cells);   // particles in the grid
     auto order_of = [](uint32_t key, int i) { return key << 28 | (uint32_t)i; };   // x sixteenth, then index
 #pragma unroll
     for (int k = 0; k < kOnePer; ++k) {
@@ -380,7 +384,7 @@ __global__ __launch_bounds__(kOneThreads) void k_cell_sort_one(int n, int num_ho
     for (int c = tid; c < nc; c += kOneThreads) start[c] = kEmpty;   // the occupied ones follow (launch_cells_permute)
     // The particles outside the grid, where they are more than a cell's usual
     // number: their places by counting the flags in index order.
-    const bool many_out = at((uint32_t)g.nb_cells + 1u) - at((uint32_t)g.nb_cells) > 64u;   // of the block
+    const bool many_out = num - __builtin_amdgcn_readfirstlane((int)inside) > 64;   // of the block
     uint32_t out_before[kOnePer];
     if (many_out) {
 #pragma unroll
@@ -488,8 +492,8 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_place_b(int T, const uint16
     const SceneDev& S = scenes[s];
     const bool valid = i < T && i - S.off < d_num[s];
     const uint32_t key = valid ? keys[i] : 0u, cell = cell_of_key(S, key);
+    uint32_t order = valid ? rank[i] : 0u;   // outside the grid not yet one
     const bool out = valid && cell >= (uint32_t)(S.cell_base + S.g.nb_cells);
-    uint32_t order = 0u;
     for (uint64_t left = __ballot(out); left != 0ull;) {   // scene by scene
         const int lead = __builtin_ctzll(left), s0 = __builtin_amdgcn_readlane(s, lead);
         const uint64_t same = __ballot(out && s == s0);
@@ -498,7 +502,7 @@ __global__ __launch_bounds__(kCsThreads) void k_cell_place_b(int T, const uint16
         left &= ~same;
     }
     if (!valid) return;
-    const uint32_t at = start[cell] + (out ? order : rank[i]);
+    const uint32_t at = start[cell] + order;
     if (at < (uint32_t)T) pairs[at] = make_uint2(key, (uint32_t)i);
 }
 
