@@ -14,8 +14,8 @@
 // States are written where they are needed next (a checkpoint, the caller's
 // result), so no step copies them.
 //
-// Where the device has no room for a segment's records, fewer are kept
-// (`rec`) and a segment is replayed once per part of it.
+// Where a segment's records would take more than half of the device's free
+// memory, fewer are kept (`rec`) and a segment is replayed once per part of it.
 
 #include <hip/hip_runtime.h>
 
